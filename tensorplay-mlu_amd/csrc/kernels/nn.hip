@@ -997,19 +997,45 @@ __global__ __launch_bounds__(kBlock) void embedding_fill_kernel(const void* idx,
 }
 
 // Row `row` of the gradient = the sum of dy's rows entries[0 .. c) in that
-// order (float32, from 0), times 1 / c with scale_grad_by_freq; the block's
-// threads split the columns.
-template <typename T, bool VEC, bool NT = true>
+// order (float32, from 0), times 1 / c with scale_grad_by_freq; THREADS
+// consecutive threads split the columns.  Four samples' loads go out together ahead of
+// their adds (a row of 31 samples is then eight round trips to memory a
+// column instead of 31); rows with at most three samples, nearly all of
+// them for spread-out indices, keep the loop that loads one at a time.
+template <typename T, bool VEC, bool NT = true, int THREADS = kBlock>
 __device__ __forceinline__ void sum_row(const S_<T>* dy, const int* entries, int c, int64_t D,
                                         int scale_grad_by_freq, S_<T>* row) {
     constexpr int N = VEC ? Packet<T>::N : 1;
+    constexpr int kBatch = 4;
     const int64_t units = D / N;
     const float scale = scale_grad_by_freq ? 1.0f / static_cast<float>(c) : 1.0f;
-    for (int64_t q = threadIdx.x; q < units; q += kBlock) {
+    for (int64_t q = threadIdx.x % THREADS; q < units; q += THREADS) {
         float acc[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) acc[j] = 0.0f;
-        for (int k = 0; k < c; ++k) {
+        int k = 0;
+        for (; k + kBatch <= c; k += kBatch) {
+            if constexpr (VEC) {
+                uint4 raw[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u)
+                    raw[u] = load_raw_nt(dy + static_cast<int64_t>(entries[k + u]) * D + q * N);
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    float v[N];
+                    unpack<T>(raw[u], v);
+#pragma unroll
+                    for (int j = 0; j < N; ++j) acc[j] += v[j];
+                }
+            } else {
+                S_<T> raw[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) raw[u] = dy[static_cast<int64_t>(entries[k + u]) * D + q];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) acc[0] += Elem<T>::load(raw[u]);
+            }
+        }
+        for (; k < c; ++k) {
             const int64_t e = entries[k];
             if constexpr (VEC) {
                 float v[N];
@@ -1031,11 +1057,59 @@ __device__ __forceinline__ void sum_row(const S_<T>* dy, const int* entries, int
     }
 }
 
+// Columns [chunk x kBlock x W, + kBlock x W) of a row with many samples: the
+// same sum in the same order as sum_row, by one block per column chunk
+// instead of one per row.  The chain of adds is c long whatever the split,
+// so what bounds it is the loads in flight: a lane takes W columns (one
+// float32, two 16-bit: four bytes) and has kHotBatch samples' loads out at
+// once (64 measured 3-5 us slower).  Samples past the row's last are loaded again from it and added as
+// zero, which leaves the sum's bits (it starts at +0 and so is never -0).
+constexpr int kHotBatch = 32;
+
+template <typename T, int W>
+__device__ __forceinline__ void sum_hot_columns(const S_<T>* dy, const int* entries, int c, int64_t D,
+                                                int scale_grad_by_freq, int64_t chunk, S_<T>* row) {
+    using Word = std::conditional_t<W * sizeof(S_<T>) == 4, uint32_t, uint16_t>;
+    const int lane = threadIdx.x % kWave;
+    const int64_t col = (chunk * kBlock + threadIdx.x) * W;
+    const bool mine = col < D;
+    const S_<T>* base = dy + (mine ? col : 0);
+    float acc[W];
+#pragma unroll
+    for (int j = 0; j < W; ++j) acc[j] = 0.0f;
+    for (int k0 = 0; k0 < c; k0 += kWave) {
+        const int m = min(kWave, c - k0);
+        const int e = entries[k0 + min(lane, m - 1)];
+        for (int j0 = 0; j0 < m; j0 += kHotBatch) {
+            Word raw[kHotBatch];
+#pragma unroll
+            for (int j = 0; j < kHotBatch; ++j) {
+                const int64_t sample = __builtin_amdgcn_readlane(e, min(j0 + j, m - 1));
+                raw[j] = *reinterpret_cast<const Word*>(base + sample * D);
+            }
+#pragma unroll
+            for (int j = 0; j < kHotBatch; ++j) {
+                const Word v = j0 + j < m ? raw[j] : Word{0};
+                if constexpr (sizeof(S_<T>) == 4) {
+                    acc[0] += __uint_as_float(v);
+                } else {
+                    acc[0] += Elem<T>::load(static_cast<uint16_t>(v));
+                    if constexpr (W == 2) acc[1] += Elem<T>::load(static_cast<uint16_t>(v >> 16));
+                }
+            }
+        }
+    }
+    if (!mine) return;
+    const float scale = scale_grad_by_freq ? 1.0f / static_cast<float>(c) : 1.0f;
+#pragma unroll
+    for (int j = 0; j < W; ++j) row[col + j] = Elem<T>::store(acc[j] * scale);
+}
+
 // Row `row` of zeros (NT: non-temporal stores).
-template <typename T, bool VEC, bool NT = true>
+template <typename T, bool VEC, bool NT = true, int THREADS = kBlock>
 __device__ __forceinline__ void zero_row(int64_t D, S_<T>* row) {
     constexpr int N = VEC ? Packet<T>::N : 1;
-    for (int64_t q = threadIdx.x; q < D / N; q += kBlock) {
+    for (int64_t q = threadIdx.x % THREADS; q < D / N; q += THREADS) {
         if constexpr (VEC) {
             if constexpr (NT) store_raw_nt(row + q * N, make_uint4(0u, 0u, 0u, 0u));
             else *reinterpret_cast<uint4*>(row + q * N) = make_uint4(0u, 0u, 0u, 0u);
@@ -1134,19 +1208,27 @@ constexpr int kRangeWaves = kRangeThreads / kWave;
 constexpr int kRangeBatch = 8;  // index loads in flight per lane
 constexpr int64_t kRangeReadCap = int64_t{128} << 20;  // bytes of indices all blocks read, each pass
 constexpr int64_t kPlanListCap = int64_t{1} << 22;     // list entries beyond which fewer regions are used
+// Rows with at least this many samples are summed by a block per column
+// chunk (sum_hot_columns) instead of one block for the row.  Token
+// frequencies follow Zipf's law: of 8192 tokens over 32000 rows the first
+// has about 550, and its one block took 1386 us of a gradient whose other
+// rows are done in 130.
+constexpr int kHotSamples = 32;
+constexpr int kHotBlocks = 512;  // blocks that walk the heavy rows' (row, column chunk) pairs
 
 template <typename I>
 __global__ __launch_bounds__(kRangeThreads) void embedding_plan_range_kernel(const void* idx, int n, int64_t V,
                                                                       int64_t padding_idx, int rows_per_block,
                                                                       int regions, int* starts, int* counts,
-                                                                      int* list) {
+                                                                      int* list, int* hot_n, int* hot) {
     __shared__ int cursor[kRangeWaves][kRangeRows];
     __shared__ int first[kRangeRows + 1];
-    __shared__ int base_s;
+    __shared__ int base_s, hot_s;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_per_block;
     const int R = static_cast<int>(V - r0 < rows_per_block ? V - r0 : rows_per_block);
     for (int k = tid; k < kRangeWaves * kRangeRows; k += kRangeThreads) (&cursor[0][0])[k] = 0;
+    if (tid == 0) hot_s = 0;
     __syncthreads();
     const int64_t share = (static_cast<int64_t>(n) + kRangeWaves - 1) / kRangeWaves;
     const int64_t s0 = min<int64_t>(n, wave * share), s1 = min<int64_t>(n, s0 + share);
@@ -1215,9 +1297,16 @@ __global__ __launch_bounds__(kRangeThreads) void embedding_plan_range_kernel(con
     const int base_b = base_s;
     const int region = static_cast<int>(blockIdx.x % static_cast<unsigned>(regions)) * n;
     for (int l = tid; l < R; l += kRangeThreads) {
+        const int c = first[l + 1] - first[l];
         starts[r0 + l] = region + base_b + first[l];
-        counts[r0 + l] = first[l + 1] - first[l];
+        counts[r0 + l] = c;
+        // this block's rows with many samples, in any order (each is summed
+        // by itself)
+        if (c >= kHotSamples) hot[r0 + atomicAdd(&hot_s, 1)] = static_cast<int>(r0 + l);
     }
+    static_assert(kRangeRows <= kRangeThreads, "one pass lists every heavy row");
+    __syncthreads();
+    if (tid == 0) hot_n[blockIdx.x] = hot_s;
     for (int64_t base = s0; base < s1; base += kRangeBatch * kWave) {
         int lr[kRangeBatch];
         if (base == s0) {
@@ -1256,20 +1345,75 @@ __global__ __launch_bounds__(kRangeThreads) void embedding_plan_range_kernel(con
 // with the default policy).
 constexpr int64_t kGatherCachedBytes = int64_t{256} << 20;
 
-template <typename T, bool VEC, bool NT>
-__global__ __launch_bounds__(kBlock) void embedding_gather_ordered_kernel(const S_<T>* dy, const int* starts,
-                                                                          const int* counts, const int* list,
-                                                                          int n_list, int64_t D,
-                                                                          int scale_grad_by_freq, S_<T>* out) {
-    const int64_t r = blockIdx.x;
+//
+// The first hot_blocks blocks take the heavy rows the plan blocks listed
+// (hot_n[p] rows from hot[p x plan_rows] on), one (row, column chunk) pair
+// after another, and the row blocks skip those rows.  They come first in
+// the grid, so their longer chains run beside the other rows' stores.
+// Measured, [32000, 4096] float32 with 8192 Zipf-distributed indices: the
+// gather 1386 -> 138 us.
+//
+// ROWS rows a block: one row of four waves, or four rows of one wave each
+// where a row is at most kSmallRowBytes (a block a row leaves most of its
+// threads without a column there, and 50257 of them are bound by how fast
+// blocks start).
+constexpr int64_t kSmallRowBytes = 2048;
+template <typename T, bool VEC, bool NT, int ROWS>
+__global__ __launch_bounds__(kBlock) void embedding_gather_ordered_kernel(
+    const S_<T>* dy, const int* starts, const int* counts, const int* list, int n_list, int64_t D,
+    int64_t V, int scale_grad_by_freq, S_<T>* out, int hot_blocks, const int* hot_n, const int* hot, int plan_blocks,
+    int plan_rows) {
+    if (static_cast<int>(blockIdx.x) < hot_blocks) {
+        // Two 16-bit columns a lane need rows of whole four-byte words.
+        constexpr int W = VEC && sizeof(S_<T>) == 2 ? 2 : 1;
+        const int chunks = static_cast<int>((D + kBlock * W - 1) / (kBlock * W));
+        // thread t counts the heavy rows of `each` plan blocks; before[t] =
+        // those of the threads before it
+        __shared__ int before[kBlock + 1];
+        const int each = (plan_blocks + kBlock - 1) / kBlock;
+        const int p0 = min(plan_blocks, static_cast<int>(threadIdx.x) * each);
+        const int p1 = min(plan_blocks, p0 + each);
+        int own = 0;
+        for (int p = p0; p < p1; ++p) own += hot_n[p];
+        before[threadIdx.x + 1] = own;
+        if (threadIdx.x == 0) before[0] = 0;
+        __syncthreads();
+        for (int step = 1; step < kBlock; step *= 2) {
+            const int add = static_cast<int>(threadIdx.x) >= step ? before[threadIdx.x + 1 - step] : 0;
+            __syncthreads();
+            before[threadIdx.x + 1] += add;
+            __syncthreads();
+        }
+        const int64_t pairs = static_cast<int64_t>(before[kBlock]) * chunks;
+        for (int64_t pair = blockIdx.x; pair < pairs; pair += hot_blocks) {
+            const int h = static_cast<int>(pair / chunks);
+            int lo = 0, hi = kBlock;  // before[lo] <= h < before[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) / 2;
+                if (before[mid] <= h) lo = mid;
+                else hi = mid;
+            }
+            int j = h - before[lo], p = lo * each;
+            while (j >= hot_n[p]) j -= hot_n[p++];
+            const int64_t r = __builtin_amdgcn_readfirstlane(hot[static_cast<int64_t>(p) * plan_rows + j]);
+            const int off = __builtin_amdgcn_readfirstlane(min(max(starts[r], 0), n_list));
+            const int c = __builtin_amdgcn_readfirstlane(max(0, min(counts[r], n_list - off)));
+            if (c > 0) sum_hot_columns<T, W>(dy, list + off, c, D, scale_grad_by_freq, pair % chunks, out + r * D);
+        }
+        return;
+    }
+    constexpr int kThreads = kBlock / ROWS;
+    const int64_t r = static_cast<int64_t>(blockIdx.x - hot_blocks) * ROWS +
+                      (ROWS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0);
+    if (ROWS > 1 && r >= V) return;
     // starts and counts stay inside [0, n_list]; the clamps keep reads inside `list`
     const int off = min(max(starts[r], 0), n_list);
     const int c = max(0, min(counts[r], n_list - off));
     S_<T>* row = out + r * D;
     if (c == 0) {
-        zero_row<T, VEC, NT>(D, row);
-    } else {
-        sum_row<T, VEC, NT>(dy, list + off, c, D, scale_grad_by_freq, row);
+        zero_row<T, VEC, NT, kThreads>(D, row);
+    } else if (hot_blocks == 0 || c < kHotSamples) {
+        sum_row<T, VEC, NT, kThreads>(dy, list + off, c, D, scale_grad_by_freq, row);
     }
     // Last, after every load: a store ahead of them would make the compiler
     // read starts and counts through vector memory instead of scalar loads
@@ -1592,28 +1736,36 @@ int tp_amd_launch_embedding_backward(int device, int dtype, int64_t n, int64_t d
         const int64_t range_blocks = blocks_for(num_weights, per_block);
         const int64_t index_bytes = index_dtype == TP_AMD_INT32 ? 4 : 8;
         if (range_blocks * n * index_bytes <= kRangeReadCap) {
-            // starts [V], counts [V], list [regions x n]: up to kPlanCursors
+            // starts [V], counts [V], list [regions x n], heavy rows a plan
+            // block [blocks] and which they are [V]: up to kPlanCursors
             // regions while the list stays under kPlanListCap entries
             const int64_t regions = std::max<int64_t>(
                 1, std::min<int64_t>({int64_t{kPlanCursors}, range_blocks, kPlanListCap / std::max<int64_t>(n, 1)}));
-            Workspace ws(static_cast<size_t>(2 * num_weights + regions * n) * sizeof(int), index);
+            Workspace ws(static_cast<size_t>(3 * num_weights + regions * n + range_blocks) * sizeof(int), index);
             int* starts = static_cast<int*>(ws.get());
             int* counts = starts + num_weights;
             int* list = counts + num_weights;
+            int* hot_n = list + regions * n;
+            int* hot = hot_n + range_blocks;
+            const int hot_blocks = n >= kHotSamples ? kHotBlocks : 0;
             dispatch_index<float>(index_dtype, [&](auto tag) {
                 using I = decltype(tag);
                 embedding_plan_range_kernel<I><<<range_blocks, kRangeThreads, 0, st>>>(
                     indices, static_cast<int>(n), num_weights, padding_idx, static_cast<int>(per_block),
-                    static_cast<int>(regions), starts, counts, list);
+                    static_cast<int>(regions), starts, counts, list, hot_n, hot);
             });
             TP_AMD_DISPATCH_NN(dtype, T, {
                 const bool vec = dim % Packet<T>::N == 0 && aligned16(grad) && aligned16(out);
                 const bool nt = num_weights * dim * static_cast<int64_t>(sizeof(S_<T>)) > kGatherCachedBytes;
+                const bool small = dim * static_cast<int64_t>(sizeof(S_<T>)) <= kSmallRowBytes;
                 auto gather = [&](auto vec_tag, auto nt_tag) {
-                    embedding_gather_ordered_kernel<T, decltype(vec_tag)::value, decltype(nt_tag)::value>
-                        <<<num_weights, kBlock, 0, st>>>(static_cast<const S_<T>*>(grad), starts, counts, list,
-                                                        static_cast<int>(regions * n), dim, scale_grad_by_freq,
-                                                        static_cast<S_<T>*>(out));
+                    constexpr bool V = decltype(vec_tag)::value, C = decltype(nt_tag)::value;
+                    auto* kernel = small ? embedding_gather_ordered_kernel<T, V, C, 4>
+                                         : embedding_gather_ordered_kernel<T, V, C, 1>;
+                    kernel<<<blocks_for(num_weights, int64_t{small ? 4 : 1}) + hot_blocks, kBlock, 0, st>>>(
+                            static_cast<const S_<T>*>(grad), starts, counts, list, static_cast<int>(regions * n),
+                            dim, num_weights, scale_grad_by_freq, static_cast<S_<T>*>(out), hot_blocks, hot_n, hot,
+                            static_cast<int>(range_blocks), static_cast<int>(per_block));
                 };
                 using Yes = std::true_type;
                 using No = std::false_type;

@@ -318,6 +318,26 @@ def test_embedding_dense_backward_heavy_rows(dev, ops, orc, dtype):
         assert_normwise(got, want, dtype, float(np.sqrt(5000)), f"heavy rows unscaled D={D}")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("D", [1032, 1100, 257, 1], ids=lambda d: f"D{d}")
+def test_embedding_dense_backward_sample_counts_around_the_split(dev, ops, orc, dtype, D):
+    """Rows with 1 to 200 samples, on both sides of the 32 from which a row's
+    columns are shared between blocks and of the batches of 4, 32 and 64
+    samples inside: bit-exact against the float32 sum in sample order, a
+    heavy padding row included; D in whole and partial chunks, packed and
+    odd."""
+    counts = [0, 1, 3, 4, 5, 31, 32, 33, 63, 64, 65, 95, 96, 97, 128, 129, 200, 40]
+    V = len(counts) + 3
+    rng = np.random.default_rng(31)
+    idx = np.repeat(np.arange(len(counts)), counts).astype(np.int64)
+    rng.shuffle(idx)
+    dy = sample(orc, (len(idx), D), dtype, 32)
+    g, i = dev.from_numpy(dy, dtype=dtype), dev.from_numpy(idx)
+    for freq in (False, True):
+        got = ops.embedding_dense_backward(g, i, V, len(counts) - 1, freq).numpy()
+        assert_bitexact(got, sample_order_sum(orc, dtype, dy, idx, V, len(counts) - 1, freq), f"freq={freq}")
+
+
 def test_embedding_declines_sparse(dev, ops, orc):
     w = dev.from_numpy(sample(orc, (10, 8), F32, 17))
     i = dev.from_numpy(np.array([1, 2], np.int64))
