@@ -187,6 +187,44 @@ __device__ __forceinline__ void store_raw_nt(void* p, const uint4& raw) {
     __builtin_nontemporal_store(raw.w, &q->w);
 }
 
+// 16 bytes at any element address: one global_load/store_dwordx4 as well
+// (global memory is in unaligned access mode on this target), for rows whose
+// length is not a whole number of packets.  A wave's contiguous span of such
+// packets covers one more line than an aligned one.
+typedef unsigned int U32x4Any __attribute__((ext_vector_type(4), aligned(2)));
+
+__device__ __forceinline__ uint4 load_raw_any(const void* p) {
+    const U32x4Any v = *static_cast<const U32x4Any*>(p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+__device__ __forceinline__ uint4 load_raw_any_nt(const void* p) {
+    const U32x4Any v = __builtin_nontemporal_load(static_cast<const U32x4Any*>(p));
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+__device__ __forceinline__ void store_raw_any_nt(void* p, const uint4& raw) {
+    const U32x4Any v = {raw.x, raw.y, raw.z, raw.w};
+    __builtin_nontemporal_store(v, static_cast<U32x4Any*>(p));
+}
+
+// The aligned or the unaligned form, by ANY.
+template <bool ANY>
+__device__ __forceinline__ uint4 load_raw(const void* p) {
+    if constexpr (ANY) return load_raw_any(p);
+    else return *static_cast<const uint4*>(p);
+}
+template <bool ANY>
+__device__ __forceinline__ uint4 load_raw_stream(const void* p) {
+    if constexpr (ANY) return load_raw_any_nt(p);
+    else return load_raw_nt(p);
+}
+template <bool ANY>
+__device__ __forceinline__ void store_raw_stream(void* p, const uint4& raw) {
+    if constexpr (ANY) store_raw_any_nt(p, raw);
+    else store_raw_nt(p, raw);
+}
+
 // Unsigned division by a runtime constant d (1 <= d < 2^31) for numerators
 // n < 2^31: with s = ceil(log2 d) and m = ceil(2^(31+s) / d) (which fits in
 // 32 bits), floor(n / d) = (n * m) >> (31 + s).  The rounding error of m
@@ -277,6 +315,16 @@ __device__ __forceinline__ uint4 buffer_load16_cached(Rsrc r, uint32_t offset) {
 __device__ __forceinline__ void buffer_store16(Rsrc r, uint32_t offset, const uint4& v) {
     const U32x4 d = {v.x, v.y, v.z, v.w};
     __builtin_amdgcn_raw_buffer_store_b128(d, r, offset, 0, kNt);
+}
+
+// One element at a byte offset (0 past the resource's end).
+template <typename T>
+__device__ __forceinline__ float buffer_load_elem(Rsrc r, uint32_t offset) {
+    if constexpr (sizeof(typename Elem<T>::storage) == 4) {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, kNt));
+    } else {
+        return Elem<T>::load(__builtin_amdgcn_raw_buffer_load_b16(r, offset, 0, kNt));
+    }
 }
 
 __device__ __forceinline__ float buffer_load_f32(Rsrc r, uint32_t offset) {

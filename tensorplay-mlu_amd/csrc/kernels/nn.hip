@@ -1545,10 +1545,13 @@ __global__ __launch_bounds__(kBlock) void nll_backward_kernel(const S_<T>* grad,
     dx[e] = Elem<T>::store(opaque(v));
 }
 
-// The same with dx as rows of 16-byte packets (C a multiple of the packet,
-// dx aligned): a row takes `blocks_per_row` blocks, each thread one packet,
-// holding the target's value if the target falls inside it.
-template <typename T, typename I>
+// The same with dx as rows of 16-byte packets: a row takes `blocks_per_row`
+// blocks, each thread one packet, holding the target's value if the target
+// falls inside it.  ANY: rows of any length (C at least kNllRowClasses),
+// their packets at any element, the last C % N elements one thread's.
+// Measured, 2048 x 50257: bfloat16 131 -> 44 us, float32 141 -> 87 us.
+constexpr int64_t kNllRowClasses = 512;  // shorter odd rows leave most of a block idle
+template <typename T, typename I, bool ANY>
 __global__ __launch_bounds__(kBlock) void nll_backward_rows_kernel(const S_<T>* grad, const void* target,
                                                                    const S_<T>* w, const S_<T>* total,
                                                                    int64_t C, uint32_t blocks_per_row,
@@ -1557,7 +1560,8 @@ __global__ __launch_bounds__(kBlock) void nll_backward_rows_kernel(const S_<T>* 
     constexpr int N = Packet<T>::N;
     const uint32_t i = blockIdx.x / blocks_per_row;
     const int64_t q = static_cast<int64_t>(blockIdx.x - i * blocks_per_row) * kBlock + threadIdx.x;
-    if (q >= C / N) return;
+    const int64_t npk = C / N;
+    if (q >= (ANY ? (C + N - 1) / N : npk)) return;
     const int64_t t = index_at<I>(target, i);
     const bool bad = t != ignore_index && (t < 0 || t >= C);
     float v[N];
@@ -1572,7 +1576,15 @@ __global__ __launch_bounds__(kBlock) void nll_backward_rows_kernel(const S_<T>* 
 #pragma unroll
         for (int j = 0; j < N; ++j) v[j] = j == k ? val : v[j];
     }
-    store_raw_nt(dx + static_cast<int64_t>(i) * C + q * N, pack<T>(v));
+    S_<T>* to = dx + static_cast<int64_t>(i) * C + q * N;
+    if (ANY && q == npk) {
+        const int rem = static_cast<int>(C - npk * N);
+#pragma unroll
+        for (int j = 0; j < N - 1; ++j)
+            if (j < rem) to[j] = Elem<T>::store(v[j]);
+        return;
+    }
+    store_raw_stream<ANY>(to, pack<T>(v));
 }
 
 template <typename T, typename F>
@@ -1854,11 +1866,13 @@ int tp_amd_launch_nll_loss_backward(int device, int dtype, int64_t n, int64_t cl
         const int64_t blocks = blocks_for(n * classes, kBlock);
         TP_AMD_DISPATCH_NN(dtype, T, {
             constexpr int N = Packet<T>::N;
-            const int64_t per_row = blocks_for(classes / N, kBlock);
-            if (classes % N == 0 && aligned16(dx) && n * per_row <= 0x7fffffff) {
+            const int64_t per_row = blocks_for(blocks_for(classes, N), kBlock);
+            const bool aligned = classes % N == 0 && aligned16(dx);
+            if ((aligned || classes >= kNllRowClasses) && n * per_row <= 0x7fffffff) {
                 dispatch_index<T>(index_dtype, [&](auto tag) {
                     using I = decltype(tag);
-                    nll_backward_rows_kernel<T, I><<<n * per_row, kBlock, 0, stream(index)>>>(
+                    auto* kernel = aligned ? nll_backward_rows_kernel<T, I, false> : nll_backward_rows_kernel<T, I, true>;
+                    kernel<<<n * per_row, kBlock, 0, stream(index)>>>(
                         static_cast<const S_<T>*>(grad), target, static_cast<const S_<T>*>(weight),
                         static_cast<const S_<T>*>(total_weight), classes, static_cast<uint32_t>(per_row),
                         ignore_index, reduction, static_cast<S_<T>*>(dx));

@@ -387,6 +387,27 @@ def test_nll_loss_int32_targets_and_bad_target(dev, ops, orc):
     assert np.isnan(dx[7]).all() and not np.isnan(np.delete(dx, 7, axis=0)).any()
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("c", [511, 512, 513, 519, 2055, 4097])
+def test_nll_loss_backward_rows_at_any_element(dev, ops, orc, dtype, c):
+    """Odd class counts around the row kernel's lower bound: targets in the
+    first, last and partial packets, one ignored and one outside."""
+    n = 37
+    t = np.random.default_rng(51).integers(0, c, size=n).astype(np.int64)
+    t[:6] = [0, 1, c - 1, c - 2, 7, -100]
+    g = orc.from_float(np.random.default_rng(52).standard_normal(n).astype(np.float32), dtype)
+    total = orc.from_float(np.zeros((), np.float32), dtype)
+    x = dev.from_numpy(sample(orc, (n, c), dtype, 53), dtype=dtype)
+    args = (dev.from_numpy(g, dtype=dtype), x, dev.from_numpy(t), None, 0, -100, dev.from_numpy(total, dtype=dtype))
+    got = ops.nll_loss_backward(*args).numpy()
+    want = orc.nll_loss_backward(dtype, g, (n, c), t, total, None, 0, -100)
+    assert_elementwise(got, want, dtype, "odd nll backward")
+    t[9] = c
+    bad = ops.nll_loss_backward(args[0], x, dev.from_numpy(t), *args[3:]).numpy()
+    assert np.isnan(as_float(bad, dtype)[9]).all()
+    assert_bitexact(np.delete(bad, 9, axis=0), np.delete(got, 9, axis=0), "the other rows")
+
+
 def test_nll_loss_large_batch(dev, ops, orc):
     n, c = 2048, 32000
     x = sample(orc, (n, c), F32, 22)

@@ -438,6 +438,30 @@ def test_softmax_row_lengths(dev, ops, orc, D):
                                     yh, g, rows, D, 1, f"backward D={D} log={log}")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("D", [2, 3, 9, 63, 333, 515, 1001, 2049, 4099, 8189, 12291, 16387, 32001, 40961, 50257,
+                               51203, 65539, 102405])
+def test_softmax_rows_at_any_element(dev, ops, orc, dtype, D):
+    """Rows whose length is not a whole number of packets, and whose tensor
+    starts off a 16-byte boundary: every row kernel (registers, the walk of
+    16-wave rows, 512-thread rows, two passes) with packets at any element
+    and a partial last packet."""
+    rows = 5 if D > 4000 else 13
+    a = sample(orc, (rows * D + 1,), dtype, 41, 3.0)
+    g = sample(orc, (rows * D + 1,), dtype, 42)
+    x = dev.from_numpy(a, dtype=dtype)[1:].view(rows, D)
+    dy = dev.from_numpy(g, dtype=dtype)[1:].view(rows, D)
+    a, g = a[1:].reshape(rows, D), g[1:].reshape(rows, D)
+    for log in (False, True):
+        y = (ops.log_softmax if log else ops.softmax)(x, -1)
+        yh = y.numpy()
+        assert_softmax(yh, orc.softmax(log, dtype, a, rows, D, 1), dtype, log, f"D={D} log={log}")
+        back = ops._log_softmax_backward_data if log else ops._softmax_backward_data
+        got = back(dy, y, -1, dtype).numpy()
+        assert_softmax_backward(got, orc.softmax_backward(log, dtype, yh, g, rows, D, 1), dtype, log,
+                                yh, g, rows, D, 1, f"backward D={D} log={log}")
+
+
 @pytest.mark.parametrize("rows,D,dtype", [(600, 8200, F32), (1000, 20000, F32), (257, 32000, F32),
                                           (600, 16400, BF16), (513, 30000, BF16)])
 def test_softmax_rows_walked_by_one_block_per_cu(dev, ops, orc, rows, D, dtype):
