@@ -20,27 +20,13 @@
 //     tiles loaded straight into LDS by buffer loads and read back with
 //     ds_read_b128 (K-major operands) or ds_read_b64_tr_b16 (transposed
 //     views, read in place); no bounds checks anywhere in the K loop.
-//   * other 16-bit products with a 256 x 256 tile per CU: 256 x 256 with
-//     8 waves (2 x 4, each wave a 128 x 64 patch of 4 x 2 MFMA tiles of
-//     32 x 32).
-//   * everything else: 128 x 128 with 4 waves (2 x 2, each 64 x 64); a
-//     product too small for those tiles to reach a quarter of the CUs
-//     (float32: even split over K) takes 64 x 64 with 2 waves (each
-//     32 x 64).
-// The last two advance K BK at a time through two LDS stages: while the
-// waves multiply out of one stage, the next K tile is written into the
-// other and the one after is already in flight from global memory, so each
-// K step needs a single barrier.  Operands sit in LDS K-major ([row][k],
-// rows padded by 16 bytes so the 16-byte fragment reads of 16 consecutive
-// rows hit distinct banks).  An operand stored K-major in memory is copied
-// with 16-byte loads; a 16-bit one stored with its M (or N) axis contiguous
-// is loaded as V x 4 blocks (V along M/N, 4 along K) and transposed in
-// registers before its LDS store, a float32 one is kept as it lies
-// ([k][row] tiles, read back one float at a time).  All kernels number their
+//   * everything else: the tile kernel, gemm_tile_kernel, at a tile shape
+//     and a split over K that plan_tiles picks.
+// The last two load operand tiles straight into LDS, 128 bytes of K a step,
+// read an operand where it lies in either orientation, and keep the next K
+// tiles' loads in flight while they multiply.  All kernels number their
 // tiles so each of the 8 XCDs walks a contiguous range in groups of 8 tile
-// rows, keeping an XCD's A and B panels hot in its own L2.  A float32
-// product of one matrix with too few tiles to fill the CUs is split over K
-// (launch_splitk).
+// rows, keeping an XCD's A and B panels hot in its own L2.
 
 #include <type_traits>
 #include <utility>
@@ -67,12 +53,19 @@ template <>
 struct Mfma<bf16_t> {
     static constexpr int V = 8;     // elements per 16-byte vector
     static constexpr int BK = 64;   // K per LDS tile
-    static constexpr int KSUB = 16; // K per fragment read
     __device__ __forceinline__ static f32x16 mma(const uint4& a, const uint4& b, f32x16 c) {
         bf16x8 av, bv;
         __builtin_memcpy(&av, &a, 16);
         __builtin_memcpy(&bv, &b, 16);
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, c, 0, 0, 0);
+    }
+    static constexpr int kPerTile = 1;  // MFMAs a 32 x 32 tile takes per fragment
+    template <int TM, int TN>
+    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[TM][TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) c[i][j] = mma(a[i], b[j], c[i][j]);
     }
 };
 
@@ -80,12 +73,19 @@ template <>
 struct Mfma<f16_t> {
     static constexpr int V = 8;
     static constexpr int BK = 64;
-    static constexpr int KSUB = 16;
     __device__ __forceinline__ static f32x16 mma(const uint4& a, const uint4& b, f32x16 c) {
         f16x8 av, bv;
         __builtin_memcpy(&av, &a, 16);
         __builtin_memcpy(&bv, &b, 16);
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, c, 0, 0, 0);
+    }
+    static constexpr int kPerTile = 1;
+    template <int TM, int TN>
+    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[TM][TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) c[i][j] = mma(a[i], b[j], c[i][j]);
     }
 };
 
@@ -93,13 +93,21 @@ template <>
 struct Mfma<float> {
     static constexpr int V = 4;
     static constexpr int BK = 32;
-    static constexpr int KSUB = 8;
-    __device__ __forceinline__ static f32x16 mma(const uint4& a, const uint4& b, f32x16 c) {
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
-        return c;
+    static constexpr int kPerTile = 4;
+    // The four k of a fragment in order for each tile, a pass over the tiles
+    // for each, so consecutive MFMAs do not wait on one accumulator.
+    template <int TM, int TN>
+    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[TM][TN]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const uint32_t u = k == 0 ? a[i].x : k == 1 ? a[i].y : k == 2 ? a[i].z : a[i].w;
+                    const uint32_t v = k == 0 ? b[j].x : k == 1 ? b[j].y : k == 2 ? b[j].z : b[j].w;
+                    c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(u), __uint_as_float(v), c[i][j], 0, 0, 0);
+                }
     }
 };
 
@@ -113,146 +121,13 @@ __device__ __forceinline__ void put_c(S* dst, S v) {
     __builtin_nontemporal_store(v, dst);
 }
 
-__device__ __forceinline__ uint32_t component(const uint4& v, int i) {
-    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-
-// One operand's tile loader: R rows (M or N) x BK, into LDS [R][BK + pad].
-// KMAJOR: element (r, k) at X[r * ld + k]; otherwise at X[k * ld + r].
-// A float32 operand with its M (or N) axis contiguous (KROWS) is copied as it
-// lies instead, [BK][R + 8]: 16-byte loads along the row, 32 lanes a row, and
-// 16-byte LDS stores; the fragment reads then take a lane's 4 consecutive k
-// as 4 single-float reads, the two lane halves 4 rows apart, which the pad of
-// 8 floats puts on the other half of the 64 banks.  (Transposing 4 x 4
-// blocks in registers before a K-major store, as the 16-bit types do, left
-// the float32 NN and TN products waiting 7-10x longer than NT: 4096^3 NN
-// 1469 us, TN 1606 us, NT 1261 us.)
-template <typename T, int R, bool KMAJOR, int THREADS>
-struct TileLoader {
-    using S = typename Elem<T>::storage;
-    static constexpr int V = Mfma<T>::V;
-    static constexpr int BK = Mfma<T>::BK;
-    static constexpr int LDS_STRIDE = BK + 16 / sizeof(S);  // elements per LDS row
-    static constexpr bool KROWS = !KMAJOR && sizeof(S) == 4;
-    static constexpr int KR_STRIDE = R + 8;                  // KROWS: elements per LDS row (one k)
-    static_assert(!KROWS || BK * KR_STRIDE <= R * LDS_STRIDE, "KROWS tile fits the K-major space");
-    // K-major: R * BK / V vectors; MN-major: (R / V) * (BK / 4) units of 4
-    // vectors (V along M/N by 4 along K).
-    static constexpr int kLoads = (KMAJOR ? R * BK / V : (R / V) * (BK / 4) * 4) / THREADS;
-    static constexpr int kUnits = kLoads / 4;  // MN-major units per thread
-    static_assert(kLoads * THREADS == (KMAJOR ? R * BK / V : (R / V) * (BK / 4) * 4) &&
-                      (KMAJOR || kUnits * 4 == kLoads),
-                  "tile shape and thread count disagree");
-    uint4 reg[kLoads];
-
-    __device__ __forceinline__ void load(const S* X, int64_t ld, int64_t r0, int64_t rows,
-                                         int64_t k0, int64_t K) {
-        const int tid = threadIdx.x;
-        if constexpr (KROWS) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int v = tid + i * THREADS;
-                const int k = v / (R / V), c = v % (R / V);
-                const int64_t gr = r0 + c * V, gk = k0 + k;
-                if (gr < rows && gk < K) {
-                    reg[i] = *reinterpret_cast<const uint4*>(X + gk * ld + gr);
-                } else {
-                    reg[i] = make_uint4(0, 0, 0, 0);
-                }
-            }
-        } else if constexpr (KMAJOR) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int v = tid + i * THREADS;
-                const int r = v / (BK / V), kc = v % (BK / V);
-                const int64_t gr = r0 + r, gk = k0 + kc * V;
-                if (gr < rows && gk < K) {
-                    reg[i] = *reinterpret_cast<const uint4*>(X + gr * ld + gk);
-                } else {
-                    reg[i] = make_uint4(0, 0, 0, 0);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < kUnits; ++u) {
-                const int unit = tid + u * THREADS;
-                const int kb = unit % (BK / 4), rb = unit / (BK / 4);
-                const int64_t gr = r0 + rb * V;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int64_t gk = k0 + kb * 4 + i;
-                    if (gr < rows && gk < K) {
-                        reg[u * 4 + i] = *reinterpret_cast<const uint4*>(X + gk * ld + gr);
-                    } else {
-                        reg[u * 4 + i] = make_uint4(0, 0, 0, 0);
-                    }
-                }
-            }
-        }
-    }
-
-    __device__ __forceinline__ void store(S* lds) const {
-        const int tid = threadIdx.x;
-        if constexpr (KROWS) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int v = tid + i * THREADS;
-                const int k = v / (R / V), c = v % (R / V);
-                *reinterpret_cast<uint4*>(lds + k * KR_STRIDE + c * V) = reg[i];
-            }
-        } else if constexpr (KMAJOR) {
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int v = tid + i * THREADS;
-                const int r = v / (BK / V), kc = v % (BK / V);
-                *reinterpret_cast<uint4*>(lds + r * LDS_STRIDE + kc * V) = reg[i];
-            }
-        } else {
-            // Consecutive lanes take consecutive K blocks of one M/N block, so
-            // the rows they write lie side by side in the LDS banks (with the
-            // M/N block varying fastest, 32 lanes would land on two banks).
-#pragma unroll
-            for (int u = 0; u < kUnits; ++u) {
-                const int unit = tid + u * THREADS;
-                const int kb = unit % (BK / 4), rb = unit / (BK / 4);
-                const uint4* in = reg + u * 4;
-                if constexpr (sizeof(S) == 4) {
-                    // 4 (k) x 4 (r) floats -> 4 rows of 4 consecutive k.
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const uint4 out = make_uint4(component(in[0], j), component(in[1], j),
-                                                     component(in[2], j), component(in[3], j));
-                        *reinterpret_cast<uint4*>(lds + (rb * V + j) * LDS_STRIDE + kb * 4) = out;
-                    }
-                } else {
-                    // 4 (k) x 8 (r) 16-bit values -> 8 rows of 4 consecutive k.
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int p = j / 2, hi = j % 2;
-                        uint32_t w[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const uint32_t c = component(in[i], p);
-                            w[i] = hi ? (c >> 16) : (c & 0xffffu);
-                        }
-                        uint2 out;
-                        out.x = w[0] | (w[1] << 16);
-                        out.y = w[2] | (w[3] << 16);
-                        *reinterpret_cast<uint2*>(lds + (rb * V + j) * LDS_STRIDE + kb * 4) = out;
-                    }
-                }
-            }
-        }
-    }
-};
-
-// XCD-aware, L2-grouped tile order: consecutive ids land on the same XCD
-// (blocks are dealt round-robin over the 8 XCDs), and each XCD walks its
-// range in groups of kGroupM tile rows.
+// XCD-aware, L2-grouped tile order: blocks are dealt round-robin over the 8
+// XCDs, and each XCD walks a contiguous range of tiles (the first total % 8
+// one tile more) in groups of kGroupM tile rows.
 __device__ __forceinline__ void tile_coords(int bid, int grid_m, int grid_n, int& pm, int& pn) {
     const int total = grid_m * grid_n;
-    int pid = bid;
-    if (total % 8 == 0) pid = (bid % 8) * (total / 8) + bid / 8;
+    const int xcd = bid % 8, q = total / 8, rest = total % 8;
+    const int pid = xcd * q + (xcd < rest ? xcd : rest) + bid / 8;
     const int in_group = kGroupM * grid_n;
     const int group = pid / in_group;
     const int first_m = group * kGroupM;
@@ -261,41 +136,240 @@ __device__ __forceinline__ void tile_coords(int bid, int grid_m, int grid_n, int
     pn = (pid % in_group) / size_m;
 }
 
+typedef __attribute__((address_space(3))) void* lds_ptr;
+typedef short short4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0), bytes,
+                                             0x00020000);
+}
+
+// K-major: rows r and r + 8 (one 16-lane group) differ in the low bit of the
+// slot; rows of one parity (the same half of a 256-byte bank line) take 8
+// distinct slots.
+__device__ __forceinline__ int kswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+// MF MFMAs with RD LDS reads and LD loads spread evenly between them.
+template <int MF, int RD, int LD, int Q>
+__device__ __forceinline__ void interleave_slot() {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    constexpr int r = RD * (Q + 1) / MF - RD * Q / MF;
+    constexpr int l = LD * (Q + 1) / MF - LD * Q / MF;
+    if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
+    if constexpr (l > 0) __builtin_amdgcn_sched_group_barrier(0x020, l, 0);
+}
+template <int MF, int RD, int LD, int... Q>
+__device__ __forceinline__ void interleave_slots(std::integer_sequence<int, Q...>) {
+    (interleave_slot<MF, RD, LD, Q>(), ...);
+}
+template <int MF, int RD, int LD>
+__device__ __forceinline__ void interleave() {
+    interleave_slots<MF, RD, LD>(std::make_integer_sequence<int, MF>{});
+}
+
+// One operand's panel of the tile kernel: R rows (M or N) by BK, 128 bytes of
+// K, loaded straight into LDS by W waves (buffer loads of 16 bytes a lane,
+// no registers in between) and read as NT 32-wide tiles a wave.  The buffer
+// resource covers exactly what the block may read, and a load past it writes
+// zeros, so ragged edges cost no branch:
+//   * K-major (element (r, k) at X[r ld + k]): LDS rows of 128 bytes, the
+//     16-byte chunk c of row r at slot c ^ kswz(r); chunks at or past K are
+//     sent out of range lane by lane (they would read the next row).
+//   * M/N-major (element (k, r) at X[k ld + r]): LDS rows (k) of R elements
+//     as they lie.  16-bit ones are read by ds_read_b64_tr_b16, whose 32
+//     lanes a clock take 64 bytes of four consecutive k: slots
+//     c ^ (2 (k & 3) ^ 8 (k & 1)) put those on four quarters of the banks
+//     (R of 128 and 256; rows of 64 take half a bank line each, and k and
+//     k + 2 swap halves).  float32 ones are read as four single floats a
+//     lane, the lane halves 4 rows of k apart: slots c ^ 8 ((k >> 2) & 1)
+//     put the halves on opposite 32 banks.  Rows at or past K read zeros;
+//     columns past R's edge read the next row's elements and only reach
+//     outputs that are not stored.
+template <typename T, bool KMAJOR, int R, int W, int NT>
+struct Panel {
+    using S = typename Elem<T>::storage;
+    static constexpr int E = sizeof(S), V = 16 / E, BK = Mfma<T>::BK;
+    static_assert(BK * E == 128, "a K tile is 128 bytes a row");
+    static constexpr int kIssue = R / 8 / W;        // load instructions per wave per K tile
+    static constexpr int kRowBytes = R * E;         // M/N-major LDS row
+    static constexpr int kPerLoad = 1024 / kRowBytes;  // its rows per load instruction
+    static constexpr int kFrags = KMAJOR ? 4 : NT;
+    static_assert(kIssue * 8 * W == R, "the waves share a panel's loads evenly");
+    // the slot of a lane's chunk must not depend on which of its loads it is
+    static_assert(KMAJOR || E == 2 ? W % 2 == 0 : (W * kPerLoad) % 8 == 0, "swizzle period");
+    // DS read instructions of one fragment set (two b64 or two paired b32
+    // reads a tile when M/N-major)
+    static constexpr int kReads = NT * (KMAJOR ? 1 : 2);
+
+    const char* base;
+    int64_t ld_bytes, bytes;  // bytes: readable from base (M/N-major: from k = 0)
+    uint32_t voff, kleft;     // kleft: K-major, elements of K from this lane's chunk of K tile 0 on
+    uint32_t frag[kFrags];
+
+    static __device__ __forceinline__ int slot_of(int c, int k) {
+        if constexpr (R == 32) return c;
+        else if constexpr (E == 4) return c ^ (8 * ((k >> 2) & 1));
+        else if constexpr (R >= 128) return c ^ ((2 * (k & 3)) ^ (8 * (k & 1)));
+        else return c ^ (4 * ((k >> 1) & 1));
+    }
+
+    __device__ __forceinline__ void init(const S* X, int64_t ld, int64_t r0, int64_t rows, int64_t K, int wave,
+                                         int lane, int wbase) {
+        const int l32 = lane % 32, half = lane / 32;
+        ld_bytes = ld * E;
+        if constexpr (KMAJOR) {
+            const int64_t mine = rows - r0 < R ? rows - r0 : R;
+            base = reinterpret_cast<const char*>(X) + r0 * ld_bytes;
+            // whole packets: an odd K comes with rows zero-padded to one
+            bytes = (mine - 1) * ld_bytes + (K + V - 1) / V * 16;
+            const int row = lane >> 3, chunk = (lane & 7) ^ kswz(8 * wave + row);
+            voff = static_cast<uint32_t>((8 * wave + row) * ld_bytes + chunk * 16);
+            kleft = static_cast<uint32_t>(K > chunk * V ? K - chunk * V : 0);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) frag[s] = (wbase + l32) * 128 + (((2 * s + half) ^ kswz(l32)) << 4);
+        } else {
+            constexpr int kSlots = kRowBytes / 16;
+            base = reinterpret_cast<const char*>(X + r0);
+            bytes = (K - 1) * ld_bytes + (rows - r0) * E;
+            const int k = wave * kPerLoad + lane / kSlots;
+            voff = static_cast<uint32_t>(k * ld_bytes + slot_of(lane % kSlots, k) * 16);
+            kleft = 0;
+            if constexpr (E == 2) {
+                // transposed reads: lane p of 16-lane group g addresses row
+                // 8 half + p / 4 and column 16 (g & 1) + 4 (p % 4)
+                const int g = lane / 16, pl = lane % 16;
+                const int krow = 8 * half + pl / 4;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const int col = wbase + t * 32 + 16 * (g & 1) + 4 * (pl % 4);
+                    frag[t] = krow * kRowBytes + (slot_of(col / 8, krow) << 4) + (col % 8) * 2;
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const int col = wbase + t * 32 + l32;
+                    frag[t] = 4 * half * kRowBytes + (slot_of(col / 4, 4 * half) << 4) + (col % 4) * 4;
+                }
+            }
+        }
+    }
+
+    // Loads of K tile kt into `tile` (this wave's share); past the last K
+    // tile every load is out of range.
+    __device__ __forceinline__ void issue(int kt, char* tile, int wave) const {
+        uint32_t off;
+        const char* from;
+        int64_t left;
+        if constexpr (KMAJOR) {
+            from = base;
+            left = bytes;
+            const uint32_t k0 = static_cast<uint32_t>(kt) * BK;
+            off = k0 < kleft ? voff + k0 * E : kOutOfRange;
+        } else {
+            const int64_t skip = static_cast<int64_t>(kt) * BK * ld_bytes;
+            from = base + skip;
+            left = bytes - skip;
+            if (left < 0) left = 0;
+            off = voff;
+        }
+        const uint32_t records = left < int64_t{kOutOfRange} ? static_cast<uint32_t>(left) : kOutOfRange;
+        const __amdgpu_buffer_rsrc_t res = rsrc(from, records);
+        const uint32_t step = static_cast<uint32_t>((KMAJOR ? 8 * W : W * kPerLoad) * ld_bytes);
+#pragma unroll
+        for (int i = 0; i < kIssue; ++i) {
+            // an out-of-range lane stays so: its offset only needs not to wrap
+            const uint32_t at = KMAJOR ? (off == kOutOfRange ? kOutOfRange : off + i * step) : off + i * step;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lds_ptr)(tile + (i * W + wave) * 1024), 16, at, 0, 0, 0);
+        }
+    }
+
+    // The fragment of substep s for the wave's 32-wide tile t: 16 bytes of K
+    // a lane.
+    __device__ __forceinline__ uint4 read(const char* tile, int t, int s) const {
+        if constexpr (KMAJOR) {
+            return *reinterpret_cast<const uint4*>(tile + t * 32 * 128 + frag[s]);
+        } else if constexpr (E == 2) {
+            const char* q = tile + frag[t] + s * 16 * kRowBytes;
+            const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(q));
+            const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) short4_t*)(q + 4 * kRowBytes));
+            uint4 v;
+            __builtin_memcpy(&v, &lo, 8);
+            __builtin_memcpy(reinterpret_cast<char*>(&v) + 8, &hi, 8);
+            return v;
+        } else {
+            const char* q = tile + frag[t] + s * 8 * kRowBytes;
+            uint4 v;
+            v.x = *reinterpret_cast<const uint32_t*>(q);
+            v.y = *reinterpret_cast<const uint32_t*>(q + kRowBytes);
+            v.z = *reinterpret_cast<const uint32_t*>(q + 2 * kRowBytes);
+            v.w = *reinterpret_cast<const uint32_t*>(q + 3 * kRowBytes);
+            return v;
+        }
+    }
+};
+
 // F32OUT: C is float32 (split-K partials of a 16-bit product), written as
 // alpha acc with no Cin.
-template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int WM, int WN, bool F32OUT = false>
-__global__ __launch_bounds__(WM * WN * kWave) void gemm_mfma_kernel(GemmArgs p) {
+//
+// Four waves (2 x 2), a K step a 128-byte slab of K, STAGES LDS stages.  A
+// step runs its four substeps' MFMAs with the next substep's fragment reads
+// between them, and in the first the loads of the K tile STAGES - 1 ahead.
+// After the third it waits until the next K tile's loads have landed (later
+// tiles' stay in flight), passes the one barrier and reads the next step's
+// first fragments under the last substep's MFMAs.  With two stages A of the
+// tile after next goes out there too, into the stage just left.  Nothing but MFMAs stands
+// between two barriers but the wait itself: the kernel this replaced staged
+// tiles through registers and LDS stores, and its waves met at the end of
+// each step with the matrix pipe idle (float32 4096^3 85 % busy).
+// BLOCKS is how many blocks a CU holds (LDS and registers).
+template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT>
+__global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p) {
     using S = typename Elem<T>::storage;
-    constexpr int THREADS = WM * WN * kWave;
-    using LA = TileLoader<T, BM, A_KMAJOR, THREADS>;
-    using LB = TileLoader<T, BN, B_KMAJOR, THREADS>;
-    constexpr int BK = Mfma<T>::BK, KSUB = Mfma<T>::KSUB;
-    constexpr int LDS_STRIDE = LA::LDS_STRIDE;
+    constexpr int WM = BM >= 64 ? 2 : 1, WN = 4 / WM, W = WM * WN;
+    constexpr int BK = Mfma<T>::BK;
     constexpr int kWaveM = BM / WM, kWaveN = BN / WN;
     constexpr int TM = kWaveM / 32, TN = kWaveN / 32;
-    constexpr int STAGE = (BM + BN) * LDS_STRIDE;  // elements per LDS stage
-    __shared__ __attribute__((aligned(16))) S lds[2 * STAGE];
+    using PA = Panel<T, A_KMAJOR, BM, W, TM>;
+    using PB = Panel<T, B_KMAJOR, BN, W, TN>;
+    constexpr int ATILE = BM * 128, STAGE = (BM + BN) * 128;
+    // An object a stage, so the compiler can tell the ones being filled from
+    // the one being read and leaves the loads in flight.
+    static_assert(STAGES >= 2 && STAGES <= 4, "LDS stages");
+    __shared__ __attribute__((aligned(1024))) char lds0[STAGE];
+    __shared__ __attribute__((aligned(1024))) char lds1[STAGE];
+    __shared__ __attribute__((aligned(1024))) char lds2[STAGES > 2 ? STAGE : 16];
+    __shared__ __attribute__((aligned(1024))) char lds3[STAGES > 3 ? STAGE : 16];
+    auto stage_at = [&](auto i) -> char* {
+        constexpr int I = decltype(i)::value % STAGES;
+        if constexpr (I == 0) return lds0;
+        else if constexpr (I == 1) return lds1;
+        else if constexpr (I == 2) return lds2;
+        else return lds3;
+    };
 
     const int grid_m = static_cast<int>((p.m + BM - 1) / BM);
     const int grid_n = static_cast<int>((p.n + BN - 1) / BN);
     int pm, pn;
     tile_coords(blockIdx.x, grid_m, grid_n, pm, pn);
     const int64_t m0 = static_cast<int64_t>(pm) * BM, n0 = static_cast<int64_t>(pn) * BN;
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int lane = threadIdx.x % kWave;
     const int wm = wave / WN, wn = wave % WN;
     const int half = lane / 32, l32 = lane % 32;
 
     // One batch entry per blockIdx.z (the host launches batches of at most
-    // 65535); a loop over the batch here would keep every address live
-    // across it and spill.
+    // 65535).
     {
         const int64_t bi = blockIdx.z;
         // Split-K partials: batch entry bi is the slice k = bi k .. of the
         // product's k_total, the last one shorter when k does not divide it.
         const int64_t kk = F32OUT && p.k_total - bi * p.k < p.k ? p.k_total - bi * p.k : p.k;
-        const int64_t nk = (kk + BK - 1) / BK;
-        const S* A = static_cast<const S*>(p.a) + bi * p.stride_a;
-        const S* B = static_cast<const S*>(p.b) + bi * p.stride_b;
+        const int nk = static_cast<int>((kk + BK - 1) / BK);
+        PA oa;
+        PB ob;
+        oa.init(static_cast<const S*>(p.a) + bi * p.stride_a, p.lda, m0, p.m, kk, wave, lane, wm * kWaveM);
+        ob.init(static_cast<const S*>(p.b) + bi * p.stride_b, p.ldb, n0, p.n, kk, wave, lane, wn * kWaveN);
         f32x16 acc[TM][TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -304,76 +378,88 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_mfma_kernel(GemmArgs p) 
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-        LA la;
-        LB lb;
-        // Prologue: K tile 0 into stage 0, K tile 1 in flight.
-        la.load(A, p.lda, m0, p.m, 0, kk);
-        lb.load(B, p.ldb, n0, p.n, 0, kk);
-        la.store(lds);
-        lb.store(lds + BM * LDS_STRIDE);
-        if (nk > 1) {
-            la.load(A, p.lda, m0, p.m, BK, kk);
-            lb.load(B, p.ldb, n0, p.n, BK, kk);
-        }
-        __syncthreads();
-        for (int64_t kt = 0; kt < nk; ++kt) {
-            const S* As = lds + (kt & 1) * STAGE;
-            const S* Bs = As + BM * LDS_STRIDE;
-            // Fragments are double-buffered across the K substeps: the LDS
-            // reads for substep s + 1 are issued before the MFMAs of s, so
-            // their latency hides behind the matrix work.
-            constexpr int NSUB = BK / KSUB;
-            uint4 af[2][TM], bf[2][TN];
-            // A lane's 4 consecutive k (k0 + j for component j) of row or
-            // column `rc`, from either LDS layout.
-            auto frag = [&](const S* base, int rc, int k0, auto krows) -> uint4 {
-                if constexpr (decltype(krows)::value) {
-                    constexpr int KS = LA::KR_STRIDE;
-                    static_assert(KS == LB::KR_STRIDE, "float32 tiles of one width");
-                    const S* q = base + k0 * KS + rc;
-                    uint4 v;
-                    __builtin_memcpy(&v.x, q, 4);
-                    __builtin_memcpy(&v.y, q + KS, 4);
-                    __builtin_memcpy(&v.z, q + 2 * KS, 4);
-                    __builtin_memcpy(&v.w, q + 3 * KS, 4);
-                    return v;
-                } else {
-                    return *reinterpret_cast<const uint4*>(base + rc * LDS_STRIDE + k0);
+        uint4 af[2][TM], bf[2][TN];
+        auto fetch = [&](const char* stage, int s, int buf) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) af[buf][i] = oa.read(stage, i, s);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bf[buf][j] = ob.read(stage + ATILE, j, s);
+        };
+        auto mma = [&](int buf) { Mfma<T>::template tiles<TM, TN>(af[buf], bf[buf], acc); };
+        constexpr int kMf = TM * TN * Mfma<T>::kPerTile;
+        constexpr int kReads = PA::kReads + PB::kReads;
+        // The loads a wave may leave in flight when it passes the barrier of a
+        // step: those of the K tiles after the next.
+        constexpr int kAhead = (STAGES - 2) * (PA::kIssue + PB::kIssue);
+        constexpr int kWait = (kAhead & 15) | (7 << 4) | ((kAhead >> 4) << 14);  // vmcnt(kAhead) lgkmcnt(0)
+        auto meet = [&]() {
+            __builtin_amdgcn_s_waitcnt(kWait);
+            // A bare barrier: the fence of __syncthreads() would wait for
+            // every load.
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        auto body = [&](auto at, int kt) {
+            constexpr int I = decltype(at)::value;
+            char* cur = stage_at(std::integral_constant<int, I>{});
+            char* next = stage_at(std::integral_constant<int, I + 1>{});
+            char* fill = stage_at(std::integral_constant<int, I + STAGES - 1>{});
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                fetch(cur, s + 1, (s + 1) & 1);
+                if (s == 0) {
+                    if (STAGES > 2) oa.issue(kt + STAGES - 1, fill, wave);
+                    ob.issue(kt + STAGES - 1, fill + ATILE, wave);
                 }
-            };
-            auto fetch = [&](int s, int buf) {
-                const int k0 = s * KSUB + half * (KSUB / 2);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-                    af[buf][i] = frag(As, wm * kWaveM + i * 32 + l32, k0, std::integral_constant<bool, LA::KROWS>{});
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    bf[buf][j] = frag(Bs, wn * kWaveN + j * 32 + l32, k0, std::integral_constant<bool, LB::KROWS>{});
-            };
-            fetch(0, 0);
-#pragma unroll
-            for (int s = 0; s < NSUB; ++s) {
-                if (s + 1 < NSUB) fetch(s + 1, (s + 1) & 1);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = Mfma<T>::mma(af[s & 1][i], bf[s & 1][j], acc[i][j]);
+                mma(s & 1);
+                if (s == 0) {
+                    interleave<kMf, kReads, PB::kIssue + (STAGES > 2 ? PA::kIssue : 0)>();
+                } else {
+                    interleave<kMf, kReads, 0>();
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            // The other stage was last read in step kt - 1, before the
-            // barrier that ended it: fill it with K tile kt + 1 and start
-            // loading tile kt + 2.
-            if (kt + 1 < nk) {
-                S* next = lds + ((kt + 1) & 1) * STAGE;
-                la.store(next);
-                lb.store(next + BM * LDS_STRIDE);
+            meet();
+            fetch(next, 0, 0);
+            if (STAGES == 2) oa.issue(kt + 2, cur, wave);
+            mma(1);
+            interleave<kMf, kReads, STAGES == 2 ? PA::kIssue : 0>();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto prologue = [&](auto i) {
+            constexpr int I = decltype(i)::value;
+            if constexpr (I < STAGES - 1) {
+                oa.issue(I, stage_at(i), wave);
+                ob.issue(I, stage_at(i) + ATILE, wave);
+            } else if constexpr (STAGES == 2) {
+                oa.issue(1, lds1, wave);
             }
-            if (kt + 2 < nk) {
-                la.load(A, p.lda, m0, p.m, (kt + 2) * BK, kk);
-                lb.load(B, p.ldb, n0, p.n, (kt + 2) * BK, kk);
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        prologue(I0{});
+        prologue(I1{});
+        if constexpr (STAGES > 2) prologue(I2{});
+        meet();
+        fetch(lds0, 0, 0);
+        for (int kt = 0; kt < nk; kt += STAGES) {
+            body(I0{}, kt);
+            if (kt + 1 >= nk) break;
+            body(I1{}, kt + 1);
+            if constexpr (STAGES > 2) {
+                if (kt + 2 >= nk) break;
+                body(I2{}, kt + 2);
             }
-            __syncthreads();
+            if constexpr (STAGES > 3) {
+                if (kt + 3 >= nk) break;
+                body(I3{}, kt + 3);
+            }
         }
+        // the last steps' out-of-range loads still write LDS
+        __builtin_amdgcn_s_waitcnt(0);
 
         // Epilogue: lane holds column l32 of each 32 x 32 tile, rows
         // 8 * (e / 4) + 4 * half + e % 4 for accumulator element e.
@@ -398,54 +484,6 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_mfma_kernel(GemmArgs p) 
         }
         S* C = static_cast<S*>(p.c) + bi * p.stride_c;
         const S* Cin = static_cast<const S*>(p.cin);
-        if (p.trans_c) {
-            // C^T: a lane's four consecutive rows r..r+3 of column `col` are
-            // four consecutive elements of row `col` of the stored C, one
-            // store when they are all inside and 16-byte aligned.  A store
-            // instruction then covers 32 rows of C with 32 bytes each, and
-            // the four of a row group complete each 128-byte line: these
-            // stores keep the default cache policy, so L2 joins the pieces
-            // before they reach HBM (float32 4096^3 as C^T: 1077 us, against
-            // 1118 us with non-temporal stores, which reach memory as
-            // partial lines).
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int64_t col = n0 + wn * kWaveN + j * 32 + l32;
-                    const int64_t rbase = m0 + wm * kWaveM + i * 32 + 4 * half;
-                    if (col >= p.n) continue;
-                    S* cp = C + col * p.ldc + rbase;
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        float v[4];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const float a = p.alpha * acc[i][j][4 * g + r];
-                            const int64_t row = rbase + 8 * g + r;
-                            if (p.beta == 0.0f || row >= p.m) {
-                                v[r] = a;  // rows past M are not stored
-                            } else {
-                                const float c = Elem<T>::load(Cin[bi * p.cin_stride_b + row * p.cin_rs + col * p.cin_cs]);
-                                v[r] = fmaf(p.beta, c, a);
-                            }
-                        }
-                        S* dst = cp + 8 * g;
-                        if constexpr (sizeof(S) == 4) {
-                            if (rbase + 8 * g + 3 < p.m && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-                                *reinterpret_cast<uint4*>(dst) = make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]),
-                                                                            __float_as_uint(v[2]), __float_as_uint(v[3]));
-                                continue;
-                            }
-                        }
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            if (rbase + 8 * g + r < p.m) dst[r] = Elem<T>::store(v[r]);
-                        }
-                    }
-                }
-            return;
-        }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -527,21 +565,9 @@ namespace big {
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int TILE = 256 * 128;   // bytes per operand tile
 constexpr int STAGE = 2 * TILE;   // bytes per LDS stage
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef short short4_t __attribute__((ext_vector_type(4)));
-
-// K-major: rows r and r + 8 (one 16-lane group) differ in the low bit of the
-// slot; rows of one parity (the same half of a 256-byte bank line) take 8
-// distinct slots.
-__device__ __forceinline__ int kswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 // M/N-major: rows k..k+3 move a 4-chunk span (64 bytes) to four distinct
 // quarters of a bank line, and a 2-chunk span to four distinct slots mod 8.
 __device__ __forceinline__ int nswz(int k) { return (2 * (k & 3)) ^ (8 * (k & 1)); }
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0), bytes,
-                                             0x00020000);
-}
 
 // One operand: the block's 256-wide panel of X (M or N from mn0), loaded by
 // W waves, read as T 32-wide tiles per wave.
@@ -615,24 +641,6 @@ struct Operand {
         }
     }
 };
-
-// MF MFMAs with RD LDS reads and LD loads spread evenly between them.
-template <int MF, int RD, int LD, int Q>
-__device__ __forceinline__ void interleave_slot() {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    constexpr int r = RD * (Q + 1) / MF - RD * Q / MF;
-    constexpr int l = LD * (Q + 1) / MF - LD * Q / MF;
-    if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
-    if constexpr (l > 0) __builtin_amdgcn_sched_group_barrier(0x020, l, 0);
-}
-template <int MF, int RD, int LD, int... Q>
-__device__ __forceinline__ void interleave_slots(std::integer_sequence<int, Q...>) {
-    (interleave_slot<MF, RD, LD, Q>(), ...);
-}
-template <int MF, int RD, int LD>
-__device__ __forceinline__ void interleave() {
-    interleave_slots<MF, RD, LD>(std::make_integer_sequence<int, MF>{});
-}
 
 template <typename T, bool A_KMAJOR, bool B_KMAJOR, int WM, int WN>
 __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kernel(GemmArgs p) {
@@ -984,15 +992,25 @@ void launch(const GemmArgs& p, hipStream_t stream) {
 
 // An operand the matrix-core kernels read in place: 16-byte aligned, and its
 // leading dimension, batch stride and contiguous extent (K when K-major, M or
-// N otherwise) whole numbers of V-element packets.
+// N otherwise) whole numbers of V-element packets; rows that do not overlap
+// (the panel's bound then is the end of its last row) and a panel (up to 256
+// rows of K, or a K tile of rows) under 4 GiB, the reach of its resource.
+template <typename T>
+bool panel_fits(int64_t ld, bool kmajor) {
+    constexpr int64_t E = sizeof(typename Elem<T>::storage);
+    const int64_t rows = !kmajor ? Mfma<T>::BK : E == 2 ? 256 : 128;  // the tallest tile, or a K tile
+    return ld >= 0 && ld < ((int64_t{1} << 32) - 4096) / (rows * E);
+}
+
 template <typename T>
 bool operand_ok(const void* ptr, int64_t ld, int64_t stride, bool kmajor, int64_t mn, int64_t k) {
     constexpr int V = Mfma<T>::V;
-    return aligned16(ptr) && ld % V == 0 && stride % V == 0 && (kmajor ? k : mn) % V == 0;
+    return aligned16(ptr) && ld % V == 0 && stride % V == 0 && (kmajor ? k : mn) % V == 0 &&
+           ((kmajor ? mn : k) == 1 || ld >= (kmajor ? k : mn)) && panel_fits<T>(ld, kmajor);
 }
 
 bool tiles_fit(const GemmArgs& p) {
-    return (p.m + 127) / 128 * ((p.n + 127) / 128) < (int64_t(1) << 31);
+    return (p.m + 63) / 64 * ((p.n + 63) / 64) < (int64_t(1) << 31) && p.k < (int64_t(1) << 31);
 }
 
 template <typename T>
@@ -1001,25 +1019,25 @@ bool mfma_eligible(const GemmArgs& p) {
            operand_ok<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, p.k) && tiles_fit(p);
 }
 
-template <typename T, int BM, int BN, int WM, int WN, bool F32OUT = false>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false>
 void launch_chunk(const GemmArgs& p, hipStream_t stream) {
-    constexpr int THREADS = WM * WN * kWave;
+    constexpr int THREADS = 4 * kWave;
     const int64_t tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
     const dim3 grid(static_cast<unsigned>(tiles), 1u, static_cast<unsigned>(p.batch));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     if (a_kmajor && b_kmajor) {
-        gemm_mfma_kernel<T, true, true, BM, BN, WM, WN, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
     } else if (a_kmajor) {
-        gemm_mfma_kernel<T, true, false, BM, BN, WM, WN, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
     } else if (b_kmajor) {
-        gemm_mfma_kernel<T, false, true, BM, BN, WM, WN, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
     } else {
-        gemm_mfma_kernel<T, false, false, BM, BN, WM, WN, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
     }
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
 
-template <typename T, int BM, int BN, int WM, int WN, bool F32OUT = false>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false>
 void launch_config(const GemmArgs& whole, hipStream_t stream) {
     constexpr int64_t kMaxZ = 65535;
     using S = typename Elem<T>::storage;
@@ -1032,254 +1050,227 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
                      : static_cast<void*>(static_cast<S*>(whole.c) + b0 * whole.stride_c);
         if (whole.cin != nullptr) p.cin = static_cast<const S*>(whole.cin) + b0 * whole.cin_stride_b;
         if (F32OUT) p.k_total = whole.k_total - b0 * whole.k;
-        launch_chunk<T, BM, BN, WM, WN, F32OUT>(p, stream);
+        launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT>(p, stream);
     }
 }
-// Split K for float32 products with too few 128 x 128 tiles to fill the
-// CUs: a single matrix whose K dwarfs M x N (mm 1024^3 has 64 tiles; the
-// Linear(4096, 1024) of a 256-row batch has 16, each running K = 4096 alone
-// on one CU).  S slices of K ride on the kernel's batch index and write
-// float32 partial products into a workspace [S][M][N]; splitk_finish_kernel
-// then adds the slices in slice order -- the result does not depend on
-// timing -- and applies alpha, beta Cin and the epilogue's rounding.
-// S doubles while the tiles times S still fit one block per CU and every
-// slice keeps at least 128 of K, a multiple of the kernel's BK = 32.
 constexpr int kFinishBlock = 256;
 
-int splitk_slices(const GemmArgs& p, int cus, int tile = 128, int min_k = 128, int bk = 32) {
-    if (p.batch != 1) return 1;
-    const int64_t tiles = ((p.m + tile - 1) / tile) * ((p.n + tile - 1) / tile);
-    int s = 1;
-    while (tiles * s * 2 <= cus && p.k % (s * 2 * bk) == 0 && p.k / (s * 2) >= min_k) s *= 2;
-    return s;
-}
-
-// Slice 0 + slice 1 + ... of element i, added in slice order; the loads go
-// out four at a time ahead of their adds.
-__device__ __forceinline__ float sum_slices(const float* part, int slices, int64_t mn, int64_t i) {
-    float acc = part[i];
-    int s = 1;
-    for (; s + 4 <= slices; s += 4) {
-        const float v0 = part[s * mn + i], v1 = part[(s + 1) * mn + i];
-        const float v2 = part[(s + 2) * mn + i], v3 = part[(s + 3) * mn + i];
-        acc += v0;
-        acc += v1;
-        acc += v2;
-        acc += v3;
-    }
-    for (; s < slices; ++s) acc += part[s * mn + i];
-    return acc;
-}
-
-// A float32 product of 33 to 64 rows (or columns) against a wide operand of
-// at least 128 tiles of 64 (a small batch through a Linear of 8192 or more
-// outputs): 64 x 64 tiles of two waves, K split up to four blocks a CU.
-// The thin kernel leaves these here.  Measured (64 x 11008 x 4096, W
-// rotated beyond the Infinity Cache): x W^T 91-95 against 104-114 us on
-// the thin kernel, x W 94-102 against 106-140 us; with 4096 columns (64
-// tiles) the thin kernel stays faster (101-110 against 109-114 us).
-int splitk32_small_batch(const GemmArgs& p, int cus) {
-    const int64_t thin = std::min(p.m, p.n), wide = std::max(p.m, p.n);
-    if (p.batch != 1 || thin <= 32 || thin > 64 || (wide + 63) / 64 < 128) return 1;
-    return splitk_slices(p, 4 * cus, 64);
-}
-
 // c = alpha * sum of the slices (+ beta Cin), the same expressions as the
-// kernels' epilogue; one thread an element, consecutive threads along a row.
-__global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(const float* part, int slices, int64_t m,
-                                                               int64_t n, float alpha, float beta,
-                                                               const float* cin, int64_t cin_rs,
-                                                               int64_t cin_cs, float* c, int64_t ldc) {
-    const int64_t mn = m * n;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kFinishBlock + threadIdx.x; i < mn;
-         i += static_cast<int64_t>(gridDim.x) * kFinishBlock) {
-        const float acc = sum_slices(part, slices, mn, i);
-        const int64_t r = i / n, col = i % n;
-        float v;
-        if (beta == 0.0f) {
-            v = alpha * acc;
-        } else if (cin_rs == 0) {
-            v = fmaf(alpha, acc, beta * cin[col * cin_cs]);
-        } else {
-            v = fmaf(beta, cin[r * cin_rs + col * cin_cs], alpha * acc);
-        }
-        c[r * ldc + col] = v;
-    }
-}
-
-template <int BM, int BN, int WM, int WN>
-void launch_splitk(const GemmArgs& p, int slices, hipStream_t stream, int device) {
-    const int64_t mn = p.m * p.n;
-    Workspace ws(static_cast<size_t>(slices * mn) * sizeof(float), device);
-    GemmArgs q = p;
-    q.batch = slices;
-    q.k = p.k / slices;
-    q.stride_a = p.trans_a ? q.k * p.lda : q.k;  // slice s starts at k = s q.k
-    q.stride_b = p.trans_b ? q.k : q.k * p.ldb;
-    q.alpha = 1.0f;
-    q.beta = 0.0f;
-    q.cin = nullptr;
-    q.c = ws.get();
-    q.ldc = p.n;
-    q.stride_c = mn;
-    launch_config<float, BM, BN, WM, WN>(q, stream);
-    const int64_t blocks = std::min<int64_t>((mn + kFinishBlock - 1) / kFinishBlock, 4 * int64_t{cu_count(device)});
-    splitk_finish_kernel<<<static_cast<unsigned>(blocks), kFinishBlock, 0, stream>>>(
-        static_cast<const float*>(ws.get()), slices, p.m, p.n, p.alpha, p.beta,
-        static_cast<const float*>(p.cin), p.cin_rs, p.cin_cs, static_cast<float*>(p.c), p.ldc);
-    TP_AMD_HIP_CHECK(hipGetLastError());
-}
-
-// The same split for 16-bit products: the slices write float32 partials
-// (the tile kernel's F32OUT epilogue) and the finish adds them in slice
-// order and rounds once to the output type.
-template <typename T>
-__global__ __launch_bounds__(kFinishBlock) void splitk_finish16_kernel(
+// kernels' epilogue, rounded once to the output type.  A thread takes V
+// consecutive columns of a row (V = 4 when the row length, ldc and C's
+// address allow whole vectors, else 1) and adds slice 0 + slice 1 + ... in
+// slice order, four slices' loads out at a time.  blockIdx.y walks the rows,
+// so no index is divided.  Float32 partials just written: bound by the
+// launch and one round trip (256 x 4096 in 4 slices 9.2 us with one element a
+// thread and 64-bit divisions, 4.0 us so).
+template <typename T, int V>
+__global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(
     const float* part, int slices, int64_t m, int64_t n, float alpha, float beta,
     const typename Elem<T>::storage* cin, int64_t cin_rs, int64_t cin_cs, typename Elem<T>::storage* c,
     int64_t ldc) {
+    typedef float Vec __attribute__((ext_vector_type(V)));
+    const int64_t col = (static_cast<int64_t>(blockIdx.x) * kFinishBlock + threadIdx.x) * V;
+    if (col >= n) return;
     const int64_t mn = m * n;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kFinishBlock + threadIdx.x; i < mn;
-         i += static_cast<int64_t>(gridDim.x) * kFinishBlock) {
-        const float acc = sum_slices(part, slices, mn, i);
-        const int64_t r = i / n, col = i % n;
-        float v;
-        if (beta == 0.0f) {
-            v = alpha * acc;
-        } else if (cin_rs == 0) {
-            v = fmaf(alpha, acc, beta * Elem<T>::load(cin[col * cin_cs]));
-        } else {
-            v = fmaf(beta, Elem<T>::load(cin[r * cin_rs + col * cin_cs]), alpha * acc);
+    for (int64_t r = blockIdx.y; r < m; r += gridDim.y) {
+        const float* at = part + r * n + col;
+        auto slice = [&](int s) { return *reinterpret_cast<const Vec*>(at + s * mn); };
+        Vec acc = slice(0);
+        int s = 1;
+        for (; s + 4 <= slices; s += 4) {
+            const Vec v0 = slice(s), v1 = slice(s + 1), v2 = slice(s + 2), v3 = slice(s + 3);
+            acc += v0;
+            acc += v1;
+            acc += v2;
+            acc += v3;
         }
-        c[r * ldc + col] = Elem<T>::store(v);
+        for (; s < slices; ++s) acc += slice(s);
+        typename Elem<T>::storage out[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            float v;
+            if (beta == 0.0f) {
+                v = alpha * acc[j];
+            } else if (cin_rs == 0) {
+                v = fmaf(alpha, acc[j], beta * Elem<T>::load(cin[(col + j) * cin_cs]));
+            } else {
+                v = fmaf(beta, Elem<T>::load(cin[r * cin_rs + (col + j) * cin_cs]), alpha * acc[j]);
+            }
+            out[j] = Elem<T>::store(v);
+        }
+        if constexpr (V == 4 && sizeof(out) == 16) {
+            *reinterpret_cast<uint4*>(c + r * ldc + col) = __builtin_bit_cast(uint4, out);
+        } else if constexpr (V == 4) {
+            *reinterpret_cast<uint2*>(c + r * ldc + col) = __builtin_bit_cast(uint2, out);
+        } else {
+            c[r * ldc + col] = out[0];
+        }
     }
 }
 
-// The 16-bit split: the most slices that keep the 128 x 128 tiles times
-// the slices within two blocks a CU, with slices of a multiple of BK and at
-// least kSplit16MinK; the last slice is shorter when K is not a multiple of
-// the slice.  A product of one row of tiles (a small batch, min(M, N) <=
-// 128) takes slices of kSplit16ShortK when that still gives every CU a
-// block: bf16 17-64 x 11008 x 4096 26-32 us against 29-34 us, 128 x 4096
-// x 4096 22.4 against 24.5 us (W rotated beyond the Infinity Cache).  With
-// more rows of tiles the extra partials cost more than the blocks gain
-// (256 x 4096 x 4096 30.9 against 29.1 us), and 1024^3 in slices of 512
-// ran 19.5 against 13.5 us unsplit.
-struct SplitPlan {
-    int64_t slices = 1, ks = 0;
-};
-
-constexpr int64_t kSplit16MinK = 1024;
-constexpr int64_t kSplit16ShortK = 512;
-
-SplitPlan splitk16_slices(const GemmArgs& p, int64_t max_blocks, int64_t min_k, int64_t bk) {
-    SplitPlan plan;
-    if (p.batch != 1) return plan;
-    const int64_t tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
-    for (int64_t s = max_blocks / tiles; s > 1; --s) {
-        const int64_t ks = ((p.k + s - 1) / s + bk - 1) / bk * bk;
-        if (ks < min_k) continue;
-        plan.ks = ks;
-        plan.slices = (p.k + ks - 1) / ks;
-        break;
-    }
-    return plan;
-}
-
-SplitPlan splitk16_plan(const GemmArgs& p, int64_t cus, int64_t bk) {
-    if (std::min(p.m, p.n) <= 128) {
-        const int64_t tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
-        const SplitPlan short_plan = splitk16_slices(p, 2 * cus, kSplit16ShortK, bk);
-        if (short_plan.slices > 1 && tiles * short_plan.slices >= cus) return short_plan;
-    }
-    return splitk16_slices(p, 2 * cus, kSplit16MinK, bk);
-}
-
-template <typename T, int BM, int BN, int WM, int WN>
-void launch_splitk16(const GemmArgs& p, const SplitPlan& plan, hipStream_t stream, int device) {
+template <typename T>
+void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t stream) {
     using S = typename Elem<T>::storage;
+    const bool vec = p.n % 4 == 0 && p.ldc % 4 == 0 &&
+                     (reinterpret_cast<uintptr_t>(p.c) & (4 * sizeof(S) - 1)) == 0;
+    const int64_t cols = vec ? p.n / 4 : p.n;
+    const dim3 grid(static_cast<unsigned>((cols + kFinishBlock - 1) / kFinishBlock),
+                    static_cast<unsigned>(std::min<int64_t>(p.m, 65535)));
+    auto* kernel = vec ? splitk_finish_kernel<T, 4> : splitk_finish_kernel<T, 1>;
+    kernel<<<grid, kFinishBlock, 0, stream>>>(part, slices, p.m, p.n, p.alpha, p.beta,
+                                              static_cast<const S*>(p.cin), p.cin_rs, p.cin_cs,
+                                              static_cast<S*>(p.c), p.ldc);
+    TP_AMD_HIP_CHECK(hipGetLastError());
+}
+
+// Splits K: the slices, K tiles of ks = a multiple of BK (the last one
+// shorter), ride on the tile kernel's batch index and write float32 partial
+// products into a workspace [slices][M][N]; splitk_finish_kernel then adds
+// them in slice order, so the result does not depend on timing.
+template <typename T, int BM, int BN, int STAGES, int BLOCKS>
+void launch_split(const GemmArgs& p, int64_t slices, int64_t ks, hipStream_t stream, int device) {
     const int64_t mn = p.m * p.n;
-    const int64_t slices = plan.slices;
     Workspace ws(static_cast<size_t>(slices * mn) * sizeof(float), device);
     GemmArgs q = p;
     q.batch = slices;
-    q.k = plan.ks;
+    q.k = ks;
     q.k_total = p.k;
-    q.stride_a = p.trans_a ? q.k * p.lda : q.k;  // slice s starts at k = s q.k
-    q.stride_b = p.trans_b ? q.k : q.k * p.ldb;
+    q.stride_a = p.trans_a ? ks * p.lda : ks;  // slice s starts at k = s ks
+    q.stride_b = p.trans_b ? ks : ks * p.ldb;
     q.alpha = 1.0f;
     q.beta = 0.0f;
     q.cin = nullptr;
     q.c = ws.get();
     q.ldc = p.n;
     q.stride_c = mn;
-    launch_config<T, BM, BN, WM, WN, true>(q, stream);
-    const int64_t blocks = std::min<int64_t>((mn + kFinishBlock - 1) / kFinishBlock, 4 * int64_t{cu_count(device)});
-    splitk_finish16_kernel<T><<<static_cast<unsigned>(blocks), kFinishBlock, 0, stream>>>(
-        static_cast<const float*>(ws.get()), static_cast<int>(slices), p.m, p.n, p.alpha, p.beta,
-        static_cast<const S*>(p.cin), p.cin_rs, p.cin_cs, static_cast<S*>(p.c), p.ldc);
-    TP_AMD_HIP_CHECK(hipGetLastError());
+    launch_config<T, BM, BN, STAGES, BLOCKS, true>(q, stream);
+    launch_finish<T>(static_cast<const float*>(ws.get()), static_cast<int>(slices), p, stream);
 }
 
-// 16-bit types take the big tile when it still gives every CU a block;
-// float32 (bound by its much slower MFMA rate) keeps the small one, whose
-// registers fit without spilling.
+// The tile kernel's shapes (LDS stages, blocks a CU) and what each is for.
+enum class Tile {
+    k128,      // 128 x 128, 2 stages, 2 blocks a CU: several rounds of tiles
+    k128Deep,  // 128 x 128, 3 stages, 1 block a CU: one round (16-bit)
+    k64x128,   // 64 x 128: 16-bit 3 stages, 2 blocks
+    k64x128Many,  // 64 x 128: 16-bit 2 stages, 3 blocks
+    k64,       // 64 x 64: 16-bit 3 stages, 3 blocks; float32 2 stages, 4 blocks
+    k32x128,   // 32 x 128, 4 stages, 2 blocks (float32)
+};
+
+struct TilePlan {
+    Tile tile;
+    int64_t slices = 1, ks = 0;
+};
+
+int64_t tiles_of(const GemmArgs& p, int64_t bm, int64_t bn) {
+    return (p.m + bm - 1) / bm * ((p.n + bn - 1) / bn) * p.batch;
+}
+
+// At most `most` slices of at least min_k.
+TilePlan split_k(Tile tile, const GemmArgs& p, int64_t most, int64_t min_k, int64_t bk) {
+    TilePlan plan{tile};
+    const int64_t s = std::min(most, p.k / min_k);
+    if (p.batch != 1 || s < 2) return plan;
+    plan.ks = ((p.k + s - 1) / s + bk - 1) / bk * bk;
+    plan.slices = (p.k + plan.ks - 1) / plan.ks;
+    return plan;
+}
+
+// A product of few rows or columns (a small batch through a Linear) is bound
+// by reading the other operand: enough blocks with enough loads in flight,
+// whatever their tiles waste on padding rows.
+//   * 16-bit, up to 64: 64 x 64 tiles, split into slices of at least 1024
+//     for up to three blocks a CU and up to eight slices, or one a CU.
+//     Measured with W rotated past the Infinity Cache (bf16, x W^T, us, the
+//     thin kernel in brackets): 8 x 11008 x 4096 19.3 (23.9), 8 x 4096 x
+//     11008 20.5 (21.6), 48 x 11008 x 4096 23.0 (40.7), 48 x 2048 x 5504
+//     15.1 (22.1); x W 8 x 11008 x 4096 19.6 (26.3).  Unsplit with two
+//     rounds of tiles (a vocabulary) 64 x 128 tiles halve the blocks.
+//   * float32, 17 to 32 rows: 32 x 128 tiles (a taller tile's padding rows
+//     cost MFMA time there), one block a CU: 20 x 11008 x 4096 47.0 (54.6),
+//     20 x 4096 x 11008 45.3 (56.7).
+//   * float32, 33 to 64: 64 x 64 tiles, up to three blocks a CU: 48 x 4096 x
+//     11008 58.5 (102), 48 x 4096 x 4096 27.3 (40.2).
+template <typename T>
+TilePlan plan_small_batch(const GemmArgs& p, int64_t cus) {
+    constexpr int64_t BK = Mfma<T>::BK;
+    const int64_t t64 = tiles_of(p, 64, 64);
+    if constexpr (std::is_same<T, float>::value) {
+        if (p.m <= 32 && p.n > 64) return split_k(Tile::k32x128, p, cus / tiles_of(p, 32, 128), 512, BK);
+        return split_k(Tile::k64, p, 3 * cus / t64, 1024, BK);
+    } else {
+        if (t64 >= 2 * cus && p.m <= 64) return TilePlan{Tile::k64x128};
+        return split_k(Tile::k64, p, std::min(3 * cus / t64, std::max<int64_t>(8, cus / t64)), 1024, BK);
+    }
+}
+
+// Share of the CUs' time that tiles of this shape spend on outputs: whole
+// rounds of one tile a CU, padding included.
+double fill(const GemmArgs& p, int64_t bm, int64_t bn, int64_t cus) {
+    const int64_t tiles = tiles_of(p, bm, bn);
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    return double(p.m) * double(p.n) * double(p.batch) / (double(bm * bn) * double(rounds * cus));
+}
+
+template <typename T>
+TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
+    constexpr int64_t BK = Mfma<T>::BK;
+    const int64_t thin = std::min(p.m, p.n);
+    const int64_t t128 = tiles_of(p, 128, 128), t64 = tiles_of(p, 64, 64);
+    if constexpr (std::is_same<T, float>::value) {
+        if (p.batch == 1 && thin > 16 && thin <= 64) {
+            const TilePlan plan = plan_small_batch<T>(p, cus);
+            if (plan.slices > 1) return plan;
+        }
+        // MFMAs of 64 cycles leave LDS and L2 idle, so 64 x 64 tiles run
+        // within 7 % of 128 x 128 ones (8192 x 4096 x 4096 2010 against 1886
+        // us) and win as soon as the larger tiles leave CUs without work:
+        // 2048 x 3000 x 1000 102 against 125 us, 3000 x 1000 x 1000 55
+        // against 68, 256 x 4096 x 1024 22 against 66 (36 split in four).
+        if (fill(p, 128, 128, cus) * 1.07 >= fill(p, 64, 64, cus)) return TilePlan{Tile::k128};
+        // Still CUs without a tile and a K worth a second launch: 256 x 1024
+        // x 4096 70 -> 26 us in four slices, 512 x 1000 x 1000 21 -> 17 in
+        // two; 256^3 7.5 us whole, 9.1 split.
+        if (t64 < cus && p.k >= 768) return split_k(Tile::k64, p, cus / t64, 192, BK);
+        return TilePlan{Tile::k64};
+    } else {
+        if (thin <= 64) return plan_small_batch<T>(p, cus);
+        // One round of 128 x 128 tiles by splitting K: when K is long, or when
+        // one row of tiles reads a wide operand once.  1500 x 700 x 5000
+        // 30.8 us in three slices, 40.6 on 64 x 128 tiles whole; 1024 x 1536
+        // x 8192 41.8 against 44.5; 128 x 11008 x 4096 33.6 against 37.3 on
+        // 64 x 64 tiles; 1280 x 1280 x 3000 28.0 in two, 26.5 whole.
+        if (t128 >= cus / 4 && t128 <= cus / 2 && (p.k > 4096 || (thin <= 128 && t64 > cus && p.k >= 2048))) {
+            const TilePlan plan = split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
+            if (plan.slices > 1) return plan;
+        }
+        // Rounds of 128 x 128 tiles, two a CU.  A short K with at most half
+        // of the last round used takes twice the tiles, three a CU (3001 x
+        // 3072 x 768: 576 tiles 28.1 us, 1152 half tiles 25.5).
+        if (t128 > cus) {
+            const int64_t last = t128 % (2 * cus);
+            if (p.k <= 1024 && t128 > 2 * cus && last != 0 && last <= cus) return TilePlan{Tile::k64x128Many};
+            return TilePlan{Tile::k128};
+        }
+        // At most one round: one block a CU with a third stage (2048^3 22.7
+        // against 26.1 us on two, 3001 x 768 x 3072 28.1 against 39.6), the
+        // tile as large as still gives half the CUs one: 1777 x 1008 x 3336
+        // 26.0 us on 64 x 128 against 35.1 on 128 x 128, 1024 x 1024 x 4096
+        // 22.7 us on 64 x 64 against 25.5 on 64 x 128.
+        if (t128 > cus / 2) return TilePlan{Tile::k128Deep};
+        if (tiles_of(p, 64, 128) > cus / 2) return TilePlan{Tile::k64x128};
+        if (t64 >= cus || p.k <= 2048) return TilePlan{Tile::k64};
+        return split_k(Tile::k64, p, 2 * cus / t64, 1024, BK);
+    }
+}
+
 template <typename T>
 void launch_mfma(const GemmArgs& p, hipStream_t stream) {
     int device = 0;
     TP_AMD_HIP_CHECK(hipGetDevice(&device));
-    if constexpr (std::is_same<T, float>::value) {
-        const int cus = cu_count(device);
-        const int batch_split = splitk32_small_batch(p, cus);
-        if (batch_split > 1) {
-            launch_splitk<64, 64, 2, 1>(p, batch_split, stream, device);
-            return;
-        }
-        const int64_t tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128) * p.batch;
-        const int slices = splitk_slices(p, cus);
-        // A [M, K] K-contiguous with B [K, N] N-contiguous (plain mm, and
-        // the dX = dY W of a linear layer) is the slowest float32 layout;
-        // the same product as C^T = B^T A^T reads B^T with its M axis
-        // contiguous and A^T K-contiguous, the fastest one, and writes C
-        // transposed.  Measured at 4096^3, after warm-up, on one box: 1077 us
-        // this way, TT itself 1070 us; the NN kernel took 1257-1300 us.
-        if (!p.trans_a && !p.trans_b && !p.trans_c && slices == 1 && !(p.batch == 1 && tiles * 4 <= cus)) {
-            GemmArgs q = p;
-            q.m = p.n;
-            q.n = p.m;
-            q.a = p.b;
-            q.lda = p.ldb;
-            q.stride_a = p.stride_b;
-            q.trans_a = true;
-            q.b = p.a;
-            q.ldb = p.lda;
-            q.stride_b = p.stride_a;
-            q.trans_b = true;
-            q.cin_rs = p.cin_cs;
-            q.cin_cs = p.cin_rs;
-            q.trans_c = true;
-            launch_config<float, 128, 128, 2, 2>(q, stream);
-            return;
-        }
-        if (p.batch == 1 && tiles * slices * 4 <= cus) {
-            // A product that 128 x 128 tiles, even split over K, leave on
-            // under a quarter of the CUs (config 1's 256^3: 4 tiles, 8
-            // blocks): 64 x 64 tiles of two waves, split down to slices of
-            // 64 of K.
-            const int small = splitk_slices(p, cus, 64, 64);
-            if (small > 1) {
-                launch_splitk<64, 64, 2, 1>(p, small, stream, device);
-            } else {
-                launch_config<float, 64, 64, 2, 1>(p, stream);
-            }
-            return;
-        }
-        if (slices > 1) {
-            launch_splitk<128, 128, 2, 2>(p, slices, stream, device);
-            return;
-        }
-    }
-    if constexpr (sizeof(typename Elem<T>::storage) == 2) {
+    const int64_t cus = cu_count(device);
+    constexpr bool k16 = sizeof(typename Elem<T>::storage) == 2;
+    if constexpr (k16) {
         if (smallk::eligible<T>(p, cu_count(device))) {
             smallk::launch<T>(p, stream);
             return;
@@ -1288,31 +1279,30 @@ void launch_mfma(const GemmArgs& p, hipStream_t stream) {
             big::launch<T>(p, stream);
             return;
         }
-        const int64_t big_tiles = ((p.m + 255) / 256) * ((p.n + 255) / 256) * p.batch;
-        if (big_tiles >= cu_count(device)) {
-            launch_config<T, 256, 256, 2, 4>(p, stream);
-            return;
-        }
-        // Few 128 x 128 tiles and a long K (a Linear of a few hundred rows):
-        // split K (splitk16_plan), up to two blocks a CU.  Measured
-        // (bf16, this split against the tiles alone): 128 x 11008 x 4096
-        // 36.4 against 57.7 us, 128 x 4096 x 4096 22.4 against 42.6 us,
-        // 1024 x 1024 x 8192 41.5 against 81.4 us; 1024^3 in slices of 512
-        // was slower (19.5 against 13.5 us) and is not split.
-        const SplitPlan plan = splitk16_plan(p, cu_count(device), Mfma<T>::BK);
-        if (plan.slices > 1) {
-            launch_splitk16<T, 128, 128, 2, 2>(p, plan, stream, device);
-            return;
-        }
-        // Too few 128 x 128 tiles for a quarter of the CUs (mm 1024^2 has
-        // 64): 64 x 64 tiles of two waves.
-        const int64_t tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128) * p.batch;
-        if (tiles * 4 <= cu_count(device)) {
-            launch_config<T, 64, 64, 2, 1>(p, stream);
-            return;
-        }
     }
-    launch_config<T, 128, 128, 2, 2>(p, stream);
+    const TilePlan plan = plan_tiles<T>(p, cus);
+    if (plan.slices > 1) {
+        if constexpr (k16) {
+            if (plan.tile == Tile::k128Deep) launch_split<T, 128, 128, 3, 1>(p, plan.slices, plan.ks, stream, device);
+            else launch_split<T, 64, 64, 3, 3>(p, plan.slices, plan.ks, stream, device);
+        } else {
+            if (plan.tile == Tile::k32x128) launch_split<T, 32, 128, 4, 2>(p, plan.slices, plan.ks, stream, device);
+            else launch_split<T, 64, 64, 2, 4>(p, plan.slices, plan.ks, stream, device);
+        }
+        return;
+    }
+    if constexpr (k16) {
+        switch (plan.tile) {
+            case Tile::k128Deep: launch_config<T, 128, 128, 3, 1>(p, stream); return;
+            case Tile::k64x128: launch_config<T, 64, 128, 3, 2>(p, stream); return;
+            case Tile::k64x128Many: launch_config<T, 64, 128, 2, 3>(p, stream); return;
+            case Tile::k64: launch_config<T, 64, 64, 3, 3>(p, stream); return;
+            default: launch_config<T, 128, 128, 2, 2>(p, stream);
+        }
+    } else {
+        if (plan.tile == Tile::k64) launch_config<T, 64, 64, 2, 4>(p, stream);
+        else launch_config<T, 128, 128, 2, 2>(p, stream);
+    }
 }
 
 // Products with an operand the matrix-core kernels cannot read in place (an
@@ -1446,7 +1436,7 @@ template <typename T>
 void launch_typed(const GemmArgs& p, hipStream_t stream) {
     if (mfma_eligible<T>(p)) {
         launch_mfma<T>(p, stream);
-    } else if (p.k > 0 && tiles_fit(p) &&
+    } else if (p.k > 0 && tiles_fit(p) && panel_fits<T>(p.k + Mfma<T>::V, true) &&
                double(p.batch) * double(p.m) * double(p.n) * double(p.k) >= kRepackMinMacs) {
         launch_repacked<T>(p, stream);
     } else {
@@ -1456,13 +1446,16 @@ void launch_typed(const GemmArgs& p, hipStream_t stream) {
 
 }  // namespace
 
-bool splitk32_takes(const GemmArgs& p, int device) { return splitk32_small_batch(p, cu_count(device)) > 1; }
-
-int64_t splitk16_blocks(const GemmArgs& p, int device, int64_t* slices) {
-    const SplitPlan plan = splitk16_plan(p, cu_count(device), Mfma<bf16_t>::BK);
-    const int64_t tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
-    *slices = plan.slices;
-    return plan.slices > 1 ? tiles * plan.slices : 0;
+bool tiles_take_thin(int dtype, const GemmArgs& p, int device) {
+    const int64_t cus = cu_count(device), thin = std::min(p.m, p.n);
+    const int64_t t64 = tiles_of(p, 64, 64);
+    if (p.batch > 1) return thin > 32 && t64 >= cus;
+    if (dtype == TP_AMD_FLOAT32) return thin > 16 && plan_small_batch<float>(p, cus).slices > 1;
+    const TilePlan plan = plan_small_batch<bf16_t>(p, cus);
+    const int64_t blocks = (plan.tile == Tile::k64 ? t64 : tiles_of(p, 64, 128)) * plan.slices;
+    if (thin > 32) return blocks >= cus / 4;
+    if (thin > 16) return blocks >= cus / 2;
+    return plan.slices > 1 && 2 * blocks >= 3 * cus;
 }
 
 void launch_gemm(int dtype, const GemmArgs& p, hipStream_t stream) {
