@@ -60,12 +60,14 @@ struct Mfma<bf16_t> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, c, 0, 0, 0);
     }
     static constexpr int kPerTile = 1;  // MFMAs a 32 x 32 tile takes per fragment
-    template <int TM, int TN>
-    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[TM][TN]) {
+    // The tiles' MFMAs of substep s, on the s-th of CH accumulators each.
+    template <int TM, int TN, int CH>
+    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[CH][TM][TN],
+                                                 int s) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) c[i][j] = mma(a[i], b[j], c[i][j]);
+            for (int j = 0; j < TN; ++j) c[s % CH][i][j] = mma(a[i], b[j], c[s % CH][i][j]);
     }
 };
 
@@ -80,12 +82,13 @@ struct Mfma<f16_t> {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, c, 0, 0, 0);
     }
     static constexpr int kPerTile = 1;
-    template <int TM, int TN>
-    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[TM][TN]) {
+    template <int TM, int TN, int CH>
+    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[CH][TM][TN],
+                                                 int s) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) c[i][j] = mma(a[i], b[j], c[i][j]);
+            for (int j = 0; j < TN; ++j) c[s % CH][i][j] = mma(a[i], b[j], c[s % CH][i][j]);
     }
 };
 
@@ -94,10 +97,12 @@ struct Mfma<float> {
     static constexpr int V = 4;
     static constexpr int BK = 32;
     static constexpr int kPerTile = 4;
-    // The four k of a fragment in order for each tile, a pass over the tiles
-    // for each, so consecutive MFMAs do not wait on one accumulator.
-    template <int TM, int TN>
-    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[TM][TN]) {
+    // The four k of a fragment in order, a pass over the tiles for each, the
+    // k-th on the k-th of CH accumulators: consecutive MFMAs do not wait on
+    // one accumulator.
+    template <int TM, int TN, int CH>
+    __device__ __forceinline__ static void tiles(const uint4 (&a)[TM], const uint4 (&b)[TN], f32x16 (&c)[CH][TM][TN],
+                                                 int) {
 #pragma unroll
         for (int k = 0; k < 4; ++k)
 #pragma unroll
@@ -106,7 +111,8 @@ struct Mfma<float> {
                 for (int j = 0; j < TN; ++j) {
                     const uint32_t u = k == 0 ? a[i].x : k == 1 ? a[i].y : k == 2 ? a[i].z : a[i].w;
                     const uint32_t v = k == 0 ? b[j].x : k == 1 ? b[j].y : k == 2 ? b[j].z : b[j].w;
-                    c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(u), __uint_as_float(v), c[i][j], 0, 0, 0);
+                    f32x16& acc = c[k % CH][i][j];
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(u), __uint_as_float(v), acc, 0, 0, 0);
                 }
     }
 };
@@ -370,13 +376,20 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
         PB ob;
         oa.init(static_cast<const S*>(p.a) + bi * p.stride_a, p.lda, m0, p.m, kk, wave, lane, wm * kWaveM);
         ob.init(static_cast<const S*>(p.b) + bi * p.stride_b, p.ldb, n0, p.n, kk, wave, lane, wn * kWaveN);
-        f32x16 acc[TM][TN];
+        // A wave of one or two 32 x 32 tiles sums each in four or two
+        // interleaved accumulators, added at the end: its MFMAs do not queue
+        // on one, and the sum's rounding error is that of a chain a fourth
+        // or half as long.
+        constexpr int CH = TM * TN == 1 ? 4 : TM * TN == 2 ? 2 : 1;
+        f32x16 sums[CH][TM][TN];
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int c = 0; c < CH; ++c)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sums[c][i][j][e] = 0.0f;
 
         uint4 af[2][TM], bf[2][TN];
         auto fetch = [&](const char* stage, int s, int buf) {
@@ -385,7 +398,7 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
 #pragma unroll
             for (int j = 0; j < TN; ++j) bf[buf][j] = ob.read(stage + ATILE, j, s);
         };
-        auto mma = [&](int buf) { Mfma<T>::template tiles<TM, TN>(af[buf], bf[buf], acc); };
+        auto mma = [&](int s) { Mfma<T>::template tiles<TM, TN, CH>(af[s & 1], bf[s & 1], sums, s); };
         constexpr int kMf = TM * TN * Mfma<T>::kPerTile;
         constexpr int kReads = PA::kReads + PB::kReads;
         // The loads a wave may leave in flight when it passes the barrier of a
@@ -412,7 +425,7 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
                     if (STAGES > 2) oa.issue(kt + STAGES - 1, fill, wave);
                     ob.issue(kt + STAGES - 1, fill + ATILE, wave);
                 }
-                mma(s & 1);
+                mma(s);
                 if (s == 0) {
                     interleave<kMf, kReads, PB::kIssue + (STAGES > 2 ? PA::kIssue : 0)>();
                 } else {
@@ -423,7 +436,7 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
             meet();
             fetch(next, 0, 0);
             if (STAGES == 2) oa.issue(kt + 2, cur, wave);
-            mma(1);
+            mma(3);
             interleave<kMf, kReads, STAGES == 2 ? PA::kIssue : 0>();
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -460,6 +473,14 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
         }
         // the last steps' out-of-range loads still write LDS
         __builtin_amdgcn_s_waitcnt(0);
+        f32x16 (&acc)[TM][TN] = sums[0];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                if constexpr (CH == 2) acc[i][j] += sums[1][i][j];
+                if constexpr (CH == 4) acc[i][j] = (acc[i][j] + sums[1][i][j]) + (sums[2][i][j] + sums[3][i][j]);
+            }
 
         // Epilogue: lane holds column l32 of each 32 x 32 tile, rows
         // 8 * (e / 4) + 4 * half + e % 4 for accumulator element e.
@@ -1204,14 +1225,6 @@ TilePlan plan_small_batch(const GemmArgs& p, int64_t cus) {
     }
 }
 
-// Share of the CUs' time that tiles of this shape spend on outputs: whole
-// rounds of one tile a CU, padding included.
-double fill(const GemmArgs& p, int64_t bm, int64_t bn, int64_t cus) {
-    const int64_t tiles = tiles_of(p, bm, bn);
-    const int64_t rounds = (tiles + cus - 1) / cus;
-    return double(p.m) * double(p.n) * double(p.batch) / (double(bm * bn) * double(rounds * cus));
-}
-
 template <typename T>
 TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
     constexpr int64_t BK = Mfma<T>::BK;
@@ -1222,17 +1235,32 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
             const TilePlan plan = plan_small_batch<T>(p, cus);
             if (plan.slices > 1) return plan;
         }
-        // MFMAs of 64 cycles leave LDS and L2 idle, so 64 x 64 tiles run
-        // within 7 % of 128 x 128 ones (8192 x 4096 x 4096 2010 against 1886
-        // us) and win as soon as the larger tiles leave CUs without work:
-        // 2048 x 3000 x 1000 102 against 125 us, 3000 x 1000 x 1000 55
-        // against 68, 256 x 4096 x 1024 22 against 66 (36 split in four).
-        if (fill(p, 128, 128, cus) * 1.07 >= fill(p, 64, 64, cus)) return TilePlan{Tile::k128};
-        // Still CUs without a tile and a K worth a second launch: 256 x 1024
-        // x 4096 70 -> 26 us in four slices, 512 x 1000 x 1000 21 -> 17 in
-        // two; 256^3 7.5 us whole, 9.1 split.
-        if (t64 < cus && p.k >= 768) return split_k(Tile::k64, p, cus / t64, 192, BK);
-        return TilePlan{Tile::k64};
+        // MFMAs of 64 cycles leave LDS and L2 idle, so a CU is busy as long
+        // as it has a tile, one of 64 x 64 at 93 % of the larger ones' rate
+        // (8192 x 4096 x 4096 2010 against 1886 us), and the time is the
+        // rounds of tiles times their K: kTileUs a k of a 64 x 64 tile, by
+        // the instruction's rate.  Slices of K even out the last round for
+        // the price of the finish, a launch and a pass over the partials.
+        // 2048 x 3000 x 1000 125 us on 128 x 128 tiles, 102 on 64 x 64; 256 x
+        // 4096 x 1024 66 and 22; 700 x 900 x 5000 89 whole, 63 in three
+        // slices; 1500 x 1500 x 4000 184 and 157; 256 x 1024 x 4096 70, 26 in
+        // four; 256^3 7.5, 8.7 in two.
+        constexpr double kTileUs = 0.0137, kFinishUs = 4.0, kPartialsPerUs = 1.25e6;
+        const double rounds128 = double((t128 + cus - 1) / cus);
+        TilePlan best{Tile::k128};
+        double least = rounds128 * double(p.k) * kTileUs * 4 * 0.93;
+        for (int64_t slices = 1; slices <= (p.batch == 1 ? 16 : 1); ++slices) {
+            const TilePlan plan = slices == 1 ? TilePlan{Tile::k64} : split_k(Tile::k64, p, slices, 192, BK);
+            if (plan.slices != slices) continue;
+            const double rounds = double((t64 * slices + cus - 1) / cus);
+            double us = rounds * double(slices == 1 ? p.k : plan.ks) * kTileUs;
+            if (slices > 1) us += kFinishUs + double(p.m) * double(p.n) * double(2 * slices + 1) / kPartialsPerUs;
+            if (us < least) {
+                least = us;
+                best = plan;
+            }
+        }
+        return best;
     } else {
         if (thin <= 64) return plan_small_batch<T>(p, cus);
         // One round of 128 x 128 tiles by splitting K: when K is long, or when
@@ -1257,7 +1285,13 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
         // tile as large as still gives half the CUs one: 1777 x 1008 x 3336
         // 26.0 us on 64 x 128 against 35.1 on 128 x 128, 1024 x 1024 x 4096
         // 22.7 us on 64 x 64 against 25.5 on 64 x 128.
-        if (t128 > cus / 2) return TilePlan{Tile::k128Deep};
+        if (t128 > cus / 2) {
+            // A long K fills the CUs better in slices, two blocks a CU: 777 x
+            // 3000 x 11000 79.6 us in three against 96.8 whole, 2000 x 1280
+            // x 6000 48.3 against 53.3; with K = 3000 they are level.
+            if (p.batch == 1 && p.k >= 4096 && t128 <= cus * 4 / 5) return split_k(Tile::k128, p, 2 * cus / t128, 1024, BK);
+            return TilePlan{Tile::k128Deep};
+        }
         if (tiles_of(p, 64, 128) > cus / 2) return TilePlan{Tile::k64x128};
         if (t64 >= cus || p.k <= 2048) return TilePlan{Tile::k64};
         return split_k(Tile::k64, p, 2 * cus / t64, 1024, BK);
@@ -1283,7 +1317,8 @@ void launch_mfma(const GemmArgs& p, hipStream_t stream) {
     const TilePlan plan = plan_tiles<T>(p, cus);
     if (plan.slices > 1) {
         if constexpr (k16) {
-            if (plan.tile == Tile::k128Deep) launch_split<T, 128, 128, 3, 1>(p, plan.slices, plan.ks, stream, device);
+            if (plan.tile == Tile::k128) launch_split<T, 128, 128, 2, 2>(p, plan.slices, plan.ks, stream, device);
+            else if (plan.tile == Tile::k128Deep) launch_split<T, 128, 128, 3, 1>(p, plan.slices, plan.ks, stream, device);
             else launch_split<T, 64, 64, 3, 3>(p, plan.slices, plan.ks, stream, device);
         } else {
             if (plan.tile == Tile::k32x128) launch_split<T, 32, 128, 4, 2>(p, plan.slices, plan.ks, stream, device);

@@ -486,6 +486,79 @@ def test_gemm_fp32_split_k(amd, dev, orc, ta, tb, cin_kind):
     check(orc, outs[0], want, F32, f"split-K fp32 ta={ta} tb={tb} {cin_kind}")
 
 
+# One size for each tile shape and split the planner picks on 256 CUs, with
+# ragged edges: M and N a few elements past or short of whole tiles, K with a
+# partial last slab (16-bit slabs are 64 deep, float32 ones 32) and K shorter
+# than one.  (m, n, k); an M/N-major operand needs its extent in packets.
+TILE16 = [(2056, 2200, 72), (1496, 1512, 200), (1112, 1000, 264), (712, 136, 8), (3000, 2904, 40),
+          (200, 304, 4104), (1208, 1000, 5000), (1496, 1512, 4104), (40, 8200, 1032), (200, 328, 24)]
+TILE32 = [(2052, 2044, 36), (1500, 1504, 100), (712, 132, 4), (300, 304, 4004), (20, 8204, 2052),
+          (44, 4100, 4108), (1500, 1504, 2100), (132, 60, 28)]
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
+                         ids=["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("dtype,m,n,k", [(BF16 if i % 2 else F16, *t) for i, t in enumerate(TILE16)]
+                         + [(F32, *t) for t in TILE32], ids=lambda v: str(v))
+def test_gemm_tiles_with_ragged_edges(amd, dev, orc, dtype, ta, tb, m, n, k):
+    """Every tile shape and split in the four layouts: NaN-padded leading
+    dimensions (a load past an edge that reached the product would show),
+    alpha and a row-broadcast bias, sampled columns against float64, and the
+    same bits twice."""
+    lib = amd.load()
+    pad, alpha, beta = 8, 0.5, 2.0
+    a = _padded(orc, (k, m) if ta else (m, k), pad, dtype, 61)
+    b = _padded(orc, (n, k) if tb else (k, n), pad, dtype, 62)
+    bias = sample(orc, (n,), dtype, 63)
+    A = orc.to_float(a, dtype)[:, :(m if ta else k)]
+    B = orc.to_float(b, dtype)[:, :(k if tb else n)]
+    A = A.T if ta else A
+    B = B.T if tb else B
+    da, db, dbias = (dev.from_numpy(v, dtype=dtype) for v in (a, b, bias))
+    outs = []
+    for _ in range(2):
+        out = dev.empty((m, n), dtype=dtype)
+        st = lib.tp_amd_launch_gemm(0, dtype, 1, m, n, k, alpha, da.data_ptr, a.shape[-1], 0, int(ta),
+                                    db.data_ptr, b.shape[-1], 0, int(tb), beta, dbias.data_ptr, 0, 1, 0,
+                                    out.data_ptr, n, 0)
+        assert st == 0, lib.tp_mlu_last_error()
+        outs.append(out.numpy())
+    assert np.array_equal(outs[0], outs[1]), "two runs differ"
+    got = orc.to_float(outs[0], dtype)
+    assert not np.isnan(got).any(), "an edge leaked into the product"
+    rng = np.random.default_rng(64)
+    cols = np.unique(np.concatenate([np.arange(min(n, 8)), np.arange(max(0, n - 70), n), rng.integers(0, n, 40)]))
+    want = alpha * (A.astype(np.float64) @ B[:, cols].astype(np.float64)) + beta * orc.to_float(bias, dtype)[cols]
+    check(orc, np.ascontiguousarray(outs[0][:, cols]), want, dtype, f"{m}x{n}x{k} ta={ta} tb={tb}")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("bt,m,n,k", [(9, 1000, 64, 200), (70, 72, 136, 40), (33, 320, 80, 328), (5, 40, 48, 4104)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)], ids=["NN", "TT"])
+def test_gemm_tiles_batched(amd, dev, orc, dtype, bt, m, n, k, ta, tb):
+    """Batches of attention-sized products on the tile kernel, few columns
+    among them, each batch with its own full Cin."""
+    lib = amd.load()
+    a = _padded(orc, (bt, k, m) if ta else (bt, m, k), 8, dtype, 65)
+    b = _padded(orc, (bt, n, k) if tb else (bt, k, n), 8, dtype, 66)
+    cin = sample(orc, (bt, m, n), dtype, 67)
+    A = orc.to_float(a, dtype)[..., :(m if ta else k)].astype(np.float64)
+    B = orc.to_float(b, dtype)[..., :(k if tb else n)].astype(np.float64)
+    A = np.swapaxes(A, -1, -2) if ta else A
+    B = np.swapaxes(B, -1, -2) if tb else B
+    want = 0.5 * np.matmul(A, B) + 2.0 * orc.to_float(cin, dtype)
+    da, db, dc = (dev.from_numpy(v, dtype=dtype) for v in (a, b, cin))
+    out = dev.empty((bt, m, n), dtype=dtype)
+    st = lib.tp_amd_launch_gemm(0, dtype, bt, m, n, k, 0.5, da.data_ptr, a.shape[-1], a.shape[-1] * a.shape[-2],
+                                int(ta), db.data_ptr, b.shape[-1], b.shape[-1] * b.shape[-2], int(tb), 2.0,
+                                dc.data_ptr, n, 1, m * n, out.data_ptr, n, m * n)
+    assert st == 0, lib.tp_mlu_last_error()
+    got = out.numpy()
+    assert not np.isnan(orc.to_float(got, dtype)).any(), "an edge leaked into the product"
+    for i in (0, bt // 2, bt - 1):
+        check(orc, got[i], want[i], dtype, f"batch {i} of {bt}x{m}x{n}x{k} ta={ta} tb={tb}")
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
                          ids=["NN", "TN", "NT", "TT"])
