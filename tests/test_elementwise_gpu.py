@@ -51,6 +51,29 @@ def test_binary_with_broadcasting(dev, ops, orc, dtype, sa, sb):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols", [(5, 4), (7, 8), (3, 9), (33, 15), (20, 4095), (9, 1001), (1, 13)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_broadcast_over_ragged_rows(dev, ops, orc, dtype, rows, cols, off):
+    """A row, a column or one element against rows of any length, on either
+    side and in place: packets that cross a row's end, the last elements,
+    and a row operand that starts off a 16-byte boundary."""
+    a = sample(orc, (rows, cols), dtype, 81)
+    row = sample(orc, (cols + off,), dtype, 82, 0.5, 2.0)
+    col = sample(orc, (rows, 1), dtype, 83, 0.5, 2.0)
+    one = sample(orc, (1, 1), dtype, 84, 0.5, 2.0)
+    da = up(dev, a, dtype)
+    for b, db in ((row[off:], up(dev, row, dtype)[off:]), (col, up(dev, col, dtype)), (one, up(dev, one, dtype))):
+        assert_bitexact(ops.add(da, db).numpy(), orc.binary(ADD, dtype, a, b, 1.0), "add")
+        assert_bitexact(ops.mul(db, da).numpy(), orc.binary(MUL, dtype, b, a), "mul, operands swapped")
+        assert_bitexact(ops.div(da, db).numpy(), orc.binary(DIV, dtype, a, b), "div")
+        work = up(dev, a, dtype)
+        ops.mul_(work, db)
+        assert_bitexact(work.numpy(), orc.binary(MUL, dtype, a, b), "in place")
+    assert_bitexact(ops.mul(up(dev, col, dtype), up(dev, row, dtype)[off:]).numpy(),
+                    orc.binary(MUL, dtype, col, row[off:]), "column by row")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_scalar_forms_and_host_scalars(dev, ops, orc, dtype):
     a = sample(orc, (8, 3), dtype)
     d = up(dev, a, dtype)
