@@ -111,14 +111,35 @@ __device__ __forceinline__ void load_params(const S_<T>* p, float (&out)[VPT][Pa
     }
 }
 
-// y = (x - mean) rstd w + b over rows of D (a multiple of the packet; a row
+// Where thread `tid`'s k-th packet of a row lies.  ANY: D is at least a packet
+// but not a whole number of them (or rows start at any element); the packet
+// after the last whole one is read and written D - N in, over elements its
+// neighbour also takes: only elements from `first` on count in sums, and both
+// write the same values.
+struct RowPacket {
+    uint32_t off;  // byte offset in the row, kOutOfRange past its end
+    int first;     // first element that counts: 0, N past the row's end
+};
+template <typename T, bool ANY>
+__device__ __forceinline__ RowPacket row_packet(int q, int64_t D) {
+    constexpr int N = Packet<T>::N;
+    const int npk = static_cast<int>(D / N);
+    if (!ANY || q < npk) return {static_cast<uint32_t>(q) * 16u, q < npk ? 0 : N};
+    const int rem = static_cast<int>(D - static_cast<int64_t>(npk) * N);
+    if (q == npk && rem > 0) return {static_cast<uint32_t>((D - N) * sizeof(S_<T>)), N - rem};
+    return {kOutOfRange, N};
+}
+
+// y = (x - mean) rstd w + b over rows of D (whole packets, or ANY; a row
 // and the statistics arrays under 4 GiB).  A block holds kRows rows at a time
 // (WAVES waves each) and walks rows with stride gridDim.x kRows, two rows a
 // step in two register sets: the next row's packets are loaded before this
 // row's reductions, so the loads stay in flight across the barriers.  w and b
 // stay in registers as packets.  Rows load with the default cache policy
 // ([8192, 4096] bf16: 22.5 us, 25.9 us with non-temporal loads).
-template <typename T, int WAVES, int VPT>
+// Rows of 2047 ([8192, 2047] bf16) took 54.5 us on the scalar kernel below,
+// 14.1 us with ANY; the backward 97 us on its scalar kernels, 29.7 us.
+template <typename T, int WAVES, int VPT, bool ANY>
 __global__ __launch_bounds__(ln_threads<WAVES>()) void layer_norm_rows_kernel(
     const S_<T>* x, const S_<T>* w, const S_<T>* b, S_<T>* y, float* mean_out, float* rstd_out,
     int64_t rows, int64_t D, float eps) {
@@ -130,7 +151,9 @@ __global__ __launch_bounds__(ln_threads<WAVES>()) void layer_norm_rows_kernel(
     const int group = threadIdx.x / kThreads;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kRows;
     const uint32_t row_bytes = static_cast<uint32_t>(D * sizeof(S_<T>));
-    const int64_t npk = D / N;
+    RowPacket at[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) at[k] = row_packet<T, ANY>(tid + k * kThreads, D);
     const float inv_d = 1.0f / static_cast<float>(D);
     const Rsrc stats_m = buffer_over(mean_out, static_cast<uint32_t>(rows * sizeof(float)));
     const Rsrc stats_r = buffer_over(rstd_out, static_cast<uint32_t>(rows * sizeof(float)));
@@ -140,15 +163,14 @@ __global__ __launch_bounds__(ln_threads<WAVES>()) void layer_norm_rows_kernel(
         const Rsrc rb = buffer_over(b, b != nullptr ? row_bytes : 0);
 #pragma unroll
         for (int k = 0; k < VPT; ++k) {
-            const uint32_t off = static_cast<uint32_t>(tid + k * kThreads) * 16u;
-            wr[k] = buffer_load16_cached(rw, off);
-            br[k] = buffer_load16_cached(rb, off);
+            wr[k] = buffer_load16_cached(rw, at[k].off);
+            br[k] = buffer_load16_cached(rb, at[k].off);
         }
     }
     auto fetch = [&](uint4 (&buf)[VPT], int64_t row) {
         const Rsrc r = buffer_over(x + (row < rows ? row : 0) * D, row < rows ? row_bytes : 0);
 #pragma unroll
-        for (int k = 0; k < VPT; ++k) buf[k] = buffer_load16_cached(r, static_cast<uint32_t>(tid + k * kThreads) * 16u);
+        for (int k = 0; k < VPT; ++k) buf[k] = buffer_load16_cached(r, at[k].off);
     };
     auto process = [&](const uint4 (&buf)[VPT], int64_t row) {
         float v[VPT][N];
@@ -157,15 +179,15 @@ __global__ __launch_bounds__(ln_threads<WAVES>()) void layer_norm_rows_kernel(
         for (int k = 0; k < VPT; ++k) {
             unpack<T>(buf[k], v[k]);  // zeros past the row's end
 #pragma unroll
-            for (int j = 0; j < N; ++j) s += v[k][j];
+            for (int j = 0; j < N; ++j) s += !ANY || j >= at[k].first ? v[k][j] : 0.0f;
         }
         const float mean = row_sum<WAVES>(s, scratch) * inv_d;
         float ss = 0.0f;
 #pragma unroll
         for (int k = 0; k < VPT; ++k) {
-            const bool in = tid + k * kThreads < npk;
 #pragma unroll
             for (int j = 0; j < N; ++j) {
+                const bool in = ANY ? j >= at[k].first : at[k].first == 0;
                 const float d = in ? v[k][j] - mean : 0.0f;
                 ss += d * d;
             }
@@ -184,7 +206,7 @@ __global__ __launch_bounds__(ln_threads<WAVES>()) void layer_norm_rows_kernel(
                 const float t = (v[k][j] - mean) * rstd;
                 o[j] = fmaf(t, w != nullptr ? wv[j] : 1.0f, b != nullptr ? bv[j] : 0.0f);
             }
-            buffer_store16(ry, static_cast<uint32_t>(tid + k * kThreads) * 16u, pack<T>(o));
+            buffer_store16(ry, at[k].off, pack<T>(o));
         }
         const uint32_t stat_off = tid == 0 && active ? static_cast<uint32_t>(row) * 4u : kOutOfRange;
         buffer_store_f32(stats_m, stat_off, mean);
@@ -203,7 +225,7 @@ __global__ __launch_bounds__(ln_threads<WAVES>()) void layer_norm_rows_kernel(
     }
 }
 
-// Any D and alignment: a block per row, reading the row twice (once for the
+// Rows too short or too long for those: a block per row, reading it twice (once for the
 // statistics, once for the output; the second read hits L2).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void layer_norm_generic_kernel(
@@ -234,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void layer_norm_generic_kernel(
     }
 }
 
-// Backward over rows of D (a multiple of the packet; a row and the
+// Backward over rows of D (whole packets, or ANY; a row and the
 // statistics under 4 GiB).  A block is GROUPS row groups of WAVES waves; group
 // g of block b takes rows (b GROUPS + g) + i gridDim.x GROUPS.  Per row
 //   xhat = (x - mean) rstd,  g = dy w,
@@ -259,7 +281,7 @@ struct BwdRow {
     float mu, rs;
 };
 
-template <typename T, int WAVES, int VPT, int GROUPS>
+template <typename T, int WAVES, int VPT, int GROUPS, bool ANY>
 __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_rows_kernel(
     const S_<T>* dy, const S_<T>* x, const float* mean, const float* rstd, const S_<T>* w,
     S_<T>* dx, float* dw_part, float* db_part, int64_t rows, int64_t D) {
@@ -269,7 +291,9 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
     __shared__ float scratch[2 * GROUPS * WAVES];
     const int tid = threadIdx.x % kThreads;
     const int group = threadIdx.x / kThreads;
-    const int64_t npk = D / N;
+    RowPacket at[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) at[k] = row_packet<T, ANY>(tid + k * kThreads, D);
     const uint32_t row_bytes = static_cast<uint32_t>(D * sizeof(S_<T>));
     const Rsrc rmean = buffer_over(mean, static_cast<uint32_t>(rows * sizeof(float)));
     const Rsrc rrstd = buffer_over(rstd, static_cast<uint32_t>(rows * sizeof(float)));
@@ -277,7 +301,7 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
     {
         const Rsrc rw = buffer_over(w, w != nullptr ? row_bytes : 0);
 #pragma unroll
-        for (int k = 0; k < VPT; ++k) wr[k] = buffer_load16_cached(rw, static_cast<uint32_t>(tid + k * kThreads) * 16u);
+        for (int k = 0; k < VPT; ++k) wr[k] = buffer_load16_cached(rw, at[k].off);
     }
     float pw[VPT][N], pb[VPT][N];
 #pragma unroll
@@ -288,22 +312,21 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
     // Row `row`'s packets and statistics (zeros past the last row).
     auto fetch = [&](BwdRow<T, VPT>& buf, int64_t row) {
         const bool ok = row < rows;
-        const int64_t at = (ok ? row : 0) * D;
-        const Rsrc rx = buffer_over(x + at, ok ? row_bytes : 0);
-        const Rsrc rd = buffer_over(dy + at, ok ? row_bytes : 0);
+        const int64_t from = (ok ? row : 0) * D;
+        const Rsrc rx = buffer_over(x + from, ok ? row_bytes : 0);
+        const Rsrc rd = buffer_over(dy + from, ok ? row_bytes : 0);
         const uint32_t soff = ok ? static_cast<uint32_t>(row) * 4u : kOutOfRange;
         buf.mu = buffer_load_f32(rmean, soff);
         buf.rs = buffer_load_f32(rrstd, soff);
 #pragma unroll
         for (int k = 0; k < VPT; ++k) {
-            const uint32_t off = static_cast<uint32_t>(tid + k * kThreads) * 16u;
-            buf.x[k] = buffer_load16_cached(rx, off);
-            buf.d[k] = buffer_load16_cached(rd, off);
+            buf.x[k] = buffer_load16_cached(rx, at[k].off);
+            buf.d[k] = buffer_load16_cached(rd, at[k].off);
         }
     };
     // xhat and g of packet k (zeros past the row's end).
     auto terms = [&](const BwdRow<T, VPT>& buf, int k, float (&xh)[N], float (&g)[N], float (&dv)[N]) {
-        const bool in = tid + k * kThreads < npk;
+        const bool in = at[k].first < N;
         float xv[N], wv[N];
         unpack<T>(buf.x[k], xv);
         unpack<T>(buf.d[k], dv);
@@ -322,6 +345,7 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
             terms(buf, k, xh, g, dv);
 #pragma unroll
             for (int j = 0; j < N; ++j) {
+                if (ANY && j < at[k].first) continue;
                 a += g[j];
                 c += g[j] * xh[j];
                 pw[k][j] = fmaf(dv[j], xh[j], pw[k][j]);
@@ -339,7 +363,7 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
             terms(buf, k, xh, g, dv);
 #pragma unroll
             for (int j = 0; j < N; ++j) o[j] = buf.rs * (g[j] - a - xh[j] * c);
-            buffer_store16(rdx, static_cast<uint32_t>(tid + k * kThreads) * 16u, pack<T>(o));
+            buffer_store16(rdx, at[k].off, pack<T>(o));
         }
     };
     const int64_t first = static_cast<int64_t>(blockIdx.x) * GROUPS;
@@ -366,23 +390,25 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
             if (group == src) {
 #pragma unroll
                 for (int k = 0; k < VPT; ++k) {
-                    const int64_t q = tid + static_cast<int64_t>(k) * kThreads;
-                    if (q < npk) {
-                        // A packet's N columns lie in one chunk.
-                        float* at = out + (q * N / kFoldChunk) * gridDim.x * kFoldChunk + q * N % kFoldChunk;
+                    if (at[k].first < N) {
+                        const int64_t c0 = at[k].off / sizeof(S_<T>);
 #pragma unroll
                         for (int j = 0; j < N; ++j) {
+                            if (ANY && j < at[k].first) continue;
+                            // a whole packet's N columns lie in one chunk
+                            const int64_t c = ANY ? c0 + j : c0;
+                            float* to = out + c / kFoldChunk * gridDim.x * kFoldChunk + c % kFoldChunk + (ANY ? 0 : j);
                             float v = mine[k][j];
-                            if (src < GROUPS - 1) v += fold[q * N + j];
+                            if (src < GROUPS - 1) v += fold[c0 + j];
                             if (src > 0) {
-                                fold[q * N + j] = v;
+                                fold[c0 + j] = v;
                             } else if constexpr (sizeof(S_<T>) == 2) {
                                 // 16-bit rows: non-temporal partials, bf16
                                 // [8192, 4096] 35.9-36.2 against 36.5-36.8
                                 // us (float32 rows: no gain)
-                                __builtin_nontemporal_store(v, &at[j]);
+                                __builtin_nontemporal_store(v, to);
                             } else {
-                                at[j] = v;
+                                *to = v;
                             }
                         }
                     }
@@ -392,7 +418,8 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
     }
 }
 
-// Any D: a block per row for dx, reading x and dy twice.
+// Rows too short or too long for that: a block per row for dx, reading x and
+// dy twice.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void layer_norm_backward_generic_kernel(
     const S_<T>* dy, const S_<T>* x, const float* mean, const float* rstd, const S_<T>* w,
@@ -626,17 +653,19 @@ void layer_norm_typed(int device, int64_t rows, int64_t D, const void* xv, const
     S* y = static_cast<S*>(yv);
     hipStream_t st = stream(device);
     // The row kernels address rows and the statistics with 32-bit byte offsets.
-    const bool vec = D % N == 0 && rows < (int64_t{1} << 30) && aligned16(x) && aligned16(y) &&
-                     (w == nullptr || aligned16(w)) && (b == nullptr || aligned16(b));
-    const RowShape rs = vec ? row_shape(D / N, 4) : RowShape{};
+    const bool whole = D % N == 0 && aligned16(x) && aligned16(y) && (w == nullptr || aligned16(w)) &&
+                       (b == nullptr || aligned16(b));
+    const RowShape rs =
+        D >= N && rows < (int64_t{1} << 30) ? row_shape((D + N - 1) / N, 4) : RowShape{};
 #define TP_AMD_LN_FWD(W, V)                                                                      \
     if constexpr (W == 1 || V == 4) {                                                            \
         if (rs.waves == W && rs.vpt == V) {                                                      \
             constexpr int kRows = ln_threads<W>() / (W * kWave);                                 \
-            const int64_t blocks = resident_grid(layer_norm_rows_kernel<T, W, V>, ln_threads<W>(), \
-                                                 device, (rows + kRows - 1) / kRows);            \
-            layer_norm_rows_kernel<T, W, V><<<blocks, ln_threads<W>(), 0, st>>>(                 \
-                x, w, b, y, mean, rstd, rows, D, eps);                                           \
+            auto* kernel = whole ? layer_norm_rows_kernel<T, W, V, false>                        \
+                                 : layer_norm_rows_kernel<T, W, V, true>;                        \
+            const int64_t blocks =                                                               \
+                resident_grid(kernel, ln_threads<W>(), device, (rows + kRows - 1) / kRows);      \
+            kernel<<<blocks, ln_threads<W>(), 0, st>>>(x, w, b, y, mean, rstd, rows, D, eps);    \
             TP_AMD_HIP_CHECK(hipGetLastError());                                                 \
             return;                                                                              \
         }                                                                                        \
@@ -660,9 +689,10 @@ void layer_norm_backward_typed(int device, int64_t rows, int64_t D, const void* 
     hipStream_t st = stream(device);
     const bool params = dwv != nullptr || dbv != nullptr;
     // The row kernels address rows and the statistics with 32-bit byte offsets.
-    const bool vec = D % N == 0 && rows < (int64_t{1} << 30) && aligned16(x) && aligned16(dy) &&
-                     (dx == nullptr || aligned16(dx)) && (w == nullptr || aligned16(w));
-    const RowShape shape = vec ? backward_row_shape(D / N, N) : RowShape{};
+    const bool whole = D % N == 0 && aligned16(x) && aligned16(dy) && (dx == nullptr || aligned16(dx)) &&
+                       (w == nullptr || aligned16(w));
+    const RowShape shape =
+        D >= N && rows < (int64_t{1} << 30) ? backward_row_shape((D + N - 1) / N, N) : RowShape{};
     if (shape.waves > 0) {
         // As many blocks as the GPU holds at once walk the rows; each leaves
         // one partial row of dW and of dB.
@@ -681,7 +711,10 @@ void layer_norm_backward_typed(int device, int64_t rows, int64_t D, const void* 
         };
         constexpr int V = bwd_vpt(N);
 #define TP_AMD_LN_BWD(W)                                                                             \
-    if (shape.waves == W) launch(layer_norm_backward_rows_kernel<T, W, V, 16 / W>, 16 / W, 16 * kWave);
+    if (shape.waves == W)                                                                             \
+        launch(whole ? layer_norm_backward_rows_kernel<T, W, V, 16 / W, false>                       \
+                     : layer_norm_backward_rows_kernel<T, W, V, 16 / W, true>,                       \
+               16 / W, 16 * kWave);
         TP_AMD_LN_BWD_SHAPES(TP_AMD_LN_BWD)
 #undef TP_AMD_LN_BWD
         TP_AMD_HIP_CHECK(hipGetLastError());

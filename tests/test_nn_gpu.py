@@ -98,6 +98,38 @@ def test_layer_norm_backward(dev, ops, orc, dtype, shape, norm):
     assert_normwise(gb2.numpy().reshape(-1), ob2, dtype, scale, "dbias without weight")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("rows,D", [(7, 4), (5, 9), (40, 17), (9, 515), (300, 1001), (70, 2047), (600, 4099), (3, 8185),
+                                    (5, 16387)])
+def test_layer_norm_rows_at_any_element(dev, ops, orc, dtype, rows, D):
+    """Rows that are not whole packets, in tensors that start off a 16-byte
+    boundary (and, once, whole rows off it): the packet that ends a row
+    overlaps its neighbour, whose elements must count once.  Sums over rows
+    are compared per column against float64."""
+    def ragged(seed, scale=1.0, shift=0.0):
+        a = sample(orc, (rows * D + 1,), dtype, seed, scale, shift)
+        return a[1:].reshape(rows, D), dev.from_numpy(a, dtype=dtype)[1:].view(rows, D)
+
+    x, dx_ = ragged(61, 1.5, -0.25)
+    dy, ddy = ragged(62)
+    w, b = sample(orc, (D,), dtype, 63), sample(orc, (D,), dtype, 64)
+    w_, b_ = dev.from_numpy(w, dtype=dtype), dev.from_numpy(b, dtype=dtype)
+    y, mean, rstd = ops.native_layer_norm(dx_, (D,), w_, b_, eps=1e-5)
+    wy, wm, wr = orc.layer_norm(dtype, x, D, w, b, 1e-5)
+    assert_normwise(y.numpy(), wy, dtype, 1, "y")
+    assert_normwise(mean.numpy(), wm, F32, 1, "mean")
+    assert_normwise(rstd.numpy(), wr, F32, 1, "rstd")
+    m, r = mean.numpy(), rstd.numpy()
+    gx, gw, gb = ops.native_layer_norm_backward(ddy, dx_, (D,), mean, rstd, w_, b_)
+    ox, ow, ob = orc.layer_norm_backward(dtype, dy, x, D, m, r, w)
+    assert_normwise(gx.numpy(), ox, dtype, 1, "dx")
+    xf, dyf = (as_float(v, dtype).astype(np.float64) for v in (x, dy))
+    xhat = (xf - m.astype(np.float64)[:, None]) * r.astype(np.float64)[:, None]
+    u = 2.0 ** -24
+    assert_pointwise(gw.numpy(), ow, dtype, (rows + 5) * u * np.abs(dyf * xhat).sum(axis=0), "dweight per column")
+    assert_pointwise(gb.numpy(), ob, dtype, (rows + 2) * u * np.abs(dyf).sum(axis=0), "dbias per column")
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["fp32", "bf16"])
 def test_layer_norm_bench_shape(dev, ops, orc, dtype):
     """[8192, 4096], the shape bench.py times: every CU holds a block of the
