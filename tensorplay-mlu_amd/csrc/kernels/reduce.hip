@@ -162,7 +162,8 @@ __device__ __forceinline__ uint4 splat(uint32_t w) { return make_uint4(w, w, w, 
 // NT: non-temporal loads (the default for rows streamed once); false keeps
 // the default policy, under which a tensor the previous kernel left in the
 // 256 MB Infinity Cache is read from there.
-template <typename Tin, int OP, int THREADS, int U = 4, bool NT = true>
+// ANY: p at any element (16-byte loads that need not be aligned).
+template <typename Tin, int OP, int THREADS, int U, bool NT, bool ANY>
 __device__ __forceinline__ float row_exact(const typename Elem<Tin>::storage* p, int64_t pb,
                                            int64_t pe, int tid) {
     constexpr int N = Packet<Tin>::N;
@@ -177,7 +178,7 @@ __device__ __forceinline__ float row_exact(const typename Elem<Tin>::storage* p,
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int64_t q = q0 + static_cast<int64_t>(u) * THREADS;
-            raw[u] = q < pe ? (NT ? load_raw_nt(p + q * N) : *reinterpret_cast<const uint4*>(p + q * N))
+            raw[u] = q < pe ? (NT ? load_raw_stream<ANY>(p + q * N) : load_raw<ANY>(p + q * N))
                             : splat(kPad);
         }
 #pragma unroll
@@ -194,7 +195,7 @@ __device__ __forceinline__ float row_exact(const typename Elem<Tin>::storage* p,
 // The same share for amax / amin on integer keys (NaN when a NaN wins or the
 // share is empty).  The padding is the NaN pattern whose key loses to every
 // value.
-template <typename Tin, int OP, int THREADS, int U = 4, bool NT = true>
+template <typename Tin, int OP, int THREADS, int U, bool NT, bool ANY>
 __device__ __forceinline__ float row_keys(const typename Elem<Tin>::storage* p, int64_t pb,
                                           int64_t pe, int tid) {
     constexpr int N = Packet<Tin>::N;
@@ -208,7 +209,7 @@ __device__ __forceinline__ float row_keys(const typename Elem<Tin>::storage* p, 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int64_t q = q0 + static_cast<int64_t>(u) * THREADS;
-            raw[u] = q < pe ? (NT ? load_raw_nt(p + q * N) : *reinterpret_cast<const uint4*>(p + q * N))
+            raw[u] = q < pe ? (NT ? load_raw_stream<ANY>(p + q * N) : load_raw<ANY>(p + q * N))
                             : splat(kPad);
         }
 #pragma unroll
@@ -225,14 +226,44 @@ __device__ __forceinline__ float row_keys(const typename Elem<Tin>::storage* p, 
     else return K::template value16<Tin>(k16);
 }
 
+// One thread's share of elements [begin, end) of a row at p (begin a
+// multiple of the packet): whole packets, then with ANY the last (end %
+// packet) elements one to a thread.
+template <typename Tin, int OP, int THREADS, int U, bool NT, bool ANY>
+__device__ __forceinline__ float row_share(const typename Elem<Tin>::storage* p, int64_t begin, int64_t end,
+                                           int tid) {
+    constexpr int N = Packet<Tin>::N;
+    const int64_t pb = begin / N, pe = end / N;
+    float acc;
+    if constexpr (kMinMax<OP>) {
+        acc = row_keys<Tin, OP, THREADS, U, NT, ANY>(p, pb, pe, tid);
+        if (acc != acc) acc = row_exact<Tin, OP, THREADS, U, NT, ANY>(p, pb, pe, tid);
+    } else {
+        acc = row_exact<Tin, OP, THREADS, U, NT, ANY>(p, pb, pe, tid);
+    }
+    if (ANY && pe * N + tid < end) {
+        const float v = Elem<Tin>::load(p[pe * N + tid]);
+        if constexpr (kMinMax<OP>) {
+            using K = KeyOps<OP>;
+            if (acc != acc) acc = v;
+            else if (v == v) acc = K::value32(K::pick(key32(__float_as_uint(acc)), key32(__float_as_uint(v))));
+        } else {
+            acc = Combine<OP>::apply(acc, v);
+        }
+    }
+    return acc;
+}
+
 // Row segments.  Segment s covers row s / nseg, elements
 // [(s % nseg) * chunk, min(r, ... + chunk)).  WAVES wavefronts share one
-// segment (1: each wave of the block takes its own segment).
-template <typename Tin, typename Tout, int OP, int WAVES, bool VEC>
+// segment (1: each wave of the block takes its own segment).  ANY: rows that
+// start at any element (r not a whole number of packets); the scalar loop
+// they took ran [8191, 4095] bfloat16 in 23-28 us, 11-12 us so (whole tensor 38-51
+// -> 13).
+template <typename Tin, typename Tout, int OP, int WAVES, bool ANY>
 __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(
     const typename Elem<Tin>::storage* x, typename Elem<Tout>::storage* out, int64_t nsegs,
     int64_t r, int64_t chunk, int64_t nseg, bool final_pass, int64_t count) {
-    constexpr int N = VEC ? Packet<Tin>::N : 1;
     constexpr int kSegsPerBlock = (kBlock / kWave) / WAVES;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int64_t seg = static_cast<int64_t>(blockIdx.x) * kSegsPerBlock + wave / WAVES;
@@ -243,21 +274,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(
         const int64_t row = seg / nseg, part = seg - row * nseg;
         const int64_t begin = part * chunk;
         const int64_t end = begin + chunk < r ? begin + chunk : r;
-        const typename Elem<Tin>::storage* p = x + row * r;
-        if constexpr (VEC) {
-            // begin and end are multiples of N (chunk and r are).
-            const int64_t pb = begin / N, pe = end / N;
-            if constexpr (kMinMax<OP>) {
-                acc = row_keys<Tin, OP, kThreads>(p, pb, pe, tid);
-                if (acc != acc) acc = row_exact<Tin, OP, kThreads>(p, pb, pe, tid);
-            } else {
-                acc = row_exact<Tin, OP, kThreads>(p, pb, pe, tid);
-            }
-        } else {
-            for (int64_t j = begin + tid; j < end; j += kThreads) {
-                acc = Combine<OP>::apply(acc, Elem<Tin>::load(p[j]));
-            }
-        }
+        acc = row_share<Tin, OP, kThreads, 4, true, ANY>(x + row * r, begin, end, tid);
     }
     acc = lane_reduce<OP>(acc);
     if constexpr (WAVES > 1) {
@@ -344,37 +361,22 @@ constexpr int fused_threads() {
 }
 constexpr int64_t segments_per_cu(int64_t packet) { return packet == 4 ? 2 : 1; }
 
-template <typename Tin, int OP, bool VEC, int BLOCK = fused_threads<Tin>()>
+template <typename Tin, int OP, bool ANY, int BLOCK = fused_threads<Tin>()>
 __global__ __launch_bounds__(BLOCK) void reduce_rows_fused_kernel(
     const typename Elem<Tin>::storage* x, typename Elem<Tin>::storage* out, float* partial,
     int64_t r, int64_t chunk, int64_t nseg, int64_t ngroups) {
-    constexpr int N = VEC ? Packet<Tin>::N : 1;
     const int64_t seg = blockIdx.x;
     const int64_t row = seg / nseg, part = seg - row * nseg;
     const int64_t begin = part * chunk;
     const int64_t end = begin + chunk < r ? begin + chunk : r;
-    const typename Elem<Tin>::storage* p = x + row * r;
     const int tid = threadIdx.x;
-    float acc = Combine<OP>::identity();
-    if constexpr (VEC) {
-        // 16-bit tensors load with the default policy, float32 ones
-        // non-temporally.  Measured on whole 4096^2 tensors called back to
-        // back: bf16 sum 5.86 us against 8.32 us non-temporal (the 32 MiB
-        // are served from the Infinity Cache), float32 11.0 us against
-        // 12.6 us with the default policy.
-        constexpr bool kNt = sizeof(typename Elem<Tin>::storage) == 4;
-        const int64_t pb = begin / N, pe = end / N;
-        if constexpr (kMinMax<OP>) {
-            acc = row_keys<Tin, OP, BLOCK, 8, kNt>(p, pb, pe, tid);
-            if (acc != acc) acc = row_exact<Tin, OP, BLOCK, 8, kNt>(p, pb, pe, tid);
-        } else {
-            acc = row_exact<Tin, OP, BLOCK, 8, kNt>(p, pb, pe, tid);
-        }
-    } else {
-        for (int64_t j = begin + tid; j < end; j += BLOCK) {
-            acc = Combine<OP>::apply(acc, Elem<Tin>::load(p[j]));
-        }
-    }
+    // 16-bit tensors load with the default policy, float32 ones
+    // non-temporally.  Measured on whole 4096^2 tensors called back to
+    // back: bf16 sum 5.86 us against 8.32 us non-temporal (the 32 MiB
+    // are served from the Infinity Cache), float32 11.0 us against
+    // 12.6 us with the default policy.
+    constexpr bool kNt = sizeof(typename Elem<Tin>::storage) == 4;
+    float acc = row_share<Tin, OP, BLOCK, 8, kNt, ANY>(x + row * r, begin, end, tid);
     acc = block_reduce<OP, BLOCK>(acc);
     // The block's group of segments, and that group's slot among the row's.
     const int64_t group = part / kFoldGroup;
@@ -419,7 +421,7 @@ __global__ __launch_bounds__(BLOCK) void reduce_rows_fused_kernel(
 
 // amax / amin of one thread's N columns over rows row0, row0 + G, ... < end
 // on integer keys (a column comes out NaN when a NaN wins or it has no rows).
-template <typename Tin, int OP, int G, bool NT>
+template <typename Tin, int OP, int G, bool NT, bool ANY>
 __device__ __forceinline__ void cols_keys(float (&acc)[Packet<Tin>::N],
                                           const typename Elem<Tin>::storage* p, int64_t row0,
                                           int64_t end, int64_t inner) {
@@ -447,12 +449,12 @@ __device__ __forceinline__ void cols_keys(float (&acc)[Packet<Tin>::N],
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const auto* q = p + (row + u * G) * inner;
-            raw[u] = NT ? load_raw_nt(q) : *reinterpret_cast<const uint4*>(q);
+            raw[u] = NT ? load_raw_stream<ANY>(q) : load_raw<ANY>(q);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) take(raw[u]);
     }
-    for (; row < end; row += G) take(*reinterpret_cast<const uint4*>(p + row * inner));
+    for (; row < end; row += G) take(load_raw<ANY>(p + row * inner));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if constexpr (kWide) {
@@ -472,6 +474,12 @@ __device__ __forceinline__ void cols_keys(float (&acc)[Packet<Tin>::N],
 // the block writes the result; otherwise it writes float32 partials
 // out[(o * nchunk + ch) * inner + col].
 //
+// ANY: rows that start at any element (inner at least a packet but not a
+// whole number of them, or x off a 16-byte boundary).  The last packet of a
+// row then starts inner - N in, over columns its neighbour also takes: both
+// compute the same value in the same order and store it.  VEC false: single
+// elements, for rows shorter than a packet.
+//
 // FUSE folds the second pass in: the partials are written and read back
 // with agent-coherent accesses; every block counts its arrival in
 // col_counters (one 128-byte line per column range o * gridDim.x +
@@ -480,23 +488,23 @@ __device__ __forceinline__ void cols_keys(float (&acc)[Packet<Tin>::N],
 // nchunk partials back in chunk order, writes the result, and resets the
 // counter to zero for the next launch.  The counters start at zero (device
 // globals are zeroed when the code object loads).
-template <typename Tin, bool VEC>
-constexpr int col_lanes() {
+constexpr int col_lanes(int64_t packet) {
     // Measured on X1 and X2 of config 3: 16-bit packets run best as 16 lanes
     // (128 columns) per row, float32 packets and single elements as 64.
-    return VEC && sizeof(typename Elem<Tin>::storage) == 2 ? 16 : 64;
+    // Ragged 16-bit rows too: [8191, 4095] mean and amin over dim 0 31.5 and
+    // 62 us by single elements, 22.8 and 24.0 so, 23.8 and 26.0 on 64 lanes.
+    return packet == 8 ? 16 : 64;
 }
 
 constexpr int64_t kMaxColCounters = 8192;
 __device__ unsigned int col_counters[kMaxColCounters * kCounterStride];
 
-template <typename Tin, typename Tout, int OP, bool VEC, bool FUSE>
+template <typename Tin, typename Tout, int OP, int LANES, bool VEC, bool FUSE, bool ANY>
 __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
     const typename Elem<Tin>::storage* x, typename Elem<Tout>::storage* out,
     typename Elem<Tin>::storage* result, int64_t outer, int64_t r, int64_t inner, int64_t chunk,
     int64_t nchunk, bool final_pass, int64_t count) {
     constexpr int N = VEC ? Packet<Tin>::N : 1;
-    constexpr int LANES = col_lanes<Tin, VEC>();
     // Non-temporal loads measured faster with 64 lanes a row, plain ones
     // with 16.
     constexpr bool NT = LANES == 64;
@@ -505,7 +513,9 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
     __shared__ float partial[G][COLS + 1];
     __shared__ bool last;
     const int lane = threadIdx.x % LANES, rg = threadIdx.x / LANES;
-    const int64_t col = (static_cast<int64_t>(blockIdx.x) * LANES + lane) * N;
+    // a packet's first column (VEC: inner if it has none)
+    auto first_col = [&](int64_t c) { return ANY && c < inner && c > inner - N ? inner - N : c; };
+    const int64_t col = first_col((static_cast<int64_t>(blockIdx.x) * LANES + lane) * N);
     const int64_t ch = blockIdx.y;
     const int64_t begin = ch * chunk;
     const int64_t end = begin + chunk < r ? begin + chunk : r;
@@ -516,7 +526,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
         bool exact = !(kMinMax<OP> && VEC);
         if constexpr (kMinMax<OP> && VEC) {
             if (col < inner) {
-                cols_keys<Tin, OP, G, NT>(acc, x + o * r * inner + col, begin + rg, end, inner);
+                cols_keys<Tin, OP, G, NT, ANY>(acc, x + o * r * inner + col, begin + rg, end, inner);
 #pragma unroll
                 for (int j = 0; j < N; ++j) exact = exact || acc[j] != acc[j];
                 if (exact) {
@@ -531,17 +541,19 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
             constexpr int U = 8;
             for (; row + (U - 1) * G < end; row += U * G) {
                 if constexpr (VEC) {
-                    Packet<Tin> v[U];
+                    uint4 raw[U];
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         const auto* q = p + (row + u * G) * inner;
-                        v[u] = NT ? load_packet_nt<Tin>(q) : load_packet<Tin>(q);
+                        raw[u] = NT ? load_raw_stream<ANY>(q) : load_raw<ANY>(q);
                     }
 #pragma unroll
-                    for (int u = 0; u < U; ++u)
+                    for (int u = 0; u < U; ++u) {
+                        float v[N];
+                        unpack<Tin>(raw[u], v);
 #pragma unroll
-                        for (int j = 0; j < N; ++j)
-                            acc[j] = Combine<OP>::apply(acc[j], Elem<Tin>::load(v[u].v[j]));
+                        for (int j = 0; j < N; ++j) acc[j] = Combine<OP>::apply(acc[j], v[j]);
+                    }
                 } else {
                     typename Elem<Tin>::storage v[U];
 #pragma unroll
@@ -553,10 +565,10 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
             }
             for (; row < end; row += G) {
                 if constexpr (VEC) {
-                    const Packet<Tin> v = load_packet<Tin>(p + row * inner);
+                    float v[N];
+                    unpack<Tin>(load_raw<ANY>(p + row * inner), v);
 #pragma unroll
-                    for (int j = 0; j < N; ++j)
-                        acc[j] = Combine<OP>::apply(acc[j], Elem<Tin>::load(v.v[j]));
+                    for (int j = 0; j < N; ++j) acc[j] = Combine<OP>::apply(acc[j], v[j]);
                 } else {
                     acc[0] = Combine<OP>::apply(acc[0], Elem<Tin>::load(p[row * inner]));
                 }
@@ -570,7 +582,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
             float v = partial[0][e];
 #pragma unroll
             for (int g = 1; g < G; ++g) v = Combine<OP>::apply(v, partial[g][e]);
-            const int64_t c = static_cast<int64_t>(blockIdx.x) * COLS + e;
+            const int64_t c = first_col(static_cast<int64_t>(blockIdx.x) * COLS + e / N * N) + e % N;
             if (c < inner) {
                 auto* dst = out + (o * nchunk + ch) * inner + c;
                 const auto val = Elem<Tout>::store(finish<OP>(v, count, final_pass));
@@ -597,7 +609,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(
             __syncthreads();
             if (last) {
                 for (int e = threadIdx.x; e < COLS; e += kBlock) {
-                    const int64_t c = static_cast<int64_t>(blockIdx.x) * COLS + e;
+                    const int64_t c = first_col(static_cast<int64_t>(blockIdx.x) * COLS + e / N * N) + e % N;
                     if (c < inner) {
                         float* q = out + o * nchunk * inner + c;
                         auto at = [&](int64_t k) {
@@ -670,7 +682,7 @@ struct SplitPlan {
     int64_t partial_floats = 0;
 };
 
-SplitPlan plan_split(int64_t outer, int64_t r, int64_t inner, int64_t cus, int64_t packet, bool vec,
+SplitPlan plan_split(int64_t outer, int64_t r, int64_t inner, int64_t cus, int64_t packet,
                      int64_t cols_per_block) {
     SplitPlan sp;
     if (inner == 1) {
@@ -680,7 +692,7 @@ SplitPlan plan_split(int64_t outer, int64_t r, int64_t inner, int64_t cus, int64
             const int64_t max_seg = r / 4096;  // >= 2 here
             if (nseg > max_seg) nseg = max_seg;
             int64_t chunk = (r + nseg - 1) / nseg;
-            if (vec) chunk = (chunk + packet - 1) / packet * packet;
+            chunk = (chunk + packet - 1) / packet * packet;
             nseg = (r + chunk - 1) / chunk;
             if (nseg > 1) {
                 sp.nseg = nseg;
@@ -724,20 +736,16 @@ void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const voi
     const int64_t cus = cu_count(device);
     constexpr int N = Packet<T>::N;
     if (inner == 1) {
-        const bool vec = r % N == 0 && aligned16(x);
-        const SplitPlan sp = plan_split(outer, r, 1, cus, N, vec, 0);
+        const bool aligned = r % N == 0 && aligned16(x);
+        const SplitPlan sp = plan_split(outer, r, 1, cus, N, 0);
         if (sp.nseg > 1) {
             TP_AMD_CHECK(outer <= kMaxFoldRows && outer * sp.ngroups <= kMaxFoldGroups,
                          "row reduction: ", outer, " rows of ", sp.nseg, " segments exceed the arrival counters");
             const int64_t nsegs = outer * sp.nseg;
             Partials partial(scratch, sp.partial_floats, device);
-            if (vec) {
-                reduce_rows_fused_kernel<T, OP, true><<<static_cast<unsigned>(nsegs), fused_threads<T>(), 0, st>>>(
-                    x, out, partial.get(), r, sp.chunk, sp.nseg, sp.ngroups);
-            } else {
-                reduce_rows_fused_kernel<T, OP, false><<<static_cast<unsigned>(nsegs), fused_threads<T>(), 0, st>>>(
-                    x, out, partial.get(), r, sp.chunk, sp.nseg, sp.ngroups);
-            }
+            auto* kernel = aligned ? reduce_rows_fused_kernel<T, OP, false> : reduce_rows_fused_kernel<T, OP, true>;
+            kernel<<<static_cast<unsigned>(nsegs), fused_threads<T>(), 0, st>>>(x, out, partial.get(), r, sp.chunk,
+                                                                                sp.nseg, sp.ngroups);
             TP_AMD_HIP_CHECK(hipGetLastError());
             return;
         }
@@ -747,39 +755,33 @@ void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const voi
         // against 45-49 us).
         const bool key16 = kMinMax<OP> && sizeof(S) == 2;
         const bool long_rows = key16 ? r * 2 >= 16384 : r >= 4096;
-        auto launch_rows = [&](auto waves_tag, auto vec_tag) {
+        auto launch_rows = [&](auto waves_tag) {
             constexpr int W = decltype(waves_tag)::value;
-            constexpr bool V = decltype(vec_tag)::value;
             constexpr int per_block = (kBlock / kWave) / W;
             const int64_t blocks = (outer + per_block - 1) / per_block;
-            reduce_rows_kernel<T, T, OP, W, V><<<blocks, kBlock, 0, st>>>(x, out, outer, r, r, 1, true, r);
+            auto* kernel = aligned ? reduce_rows_kernel<T, T, OP, W, false> : reduce_rows_kernel<T, T, OP, W, true>;
+            kernel<<<blocks, kBlock, 0, st>>>(x, out, outer, r, r, 1, true, r);
         };
-        using One = std::integral_constant<int, 1>;
-        using Four = std::integral_constant<int, 4>;
-        using Yes = std::true_type;
-        using No = std::false_type;
         if (long_rows) {
-            vec ? launch_rows(Four{}, Yes{}) : launch_rows(Four{}, No{});
+            launch_rows(std::integral_constant<int, 4>{});
         } else {
-            vec ? launch_rows(One{}, Yes{}) : launch_rows(One{}, No{});
+            launch_rows(std::integral_constant<int, 1>{});
         }
         TP_AMD_HIP_CHECK(hipGetLastError());
         return;
     }
     // Column reductions.
-    const bool vec = inner % N == 0 && aligned16(x);
-    const int64_t cols_per_block = vec ? col_lanes<T, true>() * N : col_lanes<T, false>();
-    const SplitPlan sp = plan_split(outer, r, inner, cus, N, vec, cols_per_block);
+    const bool vec = inner >= N, aligned = inner % N == 0 && aligned16(x);
+    constexpr int L = col_lanes(N);
+    const int64_t cols_per_block = vec ? L * N : 64;
+    const SplitPlan sp = plan_split(outer, r, inner, cus, N, cols_per_block);
     const int64_t bx = sp.bx, nchunk = sp.nchunk, chunk = sp.chunk;
     const dim3 grid(static_cast<unsigned>(bx), static_cast<unsigned>(nchunk), static_cast<unsigned>(sp.z));
     if (nchunk == 1) {
-        if (vec) {
-            reduce_cols_kernel<T, T, OP, true, false>
-                <<<grid, kBlock, 0, st>>>(x, out, nullptr, outer, r, inner, chunk, 1, true, r);
-        } else {
-            reduce_cols_kernel<T, T, OP, false, false>
-                <<<grid, kBlock, 0, st>>>(x, out, nullptr, outer, r, inner, chunk, 1, true, r);
-        }
+        auto* kernel = !vec      ? reduce_cols_kernel<T, T, OP, 64, false, false, false>
+                       : aligned ? reduce_cols_kernel<T, T, OP, L, true, false, false>
+                                         : reduce_cols_kernel<T, T, OP, L, true, false, true>;
+        kernel<<<grid, kBlock, 0, st>>>(x, out, nullptr, outer, r, inner, chunk, 1, true, r);
         TP_AMD_HIP_CHECK(hipGetLastError());
         return;
     }
@@ -790,13 +792,10 @@ void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const voi
     Partials partials(scratch, sp.partial_floats, device);
     float* partial = partials.get();
     // One launch: the last block of each column range folds the partials.
-    if (vec) {
-        reduce_cols_kernel<T, float, OP, true, true>
-            <<<grid, kBlock, 0, st>>>(x, partial, out, outer, r, inner, chunk, nchunk, false, r);
-    } else {
-        reduce_cols_kernel<T, float, OP, false, true>
-            <<<grid, kBlock, 0, st>>>(x, partial, out, outer, r, inner, chunk, nchunk, false, r);
-    }
+    auto* kernel = !vec      ? reduce_cols_kernel<T, float, OP, 64, false, true, false>
+                   : aligned ? reduce_cols_kernel<T, float, OP, L, true, true, false>
+                                : reduce_cols_kernel<T, float, OP, L, true, true, true>;
+    kernel<<<grid, kBlock, 0, st>>>(x, partial, out, outer, r, inner, chunk, nchunk, false, r);
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -894,10 +893,8 @@ int64_t tp_amd_reduce_partial_bytes(int compute_units, int dtype, int64_t outer,
     if (compute_units <= 0 || outer < 0 || r < 0 || inner < 0) return -1;
     if (outer == 0 || inner == 0 || r == 0) return 0;
     const int64_t packet = 16 / esize;
-    const bool vec = (inner == 1 ? r : inner) % packet == 0;
-    // col_lanes: 16 lanes of 16-bit packets, 64 lanes of float32 packets or single elements
-    const int64_t cols_per_block = vec ? (esize == 2 ? 16 : 64) * packet : 64;
-    return plan_split(outer, r, inner, compute_units, packet, vec, cols_per_block).partial_floats *
+    const int64_t cols_per_block = inner >= packet ? col_lanes(packet) * packet : 64;
+    return plan_split(outer, r, inner, compute_units, packet, cols_per_block).partial_floats *
            static_cast<int64_t>(sizeof(float));
 }
 

@@ -139,6 +139,43 @@ def test_few_long_rows_folded_in_one_launch(dev, ops, orc, dtype, shape):
             assert_bitexact(got, want, f"op {op} {shape} run {rep}")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("shape,dims", [((70, 3), [1]), ((70, 9), [1]), ((33, 515), [1]), ((9, 4099), [1]),
+                                        ((3, 8193), [1]), ((2, 70003), [1]), ((19, 4097), None),
+                                        ((300, 9), [0]), ((77, 17), [0]), ((2000, 129), [0]), ((400, 4095), [0]),
+                                        ((3, 700, 263), [1]), ((600, 5), [0])],
+                         ids=lambda v: str(v).replace(" ", ""))
+def test_reductions_of_ragged_rows(dev, ops, orc, dtype, shape, dims):
+    """Rows that are not a whole number of packets, in a tensor that starts
+    off a 16-byte boundary: packets at any element, the last elements of a
+    row one to a thread, the last packet of a column reduction over columns
+    its neighbour also takes.  NaNs, zeros of both signs and extrema in the
+    first and last elements of rows and columns."""
+    n = int(np.prod(shape))
+    a = sample(orc, (n + 1,), dtype, 71, mean=0.5)
+    a[1:][[0, shape[-1] - 1, n - 1, n // 2]] = orc.from_float(np.array([9, 8, -9, np.nan], np.float32), dtype)
+    d = dev.from_numpy(a, dtype=dtype)[1:].view(*shape)
+    a = a[1:].reshape(shape)
+    for op, fn in ((AMAX, ops.amax), (AMIN, ops.amin)):
+        want = oracle_reduce(orc, op, dtype, a, dims)
+        for rep in range(2):
+            assert_bitexact(fn(d, [] if dims is None else dims).numpy(), want, f"op {op} run {rep}")
+    zeros = orc.from_float(np.where(np.arange(n) % 3, 0.0, -0.0).astype(np.float32).reshape(shape), dtype)
+    z = dev.from_numpy(zeros, dtype=dtype)
+    for op, fn in ((AMAX, ops.amax), (AMIN, ops.amin)):
+        assert_bitexact(fn(z, [] if dims is None else dims).numpy(), oracle_reduce(orc, op, dtype, zeros, dims),
+                        f"signed zeros, op {op}")
+    for op in (SUM, MEAN):
+        want = oracle_reduce(orc, op, dtype, a, dims)
+        ok = ~np.isnan(as_float(want, dtype))
+        whole, part = (ops.sum, ops.sum_dim) if op == SUM else (ops.mean, ops.mean_dim)
+        for rep in range(2):
+            got = (whole(d) if dims is None else part(d, dims)).numpy()
+            assert np.array_equal(np.isnan(as_float(got, dtype)), ~ok)
+            if ok.any():
+                check_sum(got[ok], want[ok], dtype, f"op {op} run {rep}", a, dims, op == MEAN, mask=ok)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_long_reductions(dev, ops, orc, dtype):
     # float16 sums of 131072 elements stay below its largest finite value
