@@ -191,7 +191,16 @@ __device__ __forceinline__ void interleave() {
 //     put the halves on opposite 32 banks.  Rows at or past K read zeros;
 //     columns past R's edge read the next row's elements and only reach
 //     outputs that are not stored.
-template <typename T, bool KMAJOR, int R, int W, int NT>
+// Operands are read where they lie, at any element: the loads need no
+// alignment, but the resource's bound drops each of a load's four dwords that
+// is not wholly inside it.  Without ODD, operands are whole dwords and whole
+// packets of K, and that bound is exact.  With ODD the resource starts at the
+// dword of the first element and ends at that of the last (an aligned dword
+// never leaves the last element's page), and `finish_last` mends the last K
+// tile in LDS: it zeroes what a packet or dword across K let in, and puts in
+// the last element where that is the low half of a load's dword and so was
+// dropped.
+template <typename T, bool KMAJOR, int R, int W, int NT, bool ODD>
 struct Panel {
     using S = typename Elem<T>::storage;
     static constexpr int E = sizeof(S), V = 16 / E, BK = Mfma<T>::BK;
@@ -210,6 +219,7 @@ struct Panel {
     const char* base;
     int64_t ld_bytes, bytes;  // bytes: readable from base (M/N-major: from k = 0)
     uint32_t voff, kleft;     // kleft: K-major, elements of K from this lane's chunk of K tile 0 on
+    bool past_k, lost;        // the last K tile holds elements past K, lacks the last element
     uint32_t frag[kFrags];
 
     static __device__ __forceinline__ int slot_of(int c, int k) {
@@ -226,8 +236,9 @@ struct Panel {
         if constexpr (KMAJOR) {
             const int64_t mine = rows - r0 < R ? rows - r0 : R;
             base = reinterpret_cast<const char*>(X) + r0 * ld_bytes;
-            // whole packets: an odd K comes with rows zero-padded to one
-            bytes = (mine - 1) * ld_bytes + (K + V - 1) / V * 16;
+            bytes = (mine - 1) * ld_bytes + K * E;
+            past_k = ODD && K % V != 0;
+            lost = ODD && E == 2 && K % 2 != 0;
             const int row = lane >> 3, chunk = (lane & 7) ^ kswz(8 * wave + row);
             voff = static_cast<uint32_t>((8 * wave + row) * ld_bytes + chunk * 16);
             kleft = static_cast<uint32_t>(K > chunk * V ? K - chunk * V : 0);
@@ -237,6 +248,8 @@ struct Panel {
             constexpr int kSlots = kRowBytes / 16;
             base = reinterpret_cast<const char*>(X + r0);
             bytes = (K - 1) * ld_bytes + (rows - r0) * E;
+            past_k = ODD && E == 2 && K % BK != 0 && ((reinterpret_cast<uintptr_t>(base) + bytes) & 2) != 0;
+            lost = ODD && E == 2 && (rows - r0) % 2 != 0 && rows - r0 <= R;
             const int k = wave * kPerLoad + lane / kSlots;
             voff = static_cast<uint32_t>(k * ld_bytes + slot_of(lane % kSlots, k) * 16);
             kleft = 0;
@@ -256,6 +269,34 @@ struct Panel {
                     const int col = wbase + t * 32 + l32;
                     frag[t] = 4 * half * kRowBytes + (slot_of(col / 4, 4 * half) << 4) + (col % 4) * 4;
                 }
+            }
+        }
+        if constexpr (!ODD) return;
+        // an odd count that ends on a dword began in the middle of one
+        lost = lost && ((reinterpret_cast<uintptr_t>(base) + bytes) & 2) == 0;
+        const uint32_t lead = reinterpret_cast<uintptr_t>(base) & 3;
+        base -= lead;
+        voff += lead;
+        bytes = (bytes + lead + 3) / 4 * 4;
+    }
+
+    // Mends the last K tile; `left` = K's elements in it (1 .. BK), `extent`
+    // = the panel's rows.
+    __device__ __forceinline__ void finish_last(char* tile, int left, int64_t extent) const {
+        const int r = threadIdx.x;
+        if constexpr (KMAJOR) {
+            if (past_k && r < R) {
+                S* chunk = reinterpret_cast<S*>(tile + r * 128 + (((left / V) ^ kswz(r)) << 4));
+                for (int e = left % V; e < V; ++e) chunk[e] = S{};
+                if (lost && r == extent - 1) {
+                    chunk[left % V - 1] = *reinterpret_cast<const S*>(base + bytes - E);
+                }
+            }
+        } else {
+            if (past_k && r < R) reinterpret_cast<S*>(tile + left * kRowBytes)[r] = S{};
+            if (lost && r == extent - 1) {
+                S* chunk = reinterpret_cast<S*>(tile + (left - 1) * kRowBytes + (slot_of(r / V, left - 1) << 4));
+                chunk[r % V] = *reinterpret_cast<const S*>(base + bytes - E);
             }
         }
     }
@@ -329,15 +370,17 @@ struct Panel {
 // tiles through registers and LDS stores, and its waves met at the end of
 // each step with the matrix pipe idle (float32 4096^3 85 % busy).
 // BLOCKS is how many blocks a CU holds (LDS and registers).
-template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT>
+// ODD (see Panel) is a variant of its own: its test for the last K tile in
+// the loop costs the others 3-8 % (float32 256 x 1024 x 4096 25.3 -> 27.4 us).
+template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
 __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p) {
     using S = typename Elem<T>::storage;
     constexpr int WM = BM >= 64 ? 2 : 1, WN = 4 / WM, W = WM * WN;
     constexpr int BK = Mfma<T>::BK;
     constexpr int kWaveM = BM / WM, kWaveN = BN / WN;
     constexpr int TM = kWaveM / 32, TN = kWaveN / 32;
-    using PA = Panel<T, A_KMAJOR, BM, W, TM>;
-    using PB = Panel<T, B_KMAJOR, BN, W, TN>;
+    using PA = Panel<T, A_KMAJOR, BM, W, TM, ODD>;
+    using PB = Panel<T, B_KMAJOR, BN, W, TN, ODD>;
     constexpr int ATILE = BM * 128, STAGE = (BM + BN) * 128;
     // An object a stage, so the compiler can tell the ones being filled from
     // the one being read and leaves the loads in flight.
@@ -413,6 +456,17 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         };
+        const bool mend = ODD && (oa.past_k || oa.lost || ob.past_k || ob.lost);
+        auto finish = [&](char* last) {
+            if constexpr (!ODD) return;
+            const int left = static_cast<int>(kk - static_cast<int64_t>(nk - 1) * BK);
+            oa.finish_last(last, left, p.m - m0 < BM ? p.m - m0 : BM);
+            ob.finish_last(last + ATILE, left, p.n - n0 < BN ? p.n - n0 : BN);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the stores are in LDS
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
         auto body = [&](auto at, int kt) {
             constexpr int I = decltype(at)::value;
             char* cur = stage_at(std::integral_constant<int, I>{});
@@ -434,6 +488,7 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
                 __builtin_amdgcn_sched_barrier(0);
             }
             meet();
+            if (mend && kt + 2 == nk) finish(next);
             fetch(next, 0, 0);
             if (STAGES == 2) oa.issue(kt + 2, cur, wave);
             mma(3);
@@ -457,6 +512,7 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
         prologue(I1{});
         if constexpr (STAGES > 2) prologue(I2{});
         meet();
+        if (mend && nk == 1) finish(lds0);
         fetch(lds0, 0, 0);
         for (int kt = 0; kt < nk; kt += STAGES) {
             body(I0{}, kt);
@@ -1011,11 +1067,9 @@ void launch(const GemmArgs& p, hipStream_t stream) {
 
 }  // namespace smallk
 
-// An operand the matrix-core kernels read in place: 16-byte aligned, and its
-// leading dimension, batch stride and contiguous extent (K when K-major, M or
-// N otherwise) whole numbers of V-element packets; rows that do not overlap
-// (the panel's bound then is the end of its last row) and a panel (up to 256
-// rows of K, or a K tile of rows) under 4 GiB, the reach of its resource.
+// An operand the tile kernel reads in place: rows that do not overlap (the
+// panel's bound is the end of its last row) and a panel (a tile's rows of K,
+// or a K tile of rows) under 4 GiB, the reach of its resource.
 template <typename T>
 bool panel_fits(int64_t ld, bool kmajor) {
     constexpr int64_t E = sizeof(typename Elem<T>::storage);
@@ -1024,36 +1078,37 @@ bool panel_fits(int64_t ld, bool kmajor) {
 }
 
 template <typename T>
-bool operand_ok(const void* ptr, int64_t ld, int64_t stride, bool kmajor, int64_t mn, int64_t k) {
-    constexpr int V = Mfma<T>::V;
-    return aligned16(ptr) && ld % V == 0 && stride % V == 0 && (kmajor ? k : mn) % V == 0 &&
-           ((kmajor ? mn : k) == 1 || ld >= (kmajor ? k : mn)) && panel_fits<T>(ld, kmajor);
+bool operand_ok(int64_t ld, bool kmajor, int64_t mn, int64_t k) {
+    return ((kmajor ? mn : k) == 1 || ld >= (kmajor ? k : mn)) && panel_fits<T>(ld, kmajor);
 }
 
 bool tiles_fit(const GemmArgs& p) {
     return (p.m + 63) / 64 * ((p.n + 63) / 64) < (int64_t(1) << 31) && p.k < (int64_t(1) << 31);
 }
 
+// Whole dwords everywhere and whole packets along K: the tile kernel without
+// ODD.  (A split's slices but the last are whole K tiles.)
 template <typename T>
-bool mfma_eligible(const GemmArgs& p) {
-    return p.k > 0 && operand_ok<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, p.k) &&
-           operand_ok<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, p.k) && tiles_fit(p);
+bool whole_dwords(const void* x, int64_t ld, int64_t stride, bool kmajor, int64_t mn, int64_t k) {
+    constexpr int64_t E = sizeof(typename Elem<T>::storage);
+    if (kmajor && k % Mfma<T>::V != 0) return false;
+    return E == 4 || (reinterpret_cast<uintptr_t>(x) % 4 == 0 && ld % 2 == 0 && stride % 2 == 0 && (kmajor || mn % 2 == 0));
 }
 
-template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
 void launch_chunk(const GemmArgs& p, hipStream_t stream) {
     constexpr int THREADS = 4 * kWave;
     const int64_t tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
     const dim3 grid(static_cast<unsigned>(tiles), 1u, static_cast<unsigned>(p.batch));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     if (a_kmajor && b_kmajor) {
-        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     } else if (a_kmajor) {
-        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     } else if (b_kmajor) {
-        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     } else {
-        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     }
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
@@ -1071,7 +1126,13 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
                      : static_cast<void*>(static_cast<S*>(whole.c) + b0 * whole.stride_c);
         if (whole.cin != nullptr) p.cin = static_cast<const S*>(whole.cin) + b0 * whole.cin_stride_b;
         if (F32OUT) p.k_total = whole.k_total - b0 * whole.k;
-        launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT>(p, stream);
+        const int64_t k = F32OUT ? p.k_total : p.k;
+        if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
+            whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, false>(p, stream);
+        } else {
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, true>(p, stream);
+        }
     }
 }
 constexpr int kFinishBlock = 256;
@@ -1340,27 +1401,6 @@ void launch_mfma(const GemmArgs& p, hipStream_t stream) {
     }
 }
 
-// Products with an operand the matrix-core kernels cannot read in place (an
-// odd K or leading dimension: a vocabulary of 50257, a Linear(1023, ...), a
-// column slice at an odd offset) copy that operand into a dense K-major
-// workspace [batch][M or N][K'], K' = K rounded up to the packet, with the
-// columns K..K' zeroed.  An odd K alone only forces the K-major operands
-// into such copies (their 16-byte packets run along K and would cross the
-// end of a row); an operand stored with M or N contiguous stays where it
-// is, since the bounds-checked tile loaders give zeros for its rows k >= K,
-// and the product keeps K.  Before, an odd K repacked both operands: the
-// dX = dY W of an LM head with a 50257 vocabulary (bf16 1 x 50257 x 4096)
-// transposed the whole 400 MB weight on every call.  The copies cost a pass
-// over the operands; the general kernel
-// they replace runs ~16x slower than the matrix cores (2047^3 in bfloat16:
-// 692 us there, 63 us repacked).  Products under kRepackMinMacs
-// multiply-adds (about 160^3) keep the general kernel, which needs no
-// workspace and no extra launches: measured, 130^3 is 2 us faster there and
-// 200^3 7 us faster repacked.
-constexpr double kRepackMinMacs = double(int64_t(1) << 22);
-
-void check_status(int status) { TP_AMD_CHECK(status == 0, last_error()); }
-
 template <typename T>
 struct DtypeOf;
 template <>
@@ -1370,110 +1410,158 @@ struct DtypeOf<bf16_t> { static constexpr int value = TP_AMD_BFLOAT16; };
 template <>
 struct DtypeOf<f16_t> { static constexpr int value = TP_AMD_FLOAT16; };
 
-// A K-major source in one pass: dst row q (of bs x rows) = the source row
-// (b, r) = (q / rows, q % rows) at src + b stride + r ld, elements 0..k, then
-// zeros to kp.  A thread writes one 16-byte packet (kp is a whole number of
-// them) from element loads, which are unaligned when ld or k is odd.
-constexpr int kRepackBlock = 256;
+// dst [batch][rows_out][per_row packets] = src's rows x cols of each batch
+// entry (rows ld apart, entries `stride`), zeros around them.  Bound by
+// memory: a thread has four 16-byte packets in flight, read at any element.
+constexpr int kRepackBlock = 256, kRepackUnroll = 4;
 
 template <typename S>
-__global__ __launch_bounds__(kRepackBlock) void repack_rows_kernel(S* __restrict__ dst, const S* __restrict__ src,
-                                                                   int64_t total, int64_t rows, int64_t ld,
-                                                                   int64_t stride, int64_t k, int64_t kp) {
+__global__ __launch_bounds__(kRepackBlock) void repack_kernel(S* __restrict__ dst, const S* __restrict__ src,
+                                                              int64_t total, int64_t rows_out, int64_t per_row,
+                                                              FastDiv by_rows, FastDiv by_packets, int64_t rows,
+                                                              int64_t cols, int64_t ld, int64_t stride) {
     constexpr int N = 16 / sizeof(S);
-    const int64_t j0 = (static_cast<int64_t>(blockIdx.x) * kRepackBlock + threadIdx.x) * N;
-    if (j0 >= kp) return;
-    for (int64_t q = blockIdx.y; q < total; q += gridDim.y) {
-        const S* row = src + (q / rows) * stride + (q % rows) * ld;
-        S v[N];
+    const bool small = total < (int64_t{1} << 31);
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * (kRepackBlock * kRepackUnroll) + threadIdx.x;
+    uint4 v[kRepackUnroll];
 #pragma unroll
-        for (int e = 0; e < N; ++e) v[e] = j0 + e < k ? row[j0 + e] : S{};
-        uint4 w;
-        __builtin_memcpy(&w, v, 16);
-        *reinterpret_cast<uint4*>(dst + q * kp + j0) = w;
+    for (int u = 0; u < kRepackUnroll; ++u) {
+        const int64_t i = first + u * kRepackBlock;
+        if (i >= total) break;
+        const int64_t row = small ? fastdiv(static_cast<uint32_t>(i), by_packets) : i / per_row;
+        const int64_t b = small ? fastdiv(static_cast<uint32_t>(row), by_rows) : row / rows_out;
+        const int64_t r = row - b * rows_out, c = (i - row * per_row) * N;
+        const S* from = src + b * stride + r * ld + c;
+        if (r < rows && c + N <= cols) {
+            v[u] = load_raw_any(from);
+        } else {
+            S t[N];
+#pragma unroll
+            for (int e = 0; e < N; ++e) t[e] = r < rows && c + e < cols ? from[e] : S{};
+            __builtin_memcpy(&v[u], t, 16);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kRepackUnroll; ++u) {
+        const int64_t i = first + u * kRepackBlock;
+        if (i < total) reinterpret_cast<uint4*>(dst)[i] = v[u];
     }
 }
 
-// x logical [bs][rows][k] (element (b, r, j) at x + b stride + r ld + j when
-// K-major, + j ld + r otherwise) -> ws [bs][rows][kp], columns k..kp zero.
-// K-major sources take repack_rows_kernel; the others the transpose copy and
-// a fill of the padding.
-template <typename S>
-void repack_kmajor(int device, const void* x, int64_t ld, int64_t stride, bool kmajor, int64_t bs,
-                   int64_t rows, int64_t k, int64_t kp, void* ws, hipStream_t stream) {
-    constexpr int esize = sizeof(S);
-    if (kmajor) {
-        constexpr int N = 16 / esize;
-        const int64_t total = bs * rows;
-        const dim3 grid(static_cast<unsigned>((kp / N + kRepackBlock - 1) / kRepackBlock),
-                        static_cast<unsigned>(std::min<int64_t>(total, 65535)));
-        repack_rows_kernel<S><<<grid, kRepackBlock, 0, stream>>>(static_cast<S*>(ws), static_cast<const S*>(x),
-                                                                 total, rows, ld, stride, k, kp);
+// An operand's copy: its layout kept, rows whole 128-byte lines, and K (the
+// columns when K-major, the rows otherwise) zero-padded to kp.
+template <typename T>
+struct Repack {
+    static constexpr int64_t E = sizeof(typename Elem<T>::storage), kLine = 128 / E;
+    int64_t rows, cols, ld, stride, rows_out, ld_out, batch;
+
+    Repack(int64_t ld_, int64_t stride_, bool kmajor, int64_t batch_, int64_t mn, int64_t k, int64_t kp)
+        : rows(kmajor ? mn : k), cols(kmajor ? k : mn), ld(ld_), stride(stride_), rows_out(kmajor ? mn : kp),
+          ld_out(((kmajor ? kp : mn) + kLine - 1) / kLine * kLine), batch(stride_ == 0 ? 1 : batch_) {}
+    int64_t elems() const { return batch * rows_out * ld_out; }
+    int64_t out_stride() const { return stride == 0 ? 0 : rows_out * ld_out; }  // a broadcast operand is copied once
+    void launch(const void* src, void* dst, hipStream_t stream) const {
+        using S = typename Elem<T>::storage;
+        const int64_t per_row = ld_out * E / 16, total = batch * rows_out * per_row;
+        const bool small = total < (int64_t{1} << 31);
+        const FastDiv by_rows = make_fastdiv(small ? static_cast<uint32_t>(rows_out) : 1);
+        const FastDiv by_packets = make_fastdiv(small ? static_cast<uint32_t>(per_row) : 1);
+        constexpr int64_t kBlock = kRepackBlock * kRepackUnroll;
+        repack_kernel<S><<<static_cast<unsigned>((total + kBlock - 1) / kBlock), kRepackBlock, 0, stream>>>(
+            static_cast<S*>(dst), static_cast<const S*>(src), total, rows_out, per_row, by_rows, by_packets, rows, cols,
+            ld, stride);
         TP_AMD_HIP_CHECK(hipGetLastError());
-        return;
     }
-    const int64_t sizes[3] = {bs, rows, k};
-    const int64_t dst[3] = {rows * kp, kp, 1};
-    const int64_t src[3] = {stride, kmajor ? ld : 1, kmajor ? 1 : ld};
-    check_status(tp_amd_launch_strided_copy(device, esize, 3, sizes, ws, dst, x, src));
-    if (kp > k) {
-        const uint64_t zero = 0;
-        const int64_t pad[3] = {bs, rows, kp - k};
-        check_status(tp_amd_launch_fill(device, esize, &zero, 3, pad, static_cast<char*>(ws) + k * esize, dst));
-    }
-}
+};
 
 template <typename T>
-void launch_repacked(const GemmArgs& p, hipStream_t stream) {
+bool packets_aligned(const void* x, int64_t ld, int64_t stride) {
     constexpr int V = Mfma<T>::V;
-    constexpr int E = sizeof(typename Elem<T>::storage);
+    return aligned16(x) && ld % V == 0 && stride % V == 0;
+}
+
+// Whether a 16-bit product gains by copies of its operands that are not
+// whole aligned packets.  Read in place, such an operand costs a product that
+// fills the chip time per multiply-add (each load touches twice the cache
+// lines): about 0.70e-15 s for a K-major and 0.40e-15 s for an M/N-major one
+// (bf16 8191 x 11007 x 4095 in place 1172 us NT, 1081 NN, 1006 TN, on copies
+// 760, 794 and 815).  The copies cost one pass at about 5 TB/s and a launch
+// each: 2047^3 takes 32 us in place and would take 40.  float32 is bound by
+// its MFMAs and loses nothing in place.
+template <typename T>
+bool repack_pays(const GemmArgs& p) {
+    constexpr int64_t E = sizeof(typename Elem<T>::storage);
+    if (E != 2) return false;
+    const bool pad = p.k % Mfma<T>::V != 0;
+    double in_place = 0.0, copies = 0.0;
+    auto add = [&](const void* x, int64_t ld, int64_t stride, bool kmajor, int64_t mn) {
+        const bool odd = !packets_aligned<T>(x, ld, stride);
+        if (odd) in_place += kmajor ? 0.70e-15 : 0.40e-15;
+        if (odd || pad) {
+            copies += 5e-6 + 2.0 * E * static_cast<double>(stride == 0 ? 1 : p.batch) * static_cast<double>(mn) *
+                                 static_cast<double>(p.k) / 5e12;
+        }
+    };
+    add(p.a, p.lda, p.stride_a, !p.trans_a, p.m);
+    add(p.b, p.ldb, p.stride_b, p.trans_b, p.n);
+    return in_place * static_cast<double>(p.batch) * static_cast<double>(p.m) * static_cast<double>(p.n) *
+               static_cast<double>(p.k) > copies;
+}
+
+// A product on copies of its operands: of those the tile kernel cannot read
+// in place (rows that overlap, or too far apart for its panel), and of those
+// that are not aligned packets where that pays.
+template <typename T>
+void launch_repacked(const GemmArgs& p, bool pays, hipStream_t stream) {
     int device = 0;
     TP_AMD_HIP_CHECK(hipGetDevice(&device));
-    const int64_t kp = (p.k + V - 1) / V * V;
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
-    // An in-place MN-major operand only needs its own packets aligned; for
-    // the check K is taken as padded (its K extent is not read in packets).
-    const bool fix_a = (a_kmajor && kp != p.k) || !operand_ok<T>(p.a, p.lda, p.stride_a, a_kmajor, p.m, kp);
-    const bool fix_b = (b_kmajor && kp != p.k) || !operand_ok<T>(p.b, p.ldb, p.stride_b, b_kmajor, p.n, kp);
-    // A batch-broadcast operand (stride 0) is copied once and stays broadcast.
-    const int64_t bs_a = p.stride_a == 0 ? 1 : p.batch, bs_b = p.stride_b == 0 ? 1 : p.batch;
-    const size_t bytes_a = fix_a ? static_cast<size_t>(bs_a * p.m * kp) * E : 0;
-    const size_t off_b = (bytes_a + 255) / 256 * 256;
-    const size_t bytes_b = fix_b ? static_cast<size_t>(bs_b * p.n * kp) * E : 0;
-    Workspace ws(off_b + bytes_b, device);
+    // A K that is no whole number of packets is padded in both copies.
+    const bool pad = pays && p.k % Mfma<T>::V != 0;
+    const int64_t kp = pad ? (p.k + Mfma<T>::BK - 1) / Mfma<T>::BK * Mfma<T>::BK : p.k;
+    const bool fix_a = !operand_ok<T>(p.lda, a_kmajor, p.m, p.k) || pad || (pays && !packets_aligned<T>(p.a, p.lda, p.stride_a));
+    const bool fix_b = !operand_ok<T>(p.ldb, b_kmajor, p.n, p.k) || pad || (pays && !packets_aligned<T>(p.b, p.ldb, p.stride_b));
+    const Repack<T> a(p.lda, p.stride_a, a_kmajor, p.batch, p.m, p.k, kp), b(p.ldb, p.stride_b, b_kmajor, p.batch, p.n, p.k, kp);
+    const size_t off_b = fix_a ? (a.elems() * a.E + 255) / 256 * 256 : 0;
+    Workspace ws(off_b + (fix_b ? b.elems() * b.E : 0), device);
     GemmArgs q = p;
-    // Both operands copied: K' with zero terms on both sides (the big
-    // kernels' whole K tiles apply).  Otherwise the in-place operand bounds
-    // the product at K, and the copies' zero columns are never summed in.
-    q.k = fix_a && fix_b ? kp : p.k;
+    q.k = kp;
     if (fix_a) {
-        repack_kmajor<typename Elem<T>::storage>(device, p.a, p.lda, p.stride_a, !p.trans_a, bs_a, p.m, p.k, kp,
-                                                 ws.get(), stream);
+        a.launch(p.a, ws.get(), stream);
         q.a = ws.get();
-        q.lda = kp;
-        q.stride_a = p.stride_a == 0 ? 0 : p.m * kp;
-        q.trans_a = false;
+        q.lda = a.ld_out;
+        q.stride_a = a.out_stride();
     }
     if (fix_b) {
         void* wb = static_cast<char*>(ws.get()) + off_b;
-        repack_kmajor<typename Elem<T>::storage>(device, p.b, p.ldb, p.stride_b, p.trans_b, bs_b, p.n, p.k, kp, wb,
-                                                 stream);
+        b.launch(p.b, wb, stream);
         q.b = wb;
-        q.ldb = kp;
-        q.stride_b = p.stride_b == 0 ? 0 : p.n * kp;
-        q.trans_b = true;
+        q.ldb = b.ld_out;
+        q.stride_b = b.out_stride();
     }
-    // A thin product reads its repacked operand through the thin kernel.
+    // A thin product reads its copies through the thin kernel.
     if (!launch_gemm_thin(DtypeOf<T>::value, q, stream)) launch_mfma<T>(q, stream);
 }
 
+// A product with operands the tile kernel cannot read in place and under
+// kRepackMinMacs multiply-adds (about 160^3) takes the general kernel, which
+// needs no workspace and no extra launches.
+constexpr double kRepackMinMacs = double(int64_t(1) << 22);
+
 template <typename T>
 void launch_typed(const GemmArgs& p, hipStream_t stream) {
-    if (mfma_eligible<T>(p)) {
-        launch_mfma<T>(p, stream);
-    } else if (p.k > 0 && tiles_fit(p) && panel_fits<T>(p.k + Mfma<T>::V, true) &&
-               double(p.batch) * double(p.m) * double(p.n) * double(p.k) >= kRepackMinMacs) {
-        launch_repacked<T>(p, stream);
+    if (p.k <= 0 || !tiles_fit(p)) {
+        launch_gemm_general<T>(p, stream);
+        return;
+    }
+    const bool in_place = operand_ok<T>(p.lda, !p.trans_a, p.m, p.k) && operand_ok<T>(p.ldb, p.trans_b, p.n, p.k);
+    const bool copies_fit = panel_fits<T>((p.trans_a ? p.m : p.k) + 128, !p.trans_a) &&
+                            panel_fits<T>((p.trans_b ? p.k : p.n) + 128, p.trans_b);
+    if (in_place) {
+        if (copies_fit && repack_pays<T>(p)) launch_repacked<T>(p, true, stream);
+        else launch_mfma<T>(p, stream);
+    } else if (copies_fit && double(p.batch) * double(p.m) * double(p.n) * double(p.k) >= kRepackMinMacs) {
+        launch_repacked<T>(p, false, stream);
     } else {
         launch_gemm_general<T>(p, stream);
     }

@@ -650,6 +650,50 @@ def test_gemm_abi_small_k(amd, dev, orc, dtype, ta, tb, k, cin_kind, bt, m, n):
     check(orc, got, want, dtype, f"small-K gemm {bt}x{m}x{n}x{k} ta={ta} tb={tb} {cin_kind}")
 
 
+def _embedded(orc, shape, ld, lead, dtype, seed):
+    """A matrix (or batch of them) with rows ``ld`` apart that starts ``lead``
+    elements into its storage and ends with it; NaN in the gaps.  Returns the
+    storage and the matrix."""
+    x = np.random.default_rng(seed).standard_normal(shape).astype(np.float32) * np.float32(0.25)
+    rows, cols = int(np.prod(shape[:-1])), shape[-1]
+    flat = np.full(lead + (rows - 1) * ld + cols, np.nan, np.float32)
+    np.lib.stride_tricks.as_strided(flat[lead:], (rows, cols), (4 * ld, 4))[:] = x.reshape(rows, cols)
+    x = orc.to_float(orc.from_float(x, dtype), dtype)
+    return orc.from_float(flat, dtype), x
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
+                         ids=["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("bt,m,n,k,pad,lead", [
+    (1, 129, 67, 64, 0, 1), (1, 65, 127, 65, 1, 1), (1, 66, 131, 71, 0, 0), (1, 97, 33, 1, 1, 1), (1, 35, 70, 129, 3, 1),
+    (3, 63, 65, 193, 0, 1), (1, 257, 255, 4099, 0, 1), (1, 2601, 2603, 2602, 1, 1)],
+    ids=["whole-K-tile", "one-past", "odd-K", "K-1", "two-tiles-and-one", "batch", "split", "copies"])
+def test_gemm_operands_at_any_element(amd, dev, orc, dtype, ta, tb, bt, m, n, k, pad, lead):
+    """Operands that start, end and step at odd elements, with NaN around
+    them, are read in place (the largest 16-bit one through aligned copies),
+    up to the last element and no further."""
+    lib = amd.load()
+    lda, ldb = (m if ta else k) + pad, (n if tb is False else k) + pad
+    a, A = _embedded(orc, (bt, k, m) if ta else (bt, m, k), lda, lead, dtype, 21)
+    b, B = _embedded(orc, (bt, n, k) if tb else (bt, k, n), ldb, lead, dtype, 22)
+    da, db = dev.from_numpy(a, dtype=dtype), dev.from_numpy(b, dtype=dtype)
+    out = dev.empty((bt, m, n), dtype=dtype)
+    e = 4 if dtype == F32 else 2
+    st = lib.tp_amd_launch_gemm(0, dtype, bt, m, n, k, 1.0, da.data_ptr + lead * e, lda, (k if ta else m) * lda, int(ta),
+                                db.data_ptr + lead * e, ldb, (n if tb else k) * ldb, int(tb), 0.0, 0, 0, 0, 0,
+                                out.data_ptr, n, m * n)
+    assert st == 0, lib.tp_mlu_last_error()
+    A = np.swapaxes(A, -1, -2) if ta else A
+    B = np.swapaxes(B, -1, -2) if tb else B
+    rows = np.r_[0:2, 61:67, m - 3:m] if m > 1000 else np.arange(m)
+    rows = rows[rows < m]
+    want = np.matmul(A[:, rows].astype(np.float64), B.astype(np.float64))
+    got = out.numpy()[:, rows]
+    assert not np.isnan(orc.to_float(got, dtype)).any(), "an element outside the operands reached the product"
+    check(orc, got, want, dtype, f"odd gemm {bt}x{m}x{n}x{k} ta={ta} tb={tb}")
+
+
 @pytest.mark.parametrize("m,n,k,dtype", [(64, 64, 64, F32), (512, 512, 512, F32), (512, 512, 512, BF16),
                                          (4096, 4096, 256, BF16), (1024, 1024, 1024, F32)],
                          ids=["fma-fp32", "mfma-fp32", "mfma-bf16", "big-bf16", "mfma-fp32-1024"])
