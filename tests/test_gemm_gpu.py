@@ -694,6 +694,69 @@ def test_gemm_operands_at_any_element(amd, dev, orc, dtype, ta, tb, bt, m, n, k,
     check(orc, got, want, dtype, f"odd gemm {bt}x{m}x{n}x{k} ta={ta} tb={tb}")
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
+                         ids=["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("m,n,k,cin_kind", [(4096, 4096, 1024, "none"), (4090, 4081, 1001, "full"),
+                                            (4090, 4081, 1001, "bias-row")],
+                         ids=["whole-tiles", "ragged-full", "ragged-bias"])
+def test_large_float32_product_in_planes(amd, dev, orc, ta, tb, m, n, k, cin_kind):
+    """A float32 product of 256 tiles of 256 x 256, as six products of
+    bfloat16 planes.  Rows across the edges of tiles against float64: what
+    the planes leave out and each of the k / 16 full-size roundings are
+    under 2^-24 of a term, so the error stays under that of a sum rounded
+    term by term, 2^-24 sqrt(k) of the rows' norm."""
+    lib = amd.load()
+    rng = np.random.default_rng(31)
+    lead = 1 if k % 2 else 0
+    lda, ldb = (m if ta else k) + lead, (k if tb else n) + lead
+    a, A = _embedded(orc, (k, m) if ta else (m, k), lda, lead, F32, 32)
+    b, B = _embedded(orc, (n, k) if tb else (k, n), ldb, lead, F32, 33)
+    scale = rng.uniform(0.5, 2.0, n).astype(np.float32)
+    da, db = dev.from_numpy(a, dtype=F32), dev.from_numpy(b, dtype=F32)
+    cin, rs, cs, beta = {"none": (None, 0, 0, 0.0), "full": (rng.standard_normal((m, n)).astype(np.float32), n, 1, 2.0),
+                         "bias-row": (scale, 0, 1, -1.0)}[cin_kind]
+    dc = dev.from_numpy(cin, dtype=F32) if cin is not None else None
+    out = dev.empty((m, n), dtype=F32)
+    st = lib.tp_amd_launch_gemm(0, F32, 1, m, n, k, 0.5, da.data_ptr + 4 * lead, lda, 0, int(ta), db.data_ptr + 4 * lead,
+                                ldb, 0, int(tb), beta, dc.data_ptr if dc is not None else 0, rs, cs, 0, out.data_ptr, n, 0)
+    assert st == 0, lib.tp_mlu_last_error()
+    rows = np.r_[0, 127, 255, 256, 2047, m - 2, m - 1]
+    want = 0.5 * (np.asarray(A.T if ta else A)[rows].astype(np.float64) @ np.asarray(B.T if tb else B).astype(np.float64))
+    if cin is not None:
+        want += beta * (cin[rows] if rs else cin).astype(np.float64)
+    got = out.numpy()[rows].astype(np.float64)
+    assert np.isfinite(got).all()
+    error = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert error.max() <= 2.0**-24 * np.sqrt(k), error
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38, 1e-36, 1e-42])
+def test_large_float32_product_outside_the_planes(dev, ops, value):
+    """An element that bfloat16 planes do not hold exactly takes the whole
+    product to the float32 tiles: infinities and NaN land where IEEE
+    arithmetic puts them, and a row of such values keeps its precision."""
+    m, n, k = 4096, 4096, 1024
+    rng = np.random.default_rng(34)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = (rng.standard_normal((k, n)) * 0.25).astype(np.float32)
+    if abs(value) < 1:
+        a[300] *= np.float32(value)
+    else:
+        a[300, 17] = value
+    b[17, 40] = 0.0
+    got = ops.mm(dev.from_numpy(a), dev.from_numpy(b)).numpy()[[0, 300, m - 1]]
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = a[[0, 300, m - 1]].astype(np.float64) @ b.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    big = ~np.isfinite(want) | (np.abs(want) > 3.4e38)
+    assert np.array_equal(np.isinf(got), big & ~np.isnan(want))
+    for g, w in zip(got, want):
+        ok = np.isfinite(g) & np.isfinite(w)
+        # 1e-42 leaves a float32 few bits: half a step of 2^-149 a rounding
+        bar = 2.0**-24 * np.sqrt(k) * np.linalg.norm(w[ok]) + 2.0**-150 * k * np.sqrt(n)
+        assert np.linalg.norm(g[ok].astype(np.float64) - w[ok]) <= bar
+
+
 @pytest.mark.parametrize("m,n,k,dtype", [(64, 64, 64, F32), (512, 512, 512, F32), (512, 512, 512, BF16),
                                          (4096, 4096, 256, BF16), (1024, 1024, 1024, F32)],
                          ids=["fma-fp32", "mfma-fp32", "mfma-bf16", "big-bf16", "mfma-fp32-1024"])
