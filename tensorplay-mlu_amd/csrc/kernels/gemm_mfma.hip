@@ -739,7 +739,7 @@ struct Operand {
 // is under 2^-25 of a term, and the running sum is rounded at its full size
 // once per 16 k, eight times less often than by the float32 MFMA.  C and Cin
 // are float32, and a tile may reach past them (the planes are padded with
-// zeros).  split_pays has the times and the errors.
+// zeros).  split_planes_k has the times and the errors.
 template <typename T, bool A_KMAJOR, bool B_KMAJOR, int WM, int WN, bool SPLIT = false>
 __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kernel(GemmArgs p) {
     using O = std::conditional_t<SPLIT, float, T>;
@@ -765,13 +765,16 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
     const int lane = threadIdx.x % kWave;
     const int wm = wave / WN, wn = wave % WN;
     const int l32 = lane % 32, half = lane / 32;
-    const int n1 = static_cast<int>(p.k / BK);
-    const int nk = SPLIT ? 6 * n1 : n1;
     const int64_t bi = blockIdx.z;
+    // With SPLIT, batch entry bi is the slice of p.k from bi p.k on of
+    // k_total (the last one shorter), in every plane.
+    const int64_t kk = SPLIT && p.k_total - bi * p.k < p.k ? p.k_total - bi * p.k : p.k;
+    const int n1 = static_cast<int>(kk / BK);
+    const int nk = SPLIT ? 6 * n1 : n1;
 
     Operand<A_KMAJOR, W, TM> oa;
     Operand<B_KMAJOR, W, TN> ob;
-    const int64_t rows_k = SPLIT ? 3 * p.k : p.k;
+    const int64_t rows_k = SPLIT ? 2 * p.k_total + kk : p.k;  // to the end of a slice's last plane
     oa.init(static_cast<const In*>(p.a) + bi * p.stride_a, p.lda, m0, rows_k, wave, lane, wm * TM * 32);
     ob.init(static_cast<const In*>(p.b) + bi * p.stride_b, p.ldb, n0, rows_k, wave, lane, wn * TN * 32);
     auto issue_a = [&](int kt, char* tile) {
@@ -1201,7 +1204,8 @@ template <typename T, int V>
 __global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(
     const float* part, int slices, int64_t m, int64_t n, float alpha, float beta,
     const typename Elem<T>::storage* cin, int64_t cin_rs, int64_t cin_cs, typename Elem<T>::storage* c,
-    int64_t ldc) {
+    int64_t ldc, const uint32_t* inexact) {
+    if (inexact != nullptr && *inexact != 0) return;  // the tile kernel wrote C
     typedef float Vec __attribute__((ext_vector_type(V)));
     const int64_t col = (static_cast<int64_t>(blockIdx.x) * kFinishBlock + threadIdx.x) * V;
     if (col >= n) return;
@@ -1253,7 +1257,7 @@ void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t
     auto* kernel = vec ? splitk_finish_kernel<T, 4> : splitk_finish_kernel<T, 1>;
     kernel<<<grid, kFinishBlock, 0, stream>>>(part, slices, p.m, p.n, p.alpha, p.beta,
                                               static_cast<const S*>(p.cin), p.cin_rs, p.cin_cs,
-                                              static_cast<S*>(p.c), p.ldc);
+                                              static_cast<S*>(p.c), p.ldc, p.inexact);
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1682,13 +1686,29 @@ struct Planes {
 // x 4096 x 1000 488 and 334; 5000 x 6000 x 700 342 and 237.  Relative error
 // against float64 (normal operands): 4096 x 4096 x 8192 1.6e-6 there, 5.7e-7 in
 // planes; 4096^3 1.1e-6 and 4.0e-7; K = 1024 5.7e-7 and 1.8e-7.
-bool split_pays(const GemmArgs& p, const Planes& a, const Planes& b, int64_t cus) {
-    constexpr double kRoundUs = 0.145, kBytesPerUs = 5e6, kLaunchUs = 15.0;
-    if (p.batch != 1 || !a.fit() || !b.fit() || tiles_of(p, 256, 256) < cus) return false;
-    const double rounds = double((tiles_of(p, 256, 256) + cus - 1) / cus);
-    const double kp = double((p.k + 63) / 64 * 64);
-    const double us = rounds * kp * kRoundUs + double(a.bytes() + b.bytes()) / 6 * 10 / kBytesPerUs + kLaunchUs;
-    return us < plan_tiles<float>(p, cus).us;
+// Few tiles take slices of K, added by splitk_finish_kernel: 2048 x 4096 x
+// 4096 486 us there and 375 in two slices, 2500 x 4000 x 4000 608 and 470,
+// 3500 x 1500 x 2500 232 and 192.  The float32 tiles' expected time is 8-15 %
+// under the measured one at these sizes.
+// Returns the slices' K, or 0 where the float32 tiles are faster.
+int64_t split_planes_k(const GemmArgs& p, const Planes& a, const Planes& b, int64_t cus) {
+    constexpr double kRoundUs = 0.145, kBytesPerUs = 5e6, kLaunchUs = 15.0, kFinishUs = 4.0, kPartialsPerUs = 1.25e6;
+    constexpr int64_t kMinSlice = 512;
+    if (p.batch != 1 || !a.fit() || !b.fit()) return 0;
+    const int64_t tiles = tiles_of(p, 256, 256), kp = (p.k + 63) / 64 * 64;
+    const double pass = double(a.bytes() + b.bytes()) / 6 * 10 / kBytesPerUs + kLaunchUs;
+    double least = 1.08 * plan_tiles<float>(p, cus).us;
+    int64_t best = 0;
+    for (int64_t s = 1; s <= 8 && (s == 1 || kp >= s * kMinSlice); ++s) {
+        const int64_t ks = ((kp + s - 1) / s + 63) / 64 * 64;
+        double us = double((tiles * s + cus - 1) / cus) * double(ks) * kRoundUs + pass;
+        if (s > 1) us += kFinishUs + double(p.m) * double(p.n) * double(2 * s + 1) / kPartialsPerUs;
+        if (us < least) {
+            least = us;
+            best = ks;
+        }
+    }
+    return best;
 }
 
 bool launch_split_planes(const GemmArgs& p, hipStream_t stream) {
@@ -1696,10 +1716,12 @@ bool launch_split_planes(const GemmArgs& p, hipStream_t stream) {
     TP_AMD_HIP_CHECK(hipGetDevice(&device));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     const Planes a(p.lda, a_kmajor, p.m, p.k), b(p.ldb, b_kmajor, p.n, p.k);
-    if (!split_pays(p, a, b, cu_count(device))) return false;
+    const int64_t ks = split_planes_k(p, a, b, cu_count(device));
+    if (ks == 0) return false;
+    const int64_t kp = (p.k + 63) / 64 * 64, slices = (kp + ks - 1) / ks, mn = p.m * p.n;
     Workspace ws;
     try {
-        ws = Workspace(static_cast<size_t>(256 + a.bytes() + b.bytes()), device);
+        ws = Workspace(static_cast<size_t>(256 + a.bytes() + b.bytes() + (slices > 1 ? slices * mn * 4 : 0)), device);
     } catch (const std::exception&) {
         return false;  // no room for the planes: the float32 tiles need none
     }
@@ -1719,13 +1741,28 @@ bool launch_split_planes(const GemmArgs& p, hipStream_t stream) {
     q.b = pb;
     q.ldb = b.ld_out();
     q.plane_b = 2 * b.plane;
-    q.k = (p.k + 63) / 64 * 64;
-    const dim3 grid(static_cast<unsigned>(tiles_of(p, 256, 256)));
+    q.k = ks;
+    q.k_total = kp;
+    q.stride_a = a_kmajor ? ks : ks * q.lda;
+    q.stride_b = b_kmajor ? ks : ks * q.ldb;
+    if (slices > 1) {
+        q.alpha = 1.0f;
+        q.beta = 0.0f;
+        q.c = pb + b.bytes();
+        q.ldc = p.n;
+        q.stride_c = mn;
+    }
+    const dim3 grid(static_cast<unsigned>(tiles_of(p, 256, 256)), 1u, static_cast<unsigned>(slices));
     if (a_kmajor && b_kmajor) big::gemm_big_kernel<bf16_t, true, true, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
     else if (a_kmajor) big::gemm_big_kernel<bf16_t, true, false, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
     else if (b_kmajor) big::gemm_big_kernel<bf16_t, false, true, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
     else big::gemm_big_kernel<bf16_t, false, false, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
     TP_AMD_HIP_CHECK(hipGetLastError());
+    if (slices > 1) {
+        GemmArgs f = p;
+        f.inexact = inexact;
+        launch_finish<float>(reinterpret_cast<const float*>(pb + b.bytes()), static_cast<int>(slices), f, stream);
+    }
     return true;
 }
 

@@ -697,11 +697,12 @@ def test_gemm_operands_at_any_element(amd, dev, orc, dtype, ta, tb, bt, m, n, k,
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
                          ids=["NN", "TN", "NT", "TT"])
 @pytest.mark.parametrize("m,n,k,cin_kind", [(4096, 4096, 1024, "none"), (4090, 4081, 1001, "full"),
-                                            (4090, 4081, 1001, "bias-row")],
-                         ids=["whole-tiles", "ragged-full", "ragged-bias"])
+                                            (4090, 4081, 1001, "bias-row"), (2047, 4000, 4100, "full"),
+                                            (4096, 1000, 7000, "none")],
+                         ids=["whole-tiles", "ragged-full", "ragged-bias", "slices-full", "slices"])
 def test_large_float32_product_in_planes(amd, dev, orc, ta, tb, m, n, k, cin_kind):
-    """A float32 product of 256 tiles of 256 x 256, as six products of
-    bfloat16 planes.  Rows across the edges of tiles against float64: what
+    """A float32 product large enough for six products of bfloat16 planes, on
+    256 tiles of 256 x 256 or on fewer in slices of K.  Rows across the edges of tiles against float64: what
     the planes leave out and each of the k / 16 full-size roundings are
     under 2^-24 of a term, so the error stays under that of a sum rounded
     term by term, 2^-24 sqrt(k) of the rows' norm."""
@@ -720,7 +721,7 @@ def test_large_float32_product_in_planes(amd, dev, orc, ta, tb, m, n, k, cin_kin
     st = lib.tp_amd_launch_gemm(0, F32, 1, m, n, k, 0.5, da.data_ptr + 4 * lead, lda, 0, int(ta), db.data_ptr + 4 * lead,
                                 ldb, 0, int(tb), beta, dc.data_ptr if dc is not None else 0, rs, cs, 0, out.data_ptr, n, 0)
     assert st == 0, lib.tp_mlu_last_error()
-    rows = np.r_[0, 127, 255, 256, 2047, m - 2, m - 1]
+    rows = np.r_[0, 127, 255, 256, 1792, m - 2, m - 1]
     want = 0.5 * (np.asarray(A.T if ta else A)[rows].astype(np.float64) @ np.asarray(B.T if tb else B).astype(np.float64))
     if cin is not None:
         want += beta * (cin[rows] if rs else cin).astype(np.float64)
