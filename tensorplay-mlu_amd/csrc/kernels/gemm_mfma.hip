@@ -372,7 +372,9 @@ struct Panel {
 // BLOCKS is how many blocks a CU holds (LDS and registers).
 // ODD (see Panel) is a variant of its own: its test for the last K tile in
 // the loop costs the others 3-8 % (float32 256 x 1024 x 4096 25.3 -> 27.4 us).
-template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
+// GATED: returns at once unless *p.inexact is set (a product left by the planes).
+template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD,
+          bool GATED>
 __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p) {
     using S = typename Elem<T>::storage;
     constexpr int WM = BM >= 64 ? 2 : 1, WN = 4 / WM, W = WM * WN;
@@ -397,8 +399,8 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
         else return lds3;
     };
 
-    if constexpr (sizeof(S) == 4 && !F32OUT) {
-        if (p.inexact != nullptr && *p.inexact == 0) return;
+    if constexpr (GATED) {
+        if (*p.inexact == 0) return;
     }
     const int grid_m = static_cast<int>((p.m + BM - 1) / BM);
     const int grid_n = static_cast<int>((p.n + BN - 1) / BN);
@@ -1150,25 +1152,25 @@ bool whole_dwords(const void* x, int64_t ld, int64_t stride, bool kmajor, int64_
     return E == 4 || (reinterpret_cast<uintptr_t>(x) % 4 == 0 && ld % 2 == 0 && stride % 2 == 0 && (kmajor || mn % 2 == 0));
 }
 
-template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD, bool GATED>
 void launch_chunk(const GemmArgs& p, hipStream_t stream) {
     constexpr int THREADS = 4 * kWave;
     const int64_t tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
     const dim3 grid(static_cast<unsigned>(tiles), 1u, static_cast<unsigned>(p.batch));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     if (a_kmajor && b_kmajor) {
-        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
     } else if (a_kmajor) {
-        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
     } else if (b_kmajor) {
-        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
     } else {
-        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
     }
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
 
-template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false, bool GATED = false>
 void launch_config(const GemmArgs& whole, hipStream_t stream) {
     constexpr int64_t kMaxZ = 65535;
     using S = typename Elem<T>::storage;
@@ -1184,9 +1186,9 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
         const int64_t k = F32OUT ? p.k_total : p.k;
         if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
             whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
-            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, false>(p, stream);
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, false, GATED>(p, stream);
         } else {
-            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, true>(p, stream);
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, true, GATED>(p, stream);
         }
     }
 }
@@ -1200,12 +1202,14 @@ constexpr int kFinishBlock = 256;
 // so no index is divided.  Float32 partials just written: bound by the
 // launch and one round trip (256 x 4096 in 4 slices 9.2 us with one element a
 // thread and 64-bit divisions, 4.0 us so).
-template <typename T, int V>
+template <typename T, int V, bool GATED>
 __global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(
     const float* part, int slices, int64_t m, int64_t n, float alpha, float beta,
     const typename Elem<T>::storage* cin, int64_t cin_rs, int64_t cin_cs, typename Elem<T>::storage* c,
     int64_t ldc, const uint32_t* inexact) {
-    if (inexact != nullptr && *inexact != 0) return;  // the tile kernel wrote C
+    if constexpr (GATED) {
+        if (*inexact != 0) return;  // the tile kernel wrote C
+    }
     typedef float Vec __attribute__((ext_vector_type(V)));
     const int64_t col = (static_cast<int64_t>(blockIdx.x) * kFinishBlock + threadIdx.x) * V;
     if (col >= n) return;
@@ -1246,7 +1250,7 @@ __global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(
     }
 }
 
-template <typename T>
+template <typename T, bool GATED = false>
 void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t stream) {
     using S = typename Elem<T>::storage;
     const bool vec = p.n % 4 == 0 && p.ldc % 4 == 0 &&
@@ -1254,7 +1258,7 @@ void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t
     const int64_t cols = vec ? p.n / 4 : p.n;
     const dim3 grid(static_cast<unsigned>((cols + kFinishBlock - 1) / kFinishBlock),
                     static_cast<unsigned>(std::min<int64_t>(p.m, 65535)));
-    auto* kernel = vec ? splitk_finish_kernel<T, 4> : splitk_finish_kernel<T, 1>;
+    auto* kernel = vec ? splitk_finish_kernel<T, 4, GATED> : splitk_finish_kernel<T, 1, GATED>;
     kernel<<<grid, kFinishBlock, 0, stream>>>(part, slices, p.m, p.n, p.alpha, p.beta,
                                               static_cast<const S*>(p.cin), p.cin_rs, p.cin_cs,
                                               static_cast<S*>(p.c), p.ldc, p.inexact);
@@ -1734,7 +1738,7 @@ bool launch_split_planes(const GemmArgs& p, hipStream_t stream) {
     b.launch(p.b, pb, inexact, stream);
     GemmArgs q = p;
     q.inexact = inexact;
-    launch_config<float, 128, 128, 2, 2>(q, stream);  // runs when the word is set
+    launch_config<float, 128, 128, 2, 2, false, true>(q, stream);  // runs when the word is set
     q.a = pa;
     q.lda = a.ld_out();
     q.plane_a = 2 * a.plane;
@@ -1761,7 +1765,7 @@ bool launch_split_planes(const GemmArgs& p, hipStream_t stream) {
     if (slices > 1) {
         GemmArgs f = p;
         f.inexact = inexact;
-        launch_finish<float>(reinterpret_cast<const float*>(pb + b.bytes()), static_cast<int>(slices), f, stream);
+        launch_finish<float, true>(reinterpret_cast<const float*>(pb + b.bytes()), static_cast<int>(slices), f, stream);
     }
     return true;
 }
