@@ -20,9 +20,11 @@
 //     tiles loaded straight into LDS by buffer loads and read back with
 //     ds_read_b128 (K-major operands) or ds_read_b64_tr_b16 (transposed
 //     views, read in place); no bounds checks anywhere in the K loop.
+//   * float32, large: three bfloat16 planes an operand and six products of
+//     them on `big` (launch_split_planes).
 //   * everything else: the tile kernel, gemm_tile_kernel, at a tile shape
 //     and a split over K that plan_tiles picks.
-// The last two load operand tiles straight into LDS, 128 bytes of K a step,
+// `big` and the tile kernel load operand tiles straight into LDS, 128 bytes of K a step,
 // read an operand where it lies in either orientation, and keep the next K
 // tiles' loads in flight while they multiply.  All kernels number their
 // tiles so each of the 8 XCDs walks a contiguous range in groups of 8 tile
