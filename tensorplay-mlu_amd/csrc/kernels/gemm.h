@@ -22,12 +22,6 @@ struct GemmArgs {
     // Split-K partials (gemm_tile_kernel's float32 output): the product's
     // whole K; batch entry s covers k = s k .. min((s + 1) k, k_total).
     int64_t k_total = 0;
-    // A float32 product in bfloat16 planes (gemm_big_kernel's SPLIT): bytes
-    // from one plane of an operand to the next, and the word that is set when
-    // an operand has no exact planes.  The SPLIT kernel returns when it is
-    // set, the tile kernel when it is given and not set.
-    int64_t plane_a = 0, plane_b = 0;
-    const uint32_t* inexact = nullptr;
 };
 
 // Any shape, stride and alignment (gemm.hip).

@@ -20,11 +20,9 @@
 //     tiles loaded straight into LDS by buffer loads and read back with
 //     ds_read_b128 (K-major operands) or ds_read_b64_tr_b16 (transposed
 //     views, read in place); no bounds checks anywhere in the K loop.
-//   * float32, large: three bfloat16 planes an operand and six products of
-//     them on `big` (launch_split_planes).
 //   * everything else: the tile kernel, gemm_tile_kernel, at a tile shape
 //     and a split over K that plan_tiles picks.
-// `big` and the tile kernel load operand tiles straight into LDS, 128 bytes of K a step,
+// The last two load operand tiles straight into LDS, 128 bytes of K a step,
 // read an operand where it lies in either orientation, and keep the next K
 // tiles' loads in flight while they multiply.  All kernels number their
 // tiles so each of the 8 XCDs walks a contiguous range in groups of 8 tile
@@ -374,9 +372,7 @@ struct Panel {
 // BLOCKS is how many blocks a CU holds (LDS and registers).
 // ODD (see Panel) is a variant of its own: its test for the last K tile in
 // the loop costs the others 3-8 % (float32 256 x 1024 x 4096 25.3 -> 27.4 us).
-// GATED: returns at once unless *p.inexact is set (a product left by the planes).
-template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD,
-          bool GATED>
+template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
 __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p) {
     using S = typename Elem<T>::storage;
     constexpr int WM = BM >= 64 ? 2 : 1, WN = 4 / WM, W = WM * WN;
@@ -401,9 +397,6 @@ __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p
         else return lds3;
     };
 
-    if constexpr (GATED) {
-        if (*p.inexact == 0) return;
-    }
     const int grid_m = static_cast<int>((p.m + BM - 1) / BM);
     const int grid_n = static_cast<int>((p.n + BN - 1) / BN);
     int pm, pn;
@@ -701,17 +694,7 @@ struct Operand {
 
     // Loads of K tile kt into `tile` (this wave's share of the 32 instructions).
     __device__ __forceinline__ void issue(int kt, char* tile, int wave) const {
-        issue_at(static_cast<uint32_t>(kt) * kstep, tile, wave);
-    }
-
-    // K tile kt of a product in planes: n1 K tiles a plane, the plane of
-    // pair i in nibble i of `order`.
-    __device__ __forceinline__ void issue(int kt, int n1, uint32_t order, uint32_t plane, char* tile, int wave) const {
-        const int pair = (kt >= n1) + (kt >= 2 * n1) + (kt >= 3 * n1) + (kt >= 4 * n1) + (kt >= 5 * n1);
-        issue_at(((order >> (4 * pair)) & 3) * plane + static_cast<uint32_t>(kt - pair * n1) * kstep, tile, wave);
-    }
-
-    __device__ __forceinline__ void issue_at(uint32_t kb, char* tile, int wave) const {
+        const uint32_t kb = static_cast<uint32_t>(kt) * kstep;
 #pragma unroll
         for (int i = 0; i < kIssue; ++i) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lds_ptr)(tile + (i * W + wave) * 1024), 16, voff,
@@ -736,20 +719,10 @@ struct Operand {
     }
 };
 
-// SPLIT: a float32 product on the bfloat16 units.  An operand comes as three
-// bfloat16 planes that add up to it exactly (8 + 8 + 8 bits of its 24), and
-// the product is the six pairs of planes that reach 2^-24 of it, the small
-// ones first: lo hi, hi lo, mid mid, mid hi, hi mid, hi hi.  What is left out
-// is under 2^-25 of a term, and the running sum is rounded at its full size
-// once per 16 k, eight times less often than by the float32 MFMA.  C and Cin
-// are float32, and a tile may reach past them (the planes are padded with
-// zeros).  split_planes_k has the times and the errors.
-template <typename T, bool A_KMAJOR, bool B_KMAJOR, int WM, int WN, bool SPLIT = false>
+template <typename T, bool A_KMAJOR, bool B_KMAJOR, int WM, int WN>
 __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kernel(GemmArgs p) {
-    using O = std::conditional_t<SPLIT, float, T>;
-    using S = typename Elem<O>::storage;
-    using In = typename Elem<T>::storage;
-    static_assert(sizeof(In) == 2, "16-bit operands");
+    using S = typename Elem<T>::storage;
+    static_assert(sizeof(S) == 2, "16-bit operands");
     constexpr int W = WM * WN;
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     // Two LDS objects rather than one array: the compiler can then tell that
@@ -758,10 +731,7 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
     __shared__ __attribute__((aligned(1024))) char lds0[STAGE];
     __shared__ __attribute__((aligned(1024))) char lds1[STAGE];
 
-    if constexpr (SPLIT) {
-        if (*p.inexact != 0) return;
-    }
-    const int grid_m = static_cast<int>((p.m + BM - 1) / BM), grid_n = static_cast<int>((p.n + BN - 1) / BN);
+    const int grid_m = static_cast<int>(p.m / BM), grid_n = static_cast<int>(p.n / BN);
     int pm, pn;
     tile_coords(blockIdx.x, grid_m, grid_n, pm, pn);
     const int64_t m0 = static_cast<int64_t>(pm) * BM, n0 = static_cast<int64_t>(pn) * BN;
@@ -769,26 +739,13 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
     const int lane = threadIdx.x % kWave;
     const int wm = wave / WN, wn = wave % WN;
     const int l32 = lane % 32, half = lane / 32;
+    const int nk = static_cast<int>(p.k / BK);
     const int64_t bi = blockIdx.z;
-    // With SPLIT, batch entry bi is the slice of p.k from bi p.k on of
-    // k_total (the last one shorter), in every plane.
-    const int64_t kk = SPLIT && p.k_total - bi * p.k < p.k ? p.k_total - bi * p.k : p.k;
-    const int n1 = static_cast<int>(kk / BK);
-    const int nk = SPLIT ? 6 * n1 : n1;
 
     Operand<A_KMAJOR, W, TM> oa;
     Operand<B_KMAJOR, W, TN> ob;
-    const int64_t rows_k = SPLIT ? 2 * p.k_total + kk : p.k;  // to the end of a slice's last plane
-    oa.init(static_cast<const In*>(p.a) + bi * p.stride_a, p.lda, m0, rows_k, wave, lane, wm * TM * 32);
-    ob.init(static_cast<const In*>(p.b) + bi * p.stride_b, p.ldb, n0, rows_k, wave, lane, wn * TN * 32);
-    auto issue_a = [&](int kt, char* tile) {
-        if constexpr (SPLIT) oa.issue(kt, n1, 0x001102, static_cast<uint32_t>(p.plane_a), tile, wave);
-        else oa.issue(kt, tile, wave);
-    };
-    auto issue_b = [&](int kt, char* tile) {
-        if constexpr (SPLIT) ob.issue(kt, n1, 0x010120, static_cast<uint32_t>(p.plane_b), tile, wave);
-        else ob.issue(kt, tile, wave);
-    };
+    oa.init(static_cast<const S*>(p.a) + bi * p.stride_a, p.lda, m0, p.k, wave, lane, wm * TM * 32);
+    ob.init(static_cast<const S*>(p.b) + bi * p.stride_b, p.ldb, n0, p.k, wave, lane, wn * TN * 32);
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -827,16 +784,16 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
     // out in substeps 0 and 1 (bf16 linear 8192 x 4096 x 11008 733 -> 706 us
     // on average over three alternating runs, 4096^3 1-2 % faster, the same
     // bits).
-    // do_issue: load B of K tile kt_next into `next`; do_issue_a: load A of
+    // do_issue: load B of K tile kt_next into `next`; issue_a: load A of
     // K tile kt_next + 1 into `cur` after the barrier.
-    auto body = [&](char* cur, char* next, int kt_next, auto do_issue, auto has_next, auto do_issue_a) {
+    auto body = [&](char* cur, char* next, int kt_next, auto do_issue, auto has_next, auto issue_a) {
         constexpr bool kIssue = decltype(do_issue)::value;
-        constexpr bool kIssueA = decltype(do_issue_a)::value;
+        constexpr bool kIssueA = decltype(issue_a)::value;
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
             fetch(cur, s + 1, (s + 1) & 1);
             if constexpr (kIssue) {
-                if (s == 0) issue_b(kt_next, next + TILE);
+                if (s == 0) ob.issue(kt_next, next + TILE, wave);
             }
             mma(s & 1);
             if (kIssue && s == 0) {
@@ -850,7 +807,7 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             fetch(next, 0, 0);
-            if constexpr (kIssueA) issue_a(kt_next + 1, cur);
+            if constexpr (kIssueA) oa.issue(kt_next + 1, cur, wave);
             mma(1);
             interleave<kMf, kReads, kIssueA ? 32 / W : 0>();
         } else {
@@ -860,9 +817,9 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
     };
 
     // K tile 0 whole, and A of K tile 1 (the host guarantees nk >= 2).
-    issue_a(0, lds0);
-    issue_b(0, lds0 + TILE);
-    issue_a(1, lds1);
+    oa.issue(0, lds0, wave);
+    ob.issue(0, lds0 + TILE, wave);
+    oa.issue(1, lds1, wave);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     fetch(lds0, 0, 0);
@@ -887,23 +844,7 @@ __global__ __launch_bounds__(WM * WN * kWave, (WM * WN) / 4) void gemm_big_kerne
             const int64_t col = n0 + wn * TN * 32 + j * 32 + l32;
             const int64_t rbase = m0 + wm * TM * 32 + i * 32 + 4 * half;
             S* cp = C + rbase * p.ldc + col;
-            if constexpr (SPLIT) {
-                if (col >= p.n) continue;
-                float c0 = 0.0f;
-                if (p.beta != 0.0f && p.cin_rs == 0) c0 = p.beta * Cin[col * p.cin_cs];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = rbase + 8 * g + r;
-                        if (row >= p.m) continue;
-                        const float v = acc[i][j][4 * g + r];
-                        if (p.beta == 0.0f) put_c(&cp[(8 * g + r) * p.ldc], p.alpha * v);
-                        else if (p.cin_rs == 0) put_c(&cp[(8 * g + r) * p.ldc], fmaf(p.alpha, v, c0));
-                        else put_c(&cp[(8 * g + r) * p.ldc], fmaf(p.beta, Cin[row * p.cin_rs + col * p.cin_cs], p.alpha * v));
-                    }
-                }
-            } else if (p.beta == 0.0f) {
+            if (p.beta == 0.0f) {
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
 #pragma unroll
@@ -1154,25 +1095,25 @@ bool whole_dwords(const void* x, int64_t ld, int64_t stride, bool kmajor, int64_
     return E == 4 || (reinterpret_cast<uintptr_t>(x) % 4 == 0 && ld % 2 == 0 && stride % 2 == 0 && (kmajor || mn % 2 == 0));
 }
 
-template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD, bool GATED>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
 void launch_chunk(const GemmArgs& p, hipStream_t stream) {
     constexpr int THREADS = 4 * kWave;
     const int64_t tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
     const dim3 grid(static_cast<unsigned>(tiles), 1u, static_cast<unsigned>(p.batch));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     if (a_kmajor && b_kmajor) {
-        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     } else if (a_kmajor) {
-        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     } else if (b_kmajor) {
-        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     } else {
-        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD, GATED><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
     }
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
 
-template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false, bool GATED = false>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT = false>
 void launch_config(const GemmArgs& whole, hipStream_t stream) {
     constexpr int64_t kMaxZ = 65535;
     using S = typename Elem<T>::storage;
@@ -1188,9 +1129,9 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
         const int64_t k = F32OUT ? p.k_total : p.k;
         if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
             whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
-            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, false, GATED>(p, stream);
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, false>(p, stream);
         } else {
-            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, true, GATED>(p, stream);
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, true>(p, stream);
         }
     }
 }
@@ -1204,14 +1145,11 @@ constexpr int kFinishBlock = 256;
 // so no index is divided.  Float32 partials just written: bound by the
 // launch and one round trip (256 x 4096 in 4 slices 9.2 us with one element a
 // thread and 64-bit divisions, 4.0 us so).
-template <typename T, int V, bool GATED>
+template <typename T, int V>
 __global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(
     const float* part, int slices, int64_t m, int64_t n, float alpha, float beta,
     const typename Elem<T>::storage* cin, int64_t cin_rs, int64_t cin_cs, typename Elem<T>::storage* c,
-    int64_t ldc, const uint32_t* inexact) {
-    if constexpr (GATED) {
-        if (*inexact != 0) return;  // the tile kernel wrote C
-    }
+    int64_t ldc) {
     typedef float Vec __attribute__((ext_vector_type(V)));
     const int64_t col = (static_cast<int64_t>(blockIdx.x) * kFinishBlock + threadIdx.x) * V;
     if (col >= n) return;
@@ -1252,7 +1190,7 @@ __global__ __launch_bounds__(kFinishBlock) void splitk_finish_kernel(
     }
 }
 
-template <typename T, bool GATED = false>
+template <typename T>
 void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t stream) {
     using S = typename Elem<T>::storage;
     const bool vec = p.n % 4 == 0 && p.ldc % 4 == 0 &&
@@ -1260,10 +1198,10 @@ void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t
     const int64_t cols = vec ? p.n / 4 : p.n;
     const dim3 grid(static_cast<unsigned>((cols + kFinishBlock - 1) / kFinishBlock),
                     static_cast<unsigned>(std::min<int64_t>(p.m, 65535)));
-    auto* kernel = vec ? splitk_finish_kernel<T, 4, GATED> : splitk_finish_kernel<T, 1, GATED>;
+    auto* kernel = vec ? splitk_finish_kernel<T, 4> : splitk_finish_kernel<T, 1>;
     kernel<<<grid, kFinishBlock, 0, stream>>>(part, slices, p.m, p.n, p.alpha, p.beta,
                                               static_cast<const S*>(p.cin), p.cin_rs, p.cin_cs,
-                                              static_cast<S*>(p.c), p.ldc, p.inexact);
+                                              static_cast<S*>(p.c), p.ldc);
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1304,7 +1242,6 @@ enum class Tile {
 struct TilePlan {
     Tile tile;
     int64_t slices = 1, ks = 0;
-    double us = 0.0;  // float32: the time it is expected to take
 };
 
 int64_t tiles_of(const GemmArgs& p, int64_t bm, int64_t bn) {
@@ -1384,7 +1321,6 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
                 best = plan;
             }
         }
-        best.us = least;
         return best;
     } else {
         if (thin <= 64) return plan_small_batch<T>(p, cus);
@@ -1607,171 +1543,6 @@ void launch_repacked(const GemmArgs& p, bool pays, hipStream_t stream) {
     if (!launch_gemm_thin(DtypeOf<T>::value, q, stream)) launch_mfma<T>(q, stream);
 }
 
-// A float32 operand as three bfloat16 planes, hi + mid + lo = x exactly, in
-// the operand's layout: K-major rows hold the planes side by side, M/N-major
-// ones stack them, padded with zeros to whole 256 x 64 tiles.  Sets *inexact
-// when x has an element that three bfloat16 do not hold, or whose products
-// could leave float32's range on the way: not finite, 2^56 and above, or
-// under 2^-100 and not 0.  Bound by memory (4 bytes in, 6 out); a thread
-// takes eight elements.
-constexpr int kPlanesBlock = 256;
-
-__global__ __launch_bounds__(kPlanesBlock) void split_planes_kernel(uint16_t* __restrict__ dst,
-                                                                    const float* __restrict__ src, int64_t total,
-                                                                    FastDiv by_packets, int64_t rows, int64_t cols,
-                                                                    int64_t ld, int64_t row_step, int64_t plane,
-                                                                    uint32_t* inexact) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kPlanesBlock + threadIdx.x;
-    if (i >= total) return;
-    const int64_t row = fastdiv(static_cast<uint32_t>(i), by_packets), c = (i - row * by_packets.d) * 8;
-    const float* from = src + row * ld + c;
-    float v[8];
-    if (row < rows && c + 8 <= cols) {
-        const uint4 a = load_raw_any(from), b = load_raw_any(from + 4);
-        __builtin_memcpy(v, &a, 16);
-        __builtin_memcpy(v + 4, &b, 16);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = row < rows && c + e < cols ? from[e] : 0.0f;
-    }
-    uint16_t out[3][8];
-    bool bad = false;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const uint32_t bits = __float_as_uint(v[e]) & 0x7fffffffu;
-        bad |= bits != 0 && (bits < (27u << 23) || bits >= (183u << 23));
-        out[0][e] = float_to_bf16(v[e]);
-        const float r1 = v[e] - bf16_to_float(out[0][e]);
-        out[1][e] = float_to_bf16(r1);
-        out[2][e] = float_to_bf16(r1 - bf16_to_float(out[1][e]));
-    }
-    if (bad) atomicOr(inexact, 1u);
-    uint16_t* to = dst + row * row_step + c;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        uint4 w;
-        __builtin_memcpy(&w, out[q], 16);
-        *reinterpret_cast<uint4*>(to + q * plane) = w;
-    }
-}
-
-__global__ void clear_word_kernel(uint32_t* word) { *word = 0; }
-
-struct Planes {
-    int64_t rows, cols, ld, rows_out, cols_out, plane;
-    bool kmajor;
-
-    Planes(int64_t ld_, bool kmajor_, int64_t mn, int64_t k)
-        : rows(kmajor_ ? mn : k), cols(kmajor_ ? k : mn), ld(ld_), kmajor(kmajor_) {
-        const int64_t mnp = (mn + 255) / 256 * 256, kp = (k + 63) / 64 * 64;
-        rows_out = kmajor ? mnp : kp;
-        cols_out = kmajor ? kp : mnp;
-        plane = kmajor ? kp : kp * mnp;
-    }
-    int64_t ld_out() const { return kmajor ? 3 * cols_out : cols_out; }
-    int64_t bytes() const { return 6 * rows_out * cols_out; }
-    // The kernel's 31-bit packet index, and the product kernel's resources.
-    bool fit() const {
-        return rows_out * (cols_out / 8) < (int64_t{1} << 31) &&
-               (kmajor ? 256 * ld_out() * 2 : bytes()) < (int64_t{1} << 32) - 4096;
-    }
-    void launch(const void* src, void* dst, uint32_t* inexact, hipStream_t stream) const {
-        const int64_t total = rows_out * (cols_out / 8);
-        split_planes_kernel<<<static_cast<unsigned>((total + kPlanesBlock - 1) / kPlanesBlock), kPlanesBlock, 0, stream>>>(
-            static_cast<uint16_t*>(dst), static_cast<const float*>(src), total,
-            make_fastdiv(static_cast<uint32_t>(cols_out / 8)), rows, cols, ld, ld_out(), plane, inexact);
-        TP_AMD_HIP_CHECK(hipGetLastError());
-    }
-};
-
-// A large float32 product through bfloat16 planes: rounds of 256 x 256 tiles
-// at kRoundUs a k (six pairs), and the pass over the operands, against the
-// float32 tiles' time.  The float32 MFMA caps those at 153 TFLOP/s.  us
-// there and in planes: 8192 x 4096 x 4096 1901 and 1326 NT, 1895 and 1306 NN,
-// 1882 and 1261 TN; 4096 x 4096 x 1024 247 and 177, K = 512 130 and 106; 8192
-// x 4096 x 1000 488 and 334; 5000 x 6000 x 700 342 and 237.  Relative error
-// against float64 (normal operands): 4096 x 4096 x 8192 1.6e-6 there, 5.7e-7 in
-// planes; 4096^3 1.1e-6 and 4.0e-7; K = 1024 5.7e-7 and 1.8e-7.
-// Few tiles take slices of K, added by splitk_finish_kernel: 2048 x 4096 x
-// 4096 486 us there and 375 in two slices, 2500 x 4000 x 4000 608 and 470,
-// 3500 x 1500 x 2500 232 and 192.  The float32 tiles' expected time is 8-15 %
-// under the measured one at these sizes.
-// Returns the slices' K, or 0 where the float32 tiles are faster.
-int64_t split_planes_k(const GemmArgs& p, const Planes& a, const Planes& b, int64_t cus) {
-    constexpr double kRoundUs = 0.145, kBytesPerUs = 5e6, kLaunchUs = 15.0, kFinishUs = 4.0, kPartialsPerUs = 1.25e6;
-    constexpr int64_t kMinSlice = 512;
-    if (p.batch != 1 || !a.fit() || !b.fit()) return 0;
-    const int64_t tiles = tiles_of(p, 256, 256), kp = (p.k + 63) / 64 * 64;
-    const double pass = double(a.bytes() + b.bytes()) / 6 * 10 / kBytesPerUs + kLaunchUs;
-    double least = 1.08 * plan_tiles<float>(p, cus).us;
-    int64_t best = 0;
-    for (int64_t s = 1; s <= 8 && (s == 1 || kp >= s * kMinSlice); ++s) {
-        const int64_t ks = ((kp + s - 1) / s + 63) / 64 * 64;
-        double us = double((tiles * s + cus - 1) / cus) * double(ks) * kRoundUs + pass;
-        if (s > 1) us += kFinishUs + double(p.m) * double(p.n) * double(2 * s + 1) / kPartialsPerUs;
-        if (us < least) {
-            least = us;
-            best = ks;
-        }
-    }
-    return best;
-}
-
-bool launch_split_planes(const GemmArgs& p, hipStream_t stream) {
-    int device = 0;
-    TP_AMD_HIP_CHECK(hipGetDevice(&device));
-    const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
-    const Planes a(p.lda, a_kmajor, p.m, p.k), b(p.ldb, b_kmajor, p.n, p.k);
-    const int64_t ks = split_planes_k(p, a, b, cu_count(device));
-    if (ks == 0) return false;
-    const int64_t kp = (p.k + 63) / 64 * 64, slices = (kp + ks - 1) / ks, mn = p.m * p.n;
-    Workspace ws;
-    try {
-        ws = Workspace(static_cast<size_t>(256 + a.bytes() + b.bytes() + (slices > 1 ? slices * mn * 4 : 0)), device);
-    } catch (const std::exception&) {
-        return false;  // no room for the planes: the float32 tiles need none
-    }
-    uint32_t* inexact = static_cast<uint32_t*>(ws.get());
-    char* pa = static_cast<char*>(ws.get()) + 256;
-    char* pb = pa + a.bytes();
-    clear_word_kernel<<<1, 1, 0, stream>>>(inexact);
-    TP_AMD_HIP_CHECK(hipGetLastError());
-    a.launch(p.a, pa, inexact, stream);
-    b.launch(p.b, pb, inexact, stream);
-    GemmArgs q = p;
-    q.inexact = inexact;
-    launch_config<float, 128, 128, 2, 2, false, true>(q, stream);  // runs when the word is set
-    q.a = pa;
-    q.lda = a.ld_out();
-    q.plane_a = 2 * a.plane;
-    q.b = pb;
-    q.ldb = b.ld_out();
-    q.plane_b = 2 * b.plane;
-    q.k = ks;
-    q.k_total = kp;
-    q.stride_a = a_kmajor ? ks : ks * q.lda;
-    q.stride_b = b_kmajor ? ks : ks * q.ldb;
-    if (slices > 1) {
-        q.alpha = 1.0f;
-        q.beta = 0.0f;
-        q.c = pb + b.bytes();
-        q.ldc = p.n;
-        q.stride_c = mn;
-    }
-    const dim3 grid(static_cast<unsigned>(tiles_of(p, 256, 256)), 1u, static_cast<unsigned>(slices));
-    if (a_kmajor && b_kmajor) big::gemm_big_kernel<bf16_t, true, true, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
-    else if (a_kmajor) big::gemm_big_kernel<bf16_t, true, false, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
-    else if (b_kmajor) big::gemm_big_kernel<bf16_t, false, true, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
-    else big::gemm_big_kernel<bf16_t, false, false, 2, 2, true><<<grid, 4 * kWave, 0, stream>>>(q);
-    TP_AMD_HIP_CHECK(hipGetLastError());
-    if (slices > 1) {
-        GemmArgs f = p;
-        f.inexact = inexact;
-        launch_finish<float, true>(reinterpret_cast<const float*>(pb + b.bytes()), static_cast<int>(slices), f, stream);
-    }
-    return true;
-}
-
 // A product with operands the tile kernel cannot read in place and under
 // kRepackMinMacs multiply-adds (about 160^3) takes the general kernel, which
 // needs no workspace and no extra launches.
@@ -1787,9 +1558,6 @@ void launch_typed(const GemmArgs& p, hipStream_t stream) {
     const bool copies_fit = panel_fits<T>((p.trans_a ? p.m : p.k) + 128, !p.trans_a) &&
                             panel_fits<T>((p.trans_b ? p.k : p.n) + 128, p.trans_b);
     if (in_place) {
-        if constexpr (std::is_same<T, float>::value) {
-            if (launch_split_planes(p, stream)) return;
-        }
         if (copies_fit && repack_pays<T>(p)) launch_repacked<T>(p, true, stream);
         else launch_mfma<T>(p, stream);
     } else if (copies_fit && double(p.batch) * double(p.m) * double(p.n) * double(p.k) >= kRepackMinMacs) {

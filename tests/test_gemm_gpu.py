@@ -699,13 +699,11 @@ def test_gemm_operands_at_any_element(amd, dev, orc, dtype, ta, tb, bt, m, n, k,
 @pytest.mark.parametrize("m,n,k,cin_kind", [(4096, 4096, 1024, "none"), (4090, 4081, 1001, "full"),
                                             (4090, 4081, 1001, "bias-row"), (2047, 4000, 4100, "full"),
                                             (4096, 1000, 7000, "none")],
-                         ids=["whole-tiles", "ragged-full", "ragged-bias", "slices-full", "slices"])
-def test_large_float32_product_in_planes(amd, dev, orc, ta, tb, m, n, k, cin_kind):
-    """A float32 product large enough for six products of bfloat16 planes, on
-    256 tiles of 256 x 256 or on fewer in slices of K.  Rows across the edges of tiles against float64: what
-    the planes leave out and each of the k / 16 full-size roundings are
-    under 2^-24 of a term, so the error stays under that of a sum rounded
-    term by term, 2^-24 sqrt(k) of the rows' norm."""
+                         ids=["whole-tiles", "ragged-full", "ragged-bias", "ragged-long", "wide-long"])
+def test_large_float32_product(amd, dev, orc, ta, tb, m, n, k, cin_kind):
+    """Large float32 products in the four layouts.  Rows across the edges of
+    tiles against float64: the error stays under that of a sum rounded term
+    by term, 2^-24 sqrt(k) of the rows' norm."""
     lib = amd.load()
     rng = np.random.default_rng(31)
     lead = 1 if k % 2 else 0
@@ -731,11 +729,27 @@ def test_large_float32_product_in_planes(amd, dev, orc, ta, tb, m, n, k, cin_kin
     assert error.max() <= 2.0**-24 * np.sqrt(k), error
 
 
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 1024), (2048, 4096, 4096), (256, 1024, 4096), (40, 8200, 2048)])
+@pytest.mark.parametrize("small", [1.0, 2.0**-60], ids=["ones", "2^-120"])
+def test_float32_product_of_one_term_is_rounded_once(dev, ops, m, n, k, small):
+    """A row with one non-zero element (a diagonal, selected or masked
+    operand) makes each result one product of two float32 numbers, exact in
+    float64: the result is that product rounded once, whatever the kernel
+    and the slices of K, also for products down to 2^-121."""
+    g = np.random.default_rng(35)
+    at = g.integers(0, k, m)
+    a = np.zeros((m, k), np.float32)
+    a[np.arange(m), at] = (g.uniform(0.5, 1.5, m) * small).astype(np.float32)
+    b = (g.uniform(0.5, 1.5, (k, n)) * g.choice([-small, small], (k, n))).astype(np.float32)
+    got = ops.mm(dev.from_numpy(a), dev.from_numpy(b)).numpy()
+    want = (a[np.arange(m), at].astype(np.float64)[:, None] * b[at].astype(np.float64)).astype(np.float32)
+    assert np.array_equal(got, want), f"{np.mean(got != want):.1%} of the results are not the rounded product"
+
+
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38, 1e-36, 1e-42])
-def test_large_float32_product_outside_the_planes(dev, ops, value):
-    """An element that bfloat16 planes do not hold exactly takes the whole
-    product to the float32 tiles: infinities and NaN land where IEEE
-    arithmetic puts them, and a row of such values keeps its precision."""
+def test_large_float32_product_with_extreme_values(dev, ops, value):
+    """Infinities and NaN land where IEEE arithmetic puts them, and a row of
+    very large, very small or subnormal values keeps its precision."""
     m, n, k = 4096, 4096, 1024
     rng = np.random.default_rng(34)
     a = rng.standard_normal((m, k)).astype(np.float32)
