@@ -200,8 +200,14 @@ __device__ __forceinline__ void interleave() {
 // tile in LDS: it zeroes what a packet or dword across K let in, and puts in
 // the last element where that is the low half of a load's dword and so was
 // dropped.
-template <typename T, bool KMAJOR, int R, int W, int NT, bool ODD>
+// One resource reaches 4 GiB.  With FAR (and ODD's rules) each row of a load
+// has its own, so rows may be any distance apart, at the price of a load
+// instruction a row.
+enum class Rows { kWhole, kOdd, kFar };
+
+template <typename T, bool KMAJOR, int R, int W, int NT, Rows ROWS>
 struct Panel {
+    static constexpr bool ODD = ROWS != Rows::kWhole, FAR = ROWS == Rows::kFar;
     using S = typename Elem<T>::storage;
     static constexpr int E = sizeof(S), V = 16 / E, BK = Mfma<T>::BK;
     static_assert(BK * E == 128, "a K tile is 128 bytes a row");
@@ -219,6 +225,7 @@ struct Panel {
     const char* base;
     int64_t ld_bytes, bytes;  // bytes: readable from base (M/N-major: from k = 0)
     uint32_t voff, kleft;     // kleft: K-major, elements of K from this lane's chunk of K tile 0 on
+    uint32_t coff, lead;      // FAR: the lane's offset in its row, bytes from base to the first element
     bool past_k, lost;        // the last K tile holds elements past K, lacks the last element
     uint32_t frag[kFrags];
 
@@ -241,6 +248,7 @@ struct Panel {
             lost = ODD && E == 2 && K % 2 != 0;
             const int row = lane >> 3, chunk = (lane & 7) ^ kswz(8 * wave + row);
             voff = static_cast<uint32_t>((8 * wave + row) * ld_bytes + chunk * 16);
+            coff = static_cast<uint32_t>(chunk * 16);
             kleft = static_cast<uint32_t>(K > chunk * V ? K - chunk * V : 0);
 #pragma unroll
             for (int s = 0; s < 4; ++s) frag[s] = (wbase + l32) * 128 + (((2 * s + half) ^ kswz(l32)) << 4);
@@ -252,6 +260,7 @@ struct Panel {
             lost = ODD && E == 2 && (rows - r0) % 2 != 0 && rows - r0 <= R;
             const int k = wave * kPerLoad + lane / kSlots;
             voff = static_cast<uint32_t>(k * ld_bytes + slot_of(lane % kSlots, k) * 16);
+            coff = static_cast<uint32_t>(slot_of(lane % kSlots, k) * 16);
             kleft = 0;
             if constexpr (E == 2) {
                 // transposed reads: lane p of 16-lane group g addresses row
@@ -274,7 +283,7 @@ struct Panel {
         if constexpr (!ODD) return;
         // an odd count that ends on a dword began in the middle of one
         lost = lost && ((reinterpret_cast<uintptr_t>(base) + bytes) & 2) == 0;
-        const uint32_t lead = reinterpret_cast<uintptr_t>(base) & 3;
+        lead = reinterpret_cast<uintptr_t>(base) & 3;
         base -= lead;
         voff += lead;
         bytes = (bytes + lead + 3) / 4 * 4;
@@ -304,6 +313,10 @@ struct Panel {
     // Loads of K tile kt into `tile` (this wave's share); past the last K
     // tile every load is out of range.
     __device__ __forceinline__ void issue(int kt, char* tile, int wave) const {
+        if constexpr (FAR) {
+            issue_rows(kt, tile, wave);
+            return;
+        }
         uint32_t off;
         const char* from;
         int64_t left;
@@ -327,6 +340,30 @@ struct Panel {
             // an out-of-range lane stays so: its offset only needs not to wrap
             const uint32_t at = KMAJOR ? (off == kOutOfRange ? kOutOfRange : off + i * step) : off + i * step;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lds_ptr)(tile + (i * W + wave) * 1024), 16, at, 0, 0, 0);
+        }
+    }
+
+    // The same with FAR: row by row, the lanes of one row a load.
+    __device__ __forceinline__ void issue_rows(int kt, char* tile, int wave) const {
+        constexpr int kRows = KMAJOR ? 8 : kPerLoad;
+        const int row = threadIdx.x % kWave / (kWave / kRows);
+        const int64_t k0 = static_cast<int64_t>(kt) * BK;
+        const int64_t skip = lead + k0 * (KMAJOR ? E : ld_bytes);
+        const bool in = !KMAJOR || k0 < kleft;
+#pragma unroll
+        for (int i = 0; i < kIssue; ++i) {
+#pragma unroll 1
+            for (int r = 0; r < kRows; ++r) {
+                const int64_t at = skip + static_cast<int64_t>((i * W + wave) * kRows + r) * ld_bytes;
+                const int64_t start = at & ~int64_t{3};
+                const int64_t left = bytes > start ? bytes - start : 0;
+                const uint32_t records = left < int64_t{kOutOfRange} ? static_cast<uint32_t>(left) : kOutOfRange;
+                const __amdgpu_buffer_rsrc_t res = rsrc(base + start, records);
+                const uint32_t off = in ? coff + static_cast<uint32_t>(at & 3) : kOutOfRange;
+                if (row == r) {
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lds_ptr)(tile + (i * W + wave) * 1024), 16, off, 0, 0, 0);
+                }
+            }
         }
     }
 
@@ -372,15 +409,16 @@ struct Panel {
 // BLOCKS is how many blocks a CU holds (LDS and registers).
 // ODD (see Panel) is a variant of its own: its test for the last K tile in
 // the loop costs the others 3-8 % (float32 256 x 1024 x 4096 25.3 -> 27.4 us).
-template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
+template <typename T, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, Rows ROWS>
 __global__ __launch_bounds__(4 * kWave, BLOCKS) void gemm_tile_kernel(GemmArgs p) {
     using S = typename Elem<T>::storage;
     constexpr int WM = BM >= 64 ? 2 : 1, WN = 4 / WM, W = WM * WN;
     constexpr int BK = Mfma<T>::BK;
     constexpr int kWaveM = BM / WM, kWaveN = BN / WN;
     constexpr int TM = kWaveM / 32, TN = kWaveN / 32;
-    using PA = Panel<T, A_KMAJOR, BM, W, TM, ODD>;
-    using PB = Panel<T, B_KMAJOR, BN, W, TN, ODD>;
+    using PA = Panel<T, A_KMAJOR, BM, W, TM, ROWS>;
+    using PB = Panel<T, B_KMAJOR, BN, W, TN, ROWS>;
+    constexpr bool ODD = PA::ODD;
     constexpr int ATILE = BM * 128, STAGE = (BM + BN) * 128;
     // An object a stage, so the compiler can tell the ones being filled from
     // the one being read and leaves the loads in flight.
@@ -1067,23 +1105,24 @@ void launch(const GemmArgs& p, hipStream_t stream) {
 
 }  // namespace smallk
 
-// An operand the tile kernel reads in place: rows that do not overlap (the
-// panel's bound is the end of its last row) and a panel (a tile's rows of K,
-// or a K tile of rows) under 4 GiB, the reach of its resource.
+// Whether an operand's panel (a tile's rows of K, or a K tile of rows) lies
+// under 4 GiB, the reach of one buffer resource.
 template <typename T>
-bool panel_fits(int64_t ld, bool kmajor) {
+bool panel_near(int64_t ld, bool kmajor) {
     constexpr int64_t E = sizeof(typename Elem<T>::storage);
-    const int64_t rows = !kmajor ? Mfma<T>::BK : E == 2 ? 256 : 128;  // the tallest tile, or a K tile
-    return ld >= 0 && ld < ((int64_t{1} << 32) - 4096) / (rows * E);
+    const int64_t rows = kmajor ? 128 : Mfma<T>::BK;  // the tallest tile, or a K tile
+    return ld < ((int64_t{1} << 32) - 4096) / (rows * E);
 }
 
 template <typename T>
-bool operand_ok(int64_t ld, bool kmajor, int64_t mn, int64_t k) {
-    return ((kmajor ? mn : k) == 1 || ld >= (kmajor ? k : mn)) && panel_fits<T>(ld, kmajor);
+bool rows_far(const GemmArgs& p) {
+    return !panel_near<T>(p.lda, !p.trans_a) || !panel_near<T>(p.ldb, p.trans_b);
 }
 
+// The grid's limit, and the panels' 32-bit K (one product of a longer K is
+// always split).
 bool tiles_fit(const GemmArgs& p) {
-    return (p.m + 63) / 64 * ((p.n + 63) / 64) < (int64_t(1) << 31) && p.k < (int64_t(1) << 31);
+    return (p.m + 63) / 64 * ((p.n + 63) / 64) < (int64_t(1) << 31) && (p.k < (int64_t(1) << 32) || p.batch == 1);
 }
 
 // Whole dwords everywhere and whole packets along K: the tile kernel without
@@ -1095,20 +1134,20 @@ bool whole_dwords(const void* x, int64_t ld, int64_t stride, bool kmajor, int64_
     return E == 4 || (reinterpret_cast<uintptr_t>(x) % 4 == 0 && ld % 2 == 0 && stride % 2 == 0 && (kmajor || mn % 2 == 0));
 }
 
-template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, bool ODD>
+template <typename T, int BM, int BN, int STAGES, int BLOCKS, bool F32OUT, Rows ROWS>
 void launch_chunk(const GemmArgs& p, hipStream_t stream) {
     constexpr int THREADS = 4 * kWave;
     const int64_t tiles = ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
     const dim3 grid(static_cast<unsigned>(tiles), 1u, static_cast<unsigned>(p.batch));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     if (a_kmajor && b_kmajor) {
-        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, true, BM, BN, STAGES, BLOCKS, F32OUT, ROWS><<<grid, THREADS, 0, stream>>>(p);
     } else if (a_kmajor) {
-        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, true, false, BM, BN, STAGES, BLOCKS, F32OUT, ROWS><<<grid, THREADS, 0, stream>>>(p);
     } else if (b_kmajor) {
-        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, true, BM, BN, STAGES, BLOCKS, F32OUT, ROWS><<<grid, THREADS, 0, stream>>>(p);
     } else {
-        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ODD><<<grid, THREADS, 0, stream>>>(p);
+        gemm_tile_kernel<T, false, false, BM, BN, STAGES, BLOCKS, F32OUT, ROWS><<<grid, THREADS, 0, stream>>>(p);
     }
     TP_AMD_HIP_CHECK(hipGetLastError());
 }
@@ -1127,11 +1166,14 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
         if (whole.cin != nullptr) p.cin = static_cast<const S*>(whole.cin) + b0 * whole.cin_stride_b;
         if (F32OUT) p.k_total = whole.k_total - b0 * whole.k;
         const int64_t k = F32OUT ? p.k_total : p.k;
-        if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
-            whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
-            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, false>(p, stream);
+        if (rows_far<T>(p)) {
+            if constexpr (BM == 64 && BN == 64) launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kFar>(p, stream);
+            else TP_AMD_CHECK(false, "a tile that cannot take rows this far apart");
+        } else if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
+                   whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kWhole>(p, stream);
         } else {
-            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, true>(p, stream);
+            launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kOdd>(p, stream);
         }
     }
 }
@@ -1289,6 +1331,9 @@ TilePlan plan_small_batch(const GemmArgs& p, int64_t cus) {
 template <typename T>
 TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
     constexpr int64_t BK = Mfma<T>::BK;
+    // One tile shape is built for rows this far apart (128 x 128 x 8.5e6
+    // float32 5.5 ms, bfloat16 1.3 ms; on the general kernel 1.8 s).
+    if (rows_far<T>(p)) return split_k(Tile::k64, p, 3 * cus / tiles_of(p, 64, 64), 1024, BK);
     const int64_t thin = std::min(p.m, p.n);
     const int64_t t128 = tiles_of(p, 128, 128), t64 = tiles_of(p, 64, 64);
     if constexpr (std::is_same<T, float>::value) {
@@ -1508,19 +1553,18 @@ bool repack_pays(const GemmArgs& p) {
                static_cast<double>(p.k) > copies;
 }
 
-// A product on copies of its operands: of those the tile kernel cannot read
-// in place (rows that overlap, or too far apart for its panel), and of those
-// that are not aligned packets where that pays.
+// A product on copies of its operands that are not aligned packets, where
+// that pays.
 template <typename T>
-void launch_repacked(const GemmArgs& p, bool pays, hipStream_t stream) {
+void launch_repacked(const GemmArgs& p, hipStream_t stream) {
     int device = 0;
     TP_AMD_HIP_CHECK(hipGetDevice(&device));
     const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
     // A K that is no whole number of packets is padded in both copies.
-    const bool pad = pays && p.k % Mfma<T>::V != 0;
+    const bool pad = p.k % Mfma<T>::V != 0;
     const int64_t kp = pad ? (p.k + Mfma<T>::BK - 1) / Mfma<T>::BK * Mfma<T>::BK : p.k;
-    const bool fix_a = !operand_ok<T>(p.lda, a_kmajor, p.m, p.k) || pad || (pays && !packets_aligned<T>(p.a, p.lda, p.stride_a));
-    const bool fix_b = !operand_ok<T>(p.ldb, b_kmajor, p.n, p.k) || pad || (pays && !packets_aligned<T>(p.b, p.ldb, p.stride_b));
+    const bool fix_a = pad || !packets_aligned<T>(p.a, p.lda, p.stride_a);
+    const bool fix_b = pad || !packets_aligned<T>(p.b, p.ldb, p.stride_b);
     const Repack<T> a(p.lda, p.stride_a, a_kmajor, p.batch, p.m, p.k, kp), b(p.ldb, p.stride_b, b_kmajor, p.batch, p.n, p.k, kp);
     const size_t off_b = fix_a ? (a.elems() * a.E + 255) / 256 * 256 : 0;
     Workspace ws(off_b + (fix_b ? b.elems() * b.E : 0), device);
@@ -1543,28 +1587,11 @@ void launch_repacked(const GemmArgs& p, bool pays, hipStream_t stream) {
     if (!launch_gemm_thin(DtypeOf<T>::value, q, stream)) launch_mfma<T>(q, stream);
 }
 
-// A product with operands the tile kernel cannot read in place and under
-// kRepackMinMacs multiply-adds (about 160^3) takes the general kernel, which
-// needs no workspace and no extra launches.
-constexpr double kRepackMinMacs = double(int64_t(1) << 22);
-
 template <typename T>
 void launch_typed(const GemmArgs& p, hipStream_t stream) {
-    if (p.k <= 0 || !tiles_fit(p)) {
-        launch_gemm_general<T>(p, stream);
-        return;
-    }
-    const bool in_place = operand_ok<T>(p.lda, !p.trans_a, p.m, p.k) && operand_ok<T>(p.ldb, p.trans_b, p.n, p.k);
-    const bool copies_fit = panel_fits<T>((p.trans_a ? p.m : p.k) + 128, !p.trans_a) &&
-                            panel_fits<T>((p.trans_b ? p.k : p.n) + 128, p.trans_b);
-    if (in_place) {
-        if (copies_fit && repack_pays<T>(p)) launch_repacked<T>(p, true, stream);
-        else launch_mfma<T>(p, stream);
-    } else if (copies_fit && double(p.batch) * double(p.m) * double(p.n) * double(p.k) >= kRepackMinMacs) {
-        launch_repacked<T>(p, false, stream);
-    } else {
-        launch_gemm_general<T>(p, stream);
-    }
+    if (p.k <= 0 || !tiles_fit(p)) launch_gemm_general<T>(p, stream);
+    else if (repack_pays<T>(p)) launch_repacked<T>(p, stream);
+    else launch_mfma<T>(p, stream);
 }
 
 }  // namespace

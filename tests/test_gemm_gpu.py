@@ -330,10 +330,9 @@ def test_gemm_abi_padded_batched(amd, dev, orc, dtype, ta, tb, bt, m, n, k):
                                                 (4, 300, 270, 255, 5, True)],
                          ids=["odd-K", "odd-ld", "odd-K-batch-broadcast"])
 def test_gemm_abi_repacked_operands(amd, dev, orc, dtype, ta, tb, bt, m, n, k, pad, bcast):
-    """Products whose operands the matrix-core kernels cannot read in place
-    (odd K, odd leading dimensions, NaN in the padding) are repacked into
-    aligned K-major copies, K padded with zeros: alpha = 0.5, beta = 2 with
-    a full Cin, and in the batched case a B broadcast over the batch
+    """Operands that are not whole packets (odd K, odd leading dimensions, NaN
+    in the padding), read where they lie at these sizes: alpha = 0.5, beta =
+    2 with a full Cin, and in the batched case a B broadcast over the batch
     (stride 0)."""
     lib = amd.load()
     alpha, beta = 0.5, 2.0
@@ -692,6 +691,74 @@ def test_gemm_operands_at_any_element(amd, dev, orc, dtype, ta, tb, bt, m, n, k,
     got = out.numpy()[:, rows]
     assert not np.isnan(orc.to_float(got, dtype)).any(), "an element outside the operands reached the product"
     check(orc, got, want, dtype, f"odd gemm {bt}x{m}x{n}x{k} ta={ta} tb={tb}")
+
+
+def _spread(dev, ops, orc, shape, ld, lead, dtype, seed):
+    """A device matrix whose rows lie ``ld`` elements apart, ``lead`` elements
+    into its storage, with NaN in the gaps; and its values."""
+    x = sample(orc, shape, dtype, seed, 0.25)
+    store = dev.empty((lead + (shape[0] - 1) * ld + shape[1],), dtype=dtype)
+    ops.fill_(store, float("nan"))
+    rows = store._view(shape, (ld, 1), lead)
+    ops.copy_(rows, dev.from_numpy(x, dtype=dtype))
+    return store, rows, orc.to_float(x, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
+                         ids=["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("m,n,k,odd", [(130, 66, 136, 0), (67, 129, 71, 1)], ids=["even", "odd"])
+def test_gemm_rows_far_apart(amd, dev, ops, orc, dtype, ta, tb, m, n, k, odd):
+    """Operands whose rows are too far apart for one 4 GiB buffer resource a
+    panel (from 2^23 elements for rows of K, 2^25 for rows of M or N), with
+    odd ends and a row longer than 512 MiB among them; alpha, and a bias."""
+    lib = amd.load()
+    e = 4 if dtype == F32 else 2
+    k_apart, mn_apart = (1 << 23) + 8 + odd, (1 << 25) + 8 + odd
+    if ta == tb:  # one of them past 2^29 bytes
+        mn_apart = max(mn_apart, (1 << 29) // e + 8 + odd) if e == 2 else mn_apart
+    lda, ldb = mn_apart if ta else k_apart, k_apart if tb else mn_apart
+    sa, da, A = _spread(dev, ops, orc, (k, m) if ta else (m, k), lda, odd, dtype, 71)
+    sb, db, B = _spread(dev, ops, orc, (n, k) if tb else (k, n), ldb, odd, dtype, 72)
+    bias = sample(orc, (n,), dtype, 73)
+    dbias = dev.from_numpy(bias, dtype=dtype)
+    out = dev.empty((m, n), dtype=dtype)
+    st = lib.tp_amd_launch_gemm(0, dtype, 1, m, n, k, 0.5, da.data_ptr, lda, 0, int(ta), db.data_ptr, ldb, 0, int(tb),
+                                2.0, dbias.data_ptr, 0, 1, 0, out.data_ptr, n, 0)
+    assert st == 0, lib.tp_mlu_last_error()
+    got = out.numpy()
+    assert not np.isnan(orc.to_float(got, dtype)).any(), "a gap reached the product"
+    want = 0.5 * ((A.T if ta else A).astype(np.float64) @ (B.T if tb else B).astype(np.float64))
+    check(orc, got, want + 2.0 * orc.to_float(bias, dtype), dtype, f"far gemm {m}x{n}x{k} ta={ta} tb={tb}")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False)], ids=["NT", "NN", "TN"])
+def test_gemm_of_a_very_long_k(amd, dev, ops, orc, dtype, ta, tb):
+    """K past 2^23, where rows of K leave the reach of one resource: operands
+    of -1, 0 and 1 with a period of 1000 in K make every sum an integer under
+    2^24, so the product is exact in any order."""
+    m, n, period, reps, tail = 70, 66, 1000, 8400, 37
+    k = period * reps + tail
+    g = np.random.default_rng(74)
+    a0, b0 = (g.integers(-1, 2, (rows, period)).astype(np.float32) for rows in (m, n))
+
+    def build(x0, kmajor):
+        x0 = orc.from_float(x0, dtype)
+        rows = x0.shape[0]
+        x = dev.empty((rows, k) if kmajor else (k, rows), dtype=dtype)
+        step = 1 if kmajor else rows
+        src = dev.from_numpy(x0, dtype=dtype)
+        ops.copy_(x._view((rows, reps, period), (k if kmajor else 1, period * step, step)),
+                  src._view((rows, reps, period), (period, 0, 1)))
+        ops.copy_(x._view((rows, tail), (k if kmajor else 1, step), period * reps * step),
+                  src._view((rows, tail), (period, 1)))
+        return x if kmajor else x.t()
+
+    got = ops.mm(build(a0, not ta), build(b0, tb).t()).numpy()
+    want = reps * (a0 @ b0.T) + a0[:, :tail] @ b0[:, :tail].T
+    assert np.abs(want).max() < 2**24
+    assert np.array_equal(got, orc.from_float(want.astype(np.float32), dtype))
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
