@@ -461,11 +461,17 @@ __global__ __launch_bounds__(16 * kWave) void softmax_backward_stream_kernel(
     }
 }
 
-// (max, sum) pairs: the sum is relative to the max.
-__device__ __forceinline__ void online_merge(float& m, float& s, float m2, float s2) {
-    const float mn = fmaxf(m, m2);
-    if (mn == -INFINITY) return;  // both empty
-    s = s * exp_fast(m - mn) + s2 * exp_fast(m2 - mn);
+// The larger of a and b, NaN if either is (fmaxf returns the other operand
+// for a NaN, which would let a thread whose only numbers are NaN and -inf
+// look empty and be skipped).
+__device__ __forceinline__ float max_keep_nan(float a, float b) { return (a > b || a != a) ? a : b; }
+
+// (m, s) <- (m, s) merged with (m2, s2), each s a sum of exp(v - m).  A NaN
+// maximum makes the merged sum NaN, so the line's outputs become NaN.
+__device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
+    const float mn = max_keep_nan(m, m2);
+    if (mn == -INFINITY) return;
+    s = (m == -INFINITY ? 0.0f : s * exp_fast(m - mn)) + (m2 == -INFINITY ? 0.0f : s2 * exp_fast(m2 - mn));
     m = mn;
 }
 
@@ -474,7 +480,7 @@ __device__ __forceinline__ void block_merge(float& m, float& s) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
         const float m2 = wave_shfl_xor(m, o), s2 = wave_shfl_xor(s, o);
-        online_merge(m, s, m2, s2);
+        lse_merge(m, s, m2, s2);
     }
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (lane == 0) {
@@ -485,7 +491,7 @@ __device__ __forceinline__ void block_merge(float& m, float& s) {
     m = sm[0];
     s = ss[0];
 #pragma unroll
-    for (int w = 1; w < kBlock / kWave; ++w) online_merge(m, s, sm[w], ss[w]);
+    for (int w = 1; w < kBlock / kWave; ++w) lse_merge(m, s, sm[w], ss[w]);
 }
 
 // Rows too long to hold: a 256-thread block per row.  Pass 1 keeps a running
@@ -514,9 +520,9 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_long_kernel(
             unpack<T>(raw[u], v);
             float pm = v[0];
 #pragma unroll
-            for (int j = 1; j < N; ++j) pm = fmaxf(pm, v[j]);
-            const float mn = fmaxf(m, pm);
-            if (mn == -INFINITY) continue;
+            for (int j = 1; j < N; ++j) pm = max_keep_nan(pm, v[j]);
+            const float mn = max_keep_nan(m, pm);
+            if (mn == -INFINITY) continue;  // only -inf so far
             float t = 0.0f;
 #pragma unroll
             for (int j = 0; j < N; ++j) t += exp_fast(v[j] - mn);
@@ -527,7 +533,7 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_long_kernel(
     const bool tail = ANY && threadIdx.x < D - npk * N;  // one of the row's last D % N elements
     const float tv = tail ? Elem<T>::load(xr[npk * N + threadIdx.x]) : -INFINITY;
     if (ANY && tv != -INFINITY) {
-        const float mn = fmaxf(m, tv);
+        const float mn = max_keep_nan(m, tv);
         s = s * exp_fast(m - mn) + exp_fast(tv - mn);
         m = mn;
     }
@@ -787,20 +793,6 @@ __device__ __forceinline__ ColBlock col_block(int64_t tiles, int64_t slices, int
     cb.d0 = cb.sl * dslice;
     cb.d1 = cb.d0 + dslice < D ? cb.d0 + dslice : D;
     return cb;
-}
-
-// The larger of a and b, NaN if either is (fmaxf returns the other operand
-// for a NaN, which would let a column whose only numbers are NaN and -inf
-// look empty and be skipped).
-__device__ __forceinline__ float max_keep_nan(float a, float b) { return (a > b || a != a) ? a : b; }
-
-// (m, s) <- (m, s) merged with (m2, s2), each s a sum of exp(v - m).  A NaN
-// maximum makes the merged sum NaN, so the column's outputs become NaN.
-__device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
-    const float mn = max_keep_nan(m, m2);
-    if (mn == -INFINITY) return;
-    s = (m == -INFINITY ? 0.0f : s * exp_fast(m - mn)) + (m2 == -INFINITY ? 0.0f : s2 * exp_fast(m2 - mn));
-    m = mn;
 }
 
 template <typename T, int MODE>

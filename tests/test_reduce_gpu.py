@@ -426,6 +426,30 @@ def test_softmax_nan_over_a_leading_axis(dev, ops, orc, dtype, shape, dim):
                                 yh, g, outer, size, inner, f"backward log={log}")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("D", [333, 4099, 20000, 50257, 51203, 65539, 102405, 204800])
+def test_softmax_nan_in_a_row(dev, ops, orc, dtype, D):
+    """A NaN makes its whole row NaN in every row kernel, also where a
+    thread's first packet holds nothing but NaN, or NaN and masked (-inf)
+    elements, or stands in the row's last elements; rows without one are
+    finite, all-masked ones NaN as on the host."""
+    a = sample(orc, (7, D), dtype, 25)
+    nan, ninf = orc.from_float(np.array([np.nan, -np.inf], np.float32), dtype)
+    a[1, :8] = nan
+    a[2, :8], a[2, 3] = ninf, nan
+    a[3], a[3, D // 2], a[3, 9] = ninf, nan, a[0, 0]
+    a[4], a[4, D - 1], a[4, 0] = ninf, nan, a[0, 0]
+    a[5, D - 3] = nan
+    a[6] = ninf
+    for log in (False, True):
+        y = (ops.log_softmax if log else ops.softmax)(dev.from_numpy(a, dtype=dtype), -1).numpy()
+        got = np.isnan(as_float(y, dtype))
+        assert not got[0].any()
+        assert got[1:6].all(), f"log={log}: NaN share by row {got.mean(1)}"
+        want = orc.softmax(log, dtype, a, 7, D, 1)
+        assert np.array_equal(got, np.isnan(as_float(want, dtype)))
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("shape,dim", [((64, 1000), -1), ((40, 16400), -1), ((6, 70000), -1),
                                        ((300, 130), 0), ((5, 300, 70), 1)],
