@@ -1311,16 +1311,20 @@ TilePlan split_k(Tile tile, const GemmArgs& p, int64_t most, int64_t min_k, int6
 //     15.1 (22.1); x W 8 x 11008 x 4096 19.6 (26.3).  Unsplit with two
 //     rounds of tiles (a vocabulary) 64 x 128 tiles halve the blocks.
 //   * float32, 17 to 32 rows: 32 x 128 tiles (a taller tile's padding rows
-//     cost MFMA time there), one block a CU: 20 x 11008 x 4096 47.0 (54.6),
-//     20 x 4096 x 11008 45.3 (56.7).
+//     cost MFMA time there), one block a CU in slices of at least 128: 20 x
+//     11008 x 4096 47.0 (54.6), 20 x 4096 x 11008 45.3 (56.7), 24 x 4096 x
+//     1024 11.5 (13.9).  As many columns stay on the thin kernel: 4096 x 24 x
+//     4096 TN 25.9 there, 27 on 64 x 64 tiles.
 //   * float32, 33 to 64: 64 x 64 tiles, up to three blocks a CU: 48 x 4096 x
-//     11008 58.5 (102), 48 x 4096 x 4096 27.3 (40.2).
+//     11008 58.5 (102), 48 x 4096 x 4096 27.3 (40.2); a K too short for
+//     that, by plan_tiles' model: 48 x 4096 x 1024 13.0 (21.0), 33 x 12352 x
+//     512 13.1 (29.1).
 template <typename T>
 TilePlan plan_small_batch(const GemmArgs& p, int64_t cus) {
     constexpr int64_t BK = Mfma<T>::BK;
     const int64_t t64 = tiles_of(p, 64, 64);
     if constexpr (std::is_same<T, float>::value) {
-        if (p.m <= 32 && p.n > 64) return split_k(Tile::k32x128, p, cus / tiles_of(p, 32, 128), 512, BK);
+        if (p.m <= 32 && p.n > 64) return split_k(Tile::k32x128, p, cus / tiles_of(p, 32, 128), 128, BK);
         return split_k(Tile::k64, p, 3 * cus / t64, 1024, BK);
     } else {
         if (t64 >= 2 * cus && p.m <= 64) return TilePlan{Tile::k64x128};
@@ -1331,15 +1335,15 @@ TilePlan plan_small_batch(const GemmArgs& p, int64_t cus) {
 template <typename T>
 TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
     constexpr int64_t BK = Mfma<T>::BK;
-    // One tile shape is built for rows this far apart (128 x 128 x 8.5e6
-    // float32 5.5 ms, bfloat16 1.3 ms; on the general kernel 1.8 s).
-    if (rows_far<T>(p)) return split_k(Tile::k64, p, 3 * cus / tiles_of(p, 64, 64), 1024, BK);
     const int64_t thin = std::min(p.m, p.n);
     const int64_t t128 = tiles_of(p, 128, 128), t64 = tiles_of(p, 64, 64);
+    // One tile shape is built for rows this far apart (128 x 128 x 8.5e6
+    // float32 5.5 ms, bfloat16 1.3 ms; on the general kernel 1.8 s).
+    if (rows_far<T>(p)) return split_k(Tile::k64, p, 3 * cus / t64, 1024, BK);
     if constexpr (std::is_same<T, float>::value) {
         if (p.batch == 1 && thin > 16 && thin <= 64) {
             const TilePlan plan = plan_small_batch<T>(p, cus);
-            if (plan.slices > 1) return plan;
+            if (plan.slices > 1 && (plan.tile != Tile::k64 || 2 * t64 * plan.slices >= cus)) return plan;
         }
         // MFMAs of 64 cycles leave LDS and L2 idle, so a CU is busy as long
         // as it has a tile, one of 64 x 64 at 93 % of the larger ones' rate
@@ -1351,16 +1355,29 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
         // 4096 x 1024 66 and 22; 700 x 900 x 5000 89 whole, 63 in three
         // slices; 1500 x 1500 x 4000 184 and 157; 256 x 1024 x 4096 70, 26 in
         // four; 256^3 7.5, 8.7 in two.
-        constexpr double kTileUs = 0.0137, kFinishUs = 4.0, kPartialsPerUs = 1.25e6;
+        constexpr double kTileUs = 0.0137, kFinishUs = 2.2, kPartialsPerUs = 1.25e6;
         const double rounds128 = double((t128 + cus - 1) / cus);
         TilePlan best{Tile::k128};
         double least = rounds128 * double(p.k) * kTileUs * 4 * 0.93;
-        for (int64_t slices = 1; slices <= (p.batch == 1 ? 16 : 1); ++slices) {
-            const TilePlan plan = slices == 1 ? TilePlan{Tile::k64} : split_k(Tile::k64, p, slices, 192, BK);
-            if (plan.slices != slices) continue;
-            const double rounds = double((t64 * slices + cus - 1) / cus);
-            double us = rounds * double(slices == 1 ? p.k : plan.ks) * kTileUs;
-            if (slices > 1) us += kFinishUs + double(p.m) * double(p.n) * double(2 * slices + 1) / kPartialsPerUs;
+        // Few tiles and a long K take more slices, up to two blocks a CU; each
+        // past 16 adds its loads to the finish's chain.  From K = 16384 on the
+        // operands stream from memory, and one block a CU waits for its loads
+        // (a k takes twice as long): 128 x 128 x 65536 57 us in 16 slices,
+        // 36 in 128; x 2^20 2047 and 418; 256 x 256 x 65536 114 in 16, 78 in 32;
+        // 512 x 512 x 16384 110 in 4, 80 in 8.
+        constexpr double kSliceUs = 0.08;
+        constexpr int64_t kMinSlice = 64;
+        const double wait = p.k >= 16384 ? 1.9 : 1.0;
+        // 1 to 16, then 24, 32, 48, 64, ...
+        auto next = [](int64_t s) { return s + (s < 16 ? 1 : (s & (s - 1)) == 0 ? s / 2 : s / 3); };
+        for (int64_t slices = 1; slices <= 16 || t64 * slices <= 2 * cus; slices = next(slices)) {
+            if (slices > 1 && (p.batch != 1 || p.k < slices * kMinSlice)) break;
+            const TilePlan plan = split_k(Tile::k64, p, slices, kMinSlice, BK);
+            const int64_t blocks = t64 * plan.slices;
+            double us = double((blocks + cus - 1) / cus) * double(plan.slices == 1 ? p.k : plan.ks) * kTileUs;
+            if (blocks <= cus) us *= wait;
+            if (plan.slices > 16) us += kSliceUs * double(plan.slices - 16);
+            if (plan.slices > 1) us += kFinishUs + double(p.m) * double(p.n) * double(2 * plan.slices + 1) / kPartialsPerUs;
             if (us < least) {
                 least = us;
                 best = plan;
@@ -1600,7 +1617,10 @@ bool tiles_take_thin(int dtype, const GemmArgs& p, int device) {
     const int64_t cus = cu_count(device), thin = std::min(p.m, p.n);
     const int64_t t64 = tiles_of(p, 64, 64);
     if (p.batch > 1) return thin > 32 && t64 >= cus;
-    if (dtype == TP_AMD_FLOAT32) return thin > 16 && plan_small_batch<float>(p, cus).slices > 1;
+    if (dtype == TP_AMD_FLOAT32) {
+        if (thin > 32) return true;
+        return thin > 16 && p.m <= 32 && p.n > 64 && plan_small_batch<float>(p, cus).slices > 1;
+    }
     const TilePlan plan = plan_small_batch<bf16_t>(p, cus);
     const int64_t blocks = (plan.tile == Tile::k64 ? t64 : tiles_of(p, 64, 128)) * plan.slices;
     if (thin > 32) return blocks >= cus / 4;
