@@ -1311,10 +1311,13 @@ TilePlan split_k(Tile tile, const GemmArgs& p, int64_t most, int64_t min_k, int6
 //     15.1 (22.1); x W 8 x 11008 x 4096 19.6 (26.3).  Unsplit with two
 //     rounds of tiles (a vocabulary) 64 x 128 tiles halve the blocks.
 //   * float32, 17 to 32 rows: 32 x 128 tiles (a taller tile's padding rows
-//     cost MFMA time there), one block a CU in slices of at least 128: 20 x
-//     11008 x 4096 47.0 (54.6), 20 x 4096 x 11008 45.3 (56.7), 24 x 4096 x
-//     1024 11.5 (13.9).  As many columns stay on the thin kernel: 4096 x 24 x
-//     4096 TN 25.9 there, 27 on 64 x 64 tiles.
+//     cost MFMA time there), one block a CU in slices of at least 512, or 128
+//     for the first 16 (the finish adds each in turn): 20 x 11008 x 4096 47.0
+//     (54.6), 20 x 4096 x 11008 45.3 (56.7), 24 x 4096 x
+//     1024 11.5 (13.9).  As many columns take plan_tiles' slices of 64 x 64
+//     tiles up to 48 MiB of the wide operand (1024 x 24 x 4736 14.8, thin 20
+//     to 27; 4096 x 24 x 4096 27.5, thin 26 to 31; 14848 x 24 x 15040 264, thin
+//     191 to 252).
 //   * float32, 33 to 64: 64 x 64 tiles, up to three blocks a CU: 48 x 4096 x
 //     11008 58.5 (102), 48 x 4096 x 4096 27.3 (40.2); a K too short for
 //     that, by plan_tiles' model: 48 x 4096 x 1024 13.0 (21.0), 33 x 12352 x
@@ -1324,7 +1327,10 @@ TilePlan plan_small_batch(const GemmArgs& p, int64_t cus) {
     constexpr int64_t BK = Mfma<T>::BK;
     const int64_t t64 = tiles_of(p, 64, 64);
     if constexpr (std::is_same<T, float>::value) {
-        if (p.m <= 32 && p.n > 64) return split_k(Tile::k32x128, p, cus / tiles_of(p, 32, 128), 128, BK);
+        if (p.m <= 32 && p.n > 64) {
+            const int64_t most = std::max(p.k / 512, p.k < 512 ? 0 : std::min<int64_t>(16, p.k / 128));
+            return split_k(Tile::k32x128, p, std::min(cus / tiles_of(p, 32, 128), most), 128, BK);
+        }
         return split_k(Tile::k64, p, 3 * cus / t64, 1024, BK);
     } else {
         if (t64 >= 2 * cus && p.m <= 64) return TilePlan{Tile::k64x128};
@@ -1343,19 +1349,20 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
     if constexpr (std::is_same<T, float>::value) {
         if (p.batch == 1 && thin > 16 && thin <= 64) {
             const TilePlan plan = plan_small_batch<T>(p, cus);
-            if (plan.slices > 1 && (plan.tile != Tile::k64 || 2 * t64 * plan.slices >= cus)) return plan;
+            if (plan.slices > 1 && (plan.tile == Tile::k32x128 || (thin > 32 && 2 * t64 * plan.slices >= cus))) return plan;
         }
         // MFMAs of 64 cycles leave LDS and L2 idle, so a CU is busy as long
         // as it has a tile, one of 64 x 64 at 93 % of the larger ones' rate
         // (8192 x 4096 x 4096 2010 against 1886 us), and the time is the
         // rounds of tiles times their K: kTileUs a k of a 64 x 64 tile, by
         // the instruction's rate.  Slices of K even out the last round for
-        // the price of the finish, a launch and a pass over the partials.
+        // the price of the finish: 2.2 us, a launch that a program bound by
+        // its host calls pays too, and a pass over the partials.
         // 2048 x 3000 x 1000 125 us on 128 x 128 tiles, 102 on 64 x 64; 256 x
         // 4096 x 1024 66 and 22; 700 x 900 x 5000 89 whole, 63 in three
         // slices; 1500 x 1500 x 4000 184 and 157; 256 x 1024 x 4096 70, 26 in
-        // four; 256^3 7.5, 8.7 in two.
-        constexpr double kTileUs = 0.0137, kFinishUs = 2.2, kPartialsPerUs = 1.25e6;
+        // four; 33 x 192 x 512 11.5, 7.8 in eight; 256^3 7.5, 8.7 in two.
+        constexpr double kTileUs = 0.0137, kFinishUs = 4.0, kPartialsPerUs = 1.25e6;
         const double rounds128 = double((t128 + cus - 1) / cus);
         TilePlan best{Tile::k128};
         double least = rounds128 * double(p.k) * kTileUs * 4 * 0.93;
@@ -1366,13 +1373,13 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
         // 36 in 128; x 2^20 2047 and 418; 256 x 256 x 65536 114 in 16, 78 in 32;
         // 512 x 512 x 16384 110 in 4, 80 in 8.
         constexpr double kSliceUs = 0.08;
-        constexpr int64_t kMinSlice = 64;
+        const int64_t min_slice = p.k >= 512 ? 64 : 192;
         const double wait = p.k >= 16384 ? 1.9 : 1.0;
         // 1 to 16, then 24, 32, 48, 64, ...
         auto next = [](int64_t s) { return s + (s < 16 ? 1 : (s & (s - 1)) == 0 ? s / 2 : s / 3); };
         for (int64_t slices = 1; slices <= 16 || t64 * slices <= 2 * cus; slices = next(slices)) {
-            if (slices > 1 && (p.batch != 1 || p.k < slices * kMinSlice)) break;
-            const TilePlan plan = split_k(Tile::k64, p, slices, kMinSlice, BK);
+            if (slices > 1 && (p.batch != 1 || p.k < slices * min_slice)) break;
+            const TilePlan plan = split_k(Tile::k64, p, slices, min_slice, BK);
             const int64_t blocks = t64 * plan.slices;
             double us = double((blocks + cus - 1) / cus) * double(plan.slices == 1 ? p.k : plan.ks) * kTileUs;
             if (blocks <= cus) us *= wait;
@@ -1619,7 +1626,9 @@ bool tiles_take_thin(int dtype, const GemmArgs& p, int device) {
     if (p.batch > 1) return thin > 32 && t64 >= cus;
     if (dtype == TP_AMD_FLOAT32) {
         if (thin > 32) return true;
-        return thin > 16 && p.m <= 32 && p.n > 64 && plan_small_batch<float>(p, cus).slices > 1;
+        if (thin <= 16) return false;
+        if (p.m <= 32 && p.n > 64) return plan_small_batch<float>(p, cus).slices > 1;
+        return std::max(p.m, p.n) * p.k * 4 < (int64_t{48} << 20);
     }
     const TilePlan plan = plan_small_batch<bf16_t>(p, cus);
     const int64_t blocks = (plan.tile == Tile::k64 ? t64 : tiles_of(p, 64, 128)) * plan.slices;
