@@ -1167,7 +1167,8 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
         if (F32OUT) p.k_total = whole.k_total - b0 * whole.k;
         const int64_t k = F32OUT ? p.k_total : p.k;
         if (rows_far<T>(p)) {
-            if constexpr (BM == 64 && BN == 64) launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kFar>(p, stream);
+            constexpr bool kSlices128 = F32OUT && BM == 128 && STAGES == 3;
+            if constexpr (BM == 64 && BN == 64 || kSlices128) launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kFar>(p, stream);
             else TP_AMD_CHECK(false, "a tile that cannot take rows this far apart");
         } else if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
                    whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
@@ -1343,9 +1344,15 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
     constexpr int64_t BK = Mfma<T>::BK;
     const int64_t thin = std::min(p.m, p.n);
     const int64_t t128 = tiles_of(p, 128, 128), t64 = tiles_of(p, 64, 64);
-    // One tile shape is built for rows this far apart (128 x 128 x 8.5e6
-    // float32 5.5 ms, bfloat16 1.3 ms; on the general kernel 1.8 s).
-    if (rows_far<T>(p)) return split_k(Tile::k64, p, 3 * cus / t64, 1024, BK);
+    // Rows this far apart have the 64 x 64 tiles, and 16-bit slices the 128 x
+    // 128 ones (launch_config).
+    if (rows_far<T>(p)) {
+        if (sizeof(typename Elem<T>::storage) == 2 && thin > 64 && t128 <= cus / 4) {
+            const TilePlan plan = split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
+            if (plan.slices > 1) return plan;
+        }
+        return split_k(Tile::k64, p, 3 * cus / t64, 1024, BK);
+    }
     if constexpr (std::is_same<T, float>::value) {
         if (p.batch == 1 && thin > 16 && thin <= 64) {
             const TilePlan plan = plan_small_batch<T>(p, cus);
@@ -1393,6 +1400,14 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
         return best;
     } else {
         if (thin <= 64) return plan_small_batch<T>(p, cus);
+        // A very long K on few tiles is read from memory: 128 x 128 tiles read
+        // each operand half as often as 64 x 64 ones, one block a CU.  bf16 256
+        // x 256 x 65536 34 us against 37, x 2^20 447 against 628; 128 x 128 x
+        // 2^20 158 against 208; 512 x 512 x 16384 26 against 28; below, 64 x 64
+        // tiles are faster (256 x 256 x 16384 15 against 19).
+        if (t128 <= cus / 4 && p.k >= 16384 && p.k / (cus / t128) >= 1024) {
+            return split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
+        }
         // One round of 128 x 128 tiles by splitting K: when K is long, or when
         // one row of tiles reads a wide operand once.  1500 x 700 x 5000
         // 30.8 us in three slices, 40.6 on 64 x 128 tiles whole; 1024 x 1536
@@ -1634,7 +1649,9 @@ bool tiles_take_thin(int dtype, const GemmArgs& p, int device) {
     const int64_t blocks = (plan.tile == Tile::k64 ? t64 : tiles_of(p, 64, 128)) * plan.slices;
     if (thin > 32) return blocks >= cus / 4;
     if (thin > 16) return blocks >= cus / 2;
-    return plan.slices > 1 && 2 * blocks >= 3 * cus;
+    // As few columns write C column by column: 18368 x 8 x 2176 bf16 24.7 us
+    // on tiles, 21.4 on the thin kernel; 4416 x 16 x 7296 17.5 and 20.4.
+    return plan.slices > 1 && 2 * blocks >= 3 * cus && (p.m <= 64 || t64 < cus / 2);
 }
 
 void launch_gemm(int dtype, const GemmArgs& p, hipStream_t stream) {
