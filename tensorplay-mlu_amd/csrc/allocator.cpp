@@ -43,7 +43,7 @@ DeviceCache& cache() {
 
 Block* device_alloc(size_t nbytes, int device) {
     const int index = resolve_device(device);
-    return cache().obtain<Error>(index, nbytes);
+    return cache().obtain<OutOfMemory>(index, nbytes);
 }
 
 void device_free(Block* block) { cache().recycle(block); }

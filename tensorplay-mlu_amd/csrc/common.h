@@ -21,6 +21,11 @@ struct Error : std::runtime_error {
     explicit Error(const std::string& what) : std::runtime_error(what) {}
 };
 
+// The device has no memory left.
+struct OutOfMemory : Error {
+    using Error::Error;
+};
+
 // The device path does not handle these arguments; nothing has been written
 // and the caller runs the operator on the host (the reference's
 // TP_CNNL_TRY / std::nullopt convention, MLURuntime.h:34-51).

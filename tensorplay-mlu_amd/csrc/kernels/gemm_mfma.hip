@@ -1250,12 +1250,11 @@ void launch_finish(const float* part, int slices, const GemmArgs& p, hipStream_t
 
 // Splits K: the slices, K tiles of ks = a multiple of BK (the last one
 // shorter), ride on the tile kernel's batch index and write float32 partial
-// products into a workspace [slices][M][N]; splitk_finish_kernel then adds
+// products into `part`, [slices][M][N]; splitk_finish_kernel then adds
 // them in slice order, so the result does not depend on timing.
 template <typename T, int BM, int BN, int STAGES, int BLOCKS>
-void launch_split(const GemmArgs& p, int64_t slices, int64_t ks, hipStream_t stream, int device) {
+void launch_split(const GemmArgs& p, int64_t slices, int64_t ks, void* part, hipStream_t stream) {
     const int64_t mn = p.m * p.n;
-    Workspace ws(static_cast<size_t>(slices * mn) * sizeof(float), device);
     GemmArgs q = p;
     q.batch = slices;
     q.k = ks;
@@ -1265,11 +1264,11 @@ void launch_split(const GemmArgs& p, int64_t slices, int64_t ks, hipStream_t str
     q.alpha = 1.0f;
     q.beta = 0.0f;
     q.cin = nullptr;
-    q.c = ws.get();
+    q.c = part;
     q.ldc = p.n;
     q.stride_c = mn;
     launch_config<T, BM, BN, STAGES, BLOCKS, true>(q, stream);
-    launch_finish<T>(static_cast<const float*>(ws.get()), static_cast<int>(slices), p, stream);
+    launch_finish<T>(static_cast<const float*>(part), static_cast<int>(slices), p, stream);
 }
 
 // The tile kernel's shapes (LDS stages, blocks a CU) and what each is for.
@@ -1459,15 +1458,20 @@ void launch_mfma(const GemmArgs& p, hipStream_t stream) {
             return;
         }
     }
-    const TilePlan plan = plan_tiles<T>(p, cus);
+    TilePlan plan = plan_tiles<T>(p, cus);
+    Workspace part;
+    if (plan.slices > 1) {
+        part = Workspace::if_room(static_cast<size_t>(plan.slices * p.m * p.n) * sizeof(float), device);
+        if (part.get() == nullptr) plan = TilePlan{Tile::k64};  // whole K needs no memory
+    }
     if (plan.slices > 1) {
         if constexpr (k16) {
-            if (plan.tile == Tile::k128) launch_split<T, 128, 128, 2, 2>(p, plan.slices, plan.ks, stream, device);
-            else if (plan.tile == Tile::k128Deep) launch_split<T, 128, 128, 3, 1>(p, plan.slices, plan.ks, stream, device);
-            else launch_split<T, 64, 64, 3, 3>(p, plan.slices, plan.ks, stream, device);
+            if (plan.tile == Tile::k128) launch_split<T, 128, 128, 2, 2>(p, plan.slices, plan.ks, part.get(), stream);
+            else if (plan.tile == Tile::k128Deep) launch_split<T, 128, 128, 3, 1>(p, plan.slices, plan.ks, part.get(), stream);
+            else launch_split<T, 64, 64, 3, 3>(p, plan.slices, plan.ks, part.get(), stream);
         } else {
-            if (plan.tile == Tile::k32x128) launch_split<T, 32, 128, 4, 2>(p, plan.slices, plan.ks, stream, device);
-            else launch_split<T, 64, 64, 2, 4>(p, plan.slices, plan.ks, stream, device);
+            if (plan.tile == Tile::k32x128) launch_split<T, 32, 128, 4, 2>(p, plan.slices, plan.ks, part.get(), stream);
+            else launch_split<T, 64, 64, 2, 4>(p, plan.slices, plan.ks, part.get(), stream);
         }
         return;
     }
@@ -1606,7 +1610,11 @@ void launch_repacked(const GemmArgs& p, hipStream_t stream) {
     const bool fix_b = pad || !packets_aligned<T>(p.b, p.ldb, p.stride_b);
     const Repack<T> a(p.lda, p.stride_a, a_kmajor, p.batch, p.m, p.k, kp), b(p.ldb, p.stride_b, b_kmajor, p.batch, p.n, p.k, kp);
     const size_t off_b = fix_a ? (a.elems() * a.E + 255) / 256 * 256 : 0;
-    Workspace ws(off_b + (fix_b ? b.elems() * b.E : 0), device);
+    const Workspace ws = Workspace::if_room(off_b + (fix_b ? b.elems() * b.E : 0), device);
+    if (ws.get() == nullptr) {
+        launch_mfma<T>(p, stream);  // in place
+        return;
+    }
     GemmArgs q = p;
     q.k = kp;
     if (fix_a) {

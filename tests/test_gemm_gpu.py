@@ -763,6 +763,43 @@ def test_gemm_of_a_very_long_k(amd, dev, ops, orc, dtype, ta, tb):
     assert np.array_equal(got, orc.from_float(want.astype(np.float32), dtype))
 
 
+def test_gemm_without_room_for_scratch(amd, dev, orc):
+    """With the device's memory taken up to a few MiB, products that would be
+    cut into slices of K or copied to aligned rows run without: the same
+    results to rounding, no error."""
+    lib = amd.load()
+    # 28 MB of slices (16-bit), 35 MB of slices (float32), 27 MB of copies
+    cases = []
+    for dtype, m, n, k in ((BF16, 776, 3000, 11000), (F32, 1500, 1500, 4000), (BF16, 2601, 2603, 2602)):
+        a, b = sample(orc, (m, k), dtype, 81, 0.25), sample(orc, (n, k), dtype, 82, 0.25)
+        da, db, out = dev.from_numpy(a, dtype=dtype), dev.from_numpy(b, dtype=dtype), dev.empty((m, n), dtype=dtype)
+        cases.append((dtype, m, n, k, da, db, out))
+
+    def run():
+        for dtype, m, n, k, da, db, out in cases:
+            st = lib.tp_amd_launch_gemm(0, dtype, 1, m, n, k, 1.0, da.data_ptr, k, 0, 0, db.data_ptr, k, 0, 1, 0.0, 0, 0,
+                                        0, 0, out.data_ptr, n, 0)
+            assert st == 0, lib.tp_mlu_last_error()
+        return [orc.to_float(out.numpy(), dtype) for dtype, *_, out in cases]
+
+    want = run()
+    lib.tp_mlu_empty_cache()
+    held, size = [], 1 << 36
+    while size >= 8 << 20:
+        try:
+            held.append(dev.empty((size,), dtype="uint8"))
+        except RuntimeError:
+            size //= 2
+    try:
+        got = run()
+    finally:
+        held.clear()
+        lib.tp_mlu_empty_cache()
+    for (dtype, m, n, k, *_), g, w in zip(cases, got, want):
+        assert np.linalg.norm(g - w) <= (1e-5 if dtype == F32 else 4e-3) * np.linalg.norm(w), (m, n, k)
+    assert any(not np.array_equal(g, w) for g, w in zip(got, want)), "the slices' memory was there"
+
+
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)],
                          ids=["NN", "TN", "NT", "TT"])
 @pytest.mark.parametrize("m,n,k,cin_kind", [(4096, 4096, 1024, "none"), (4090, 4081, 1001, "full"),
