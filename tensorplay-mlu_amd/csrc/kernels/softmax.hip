@@ -520,23 +520,28 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_long_kernel(
             unpack<T>(raw[u], v);
             float pm = v[0];
 #pragma unroll
-            for (int j = 1; j < N; ++j) pm = max_keep_nan(pm, v[j]);
-            const float mn = max_keep_nan(m, pm);
-            if (mn == -INFINITY) continue;  // only -inf so far
+            for (int j = 1; j < N; ++j) pm = fmaxf(pm, v[j]);
+            // With nothing but -inf (or NaN) so far, exponentials relative
+            // to 0: 0 of -inf, and NaN stays.
+            const float mn = fmaxf(m, pm), shift = mn == -INFINITY ? 0.0f : mn;
             float t = 0.0f;
 #pragma unroll
-            for (int j = 0; j < N; ++j) t += exp_fast(v[j] - mn);
-            s = s * exp_fast(m - mn) + t;
+            for (int j = 0; j < N; ++j) t += exp_fast(v[j] - shift);
+            s = s * exp_fast(m - shift) + t;
             m = mn;
         }
     }
     const bool tail = ANY && threadIdx.x < D - npk * N;  // one of the row's last D % N elements
     const float tv = tail ? Elem<T>::load(xr[npk * N + threadIdx.x]) : -INFINITY;
     if (ANY && tv != -INFINITY) {
-        const float mn = max_keep_nan(m, tv);
+        const float mn = fmaxf(m, tv);
         s = s * exp_fast(m - mn) + exp_fast(tv - mn);
         m = mn;
     }
+    // fmaxf lets a NaN go, and each exponential of one is NaN: the sum keeps
+    // it, and the merge takes it from the maximum (NaN kept by the maximum
+    // of every packet: 8-18 % of the kernel).
+    if (s != s) m = s;
     block_merge(m, s);
     const float shift = m == -INFINITY ? 0.0f : m;
     const float lse = logf(s);
