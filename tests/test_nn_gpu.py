@@ -99,8 +99,8 @@ def test_layer_norm_backward(dev, ops, orc, dtype, shape, norm):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
-@pytest.mark.parametrize("rows,D", [(7, 4), (5, 9), (40, 17), (9, 515), (300, 1001), (70, 2047), (600, 4099), (3, 8185),
-                                    (5, 16387)])
+@pytest.mark.parametrize("rows,D", [(7, 4), (5, 9), (40, 17), (1000, 118), (9, 515), (300, 1001), (70, 2047), (600, 4099),
+                                    (3, 8185), (5, 16387)])
 def test_layer_norm_rows_at_any_element(dev, ops, orc, dtype, rows, D):
     """Rows that are not whole packets, in tensors that start off a 16-byte
     boundary (and, once, whole rows off it): the packet that ends a row
