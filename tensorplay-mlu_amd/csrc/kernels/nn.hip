@@ -1258,7 +1258,7 @@ constexpr int64_t kPlanListCap = int64_t{1} << 22;     // list entries beyond wh
 // has about 550, and its one block took 1386 us of a gradient whose other
 // rows are done in 130.
 constexpr int kHotSamples = 32;
-constexpr int kHotBlocks = 512;  // blocks that walk the heavy rows' (row, column chunk) pairs
+constexpr int kHotBlocks = 512;  // most blocks that walk the heavy rows' (row, column chunk) pairs
 
 template <typename I>
 __global__ __launch_bounds__(kRangeThreads) void embedding_plan_range_kernel(const void* idx, int n, int64_t V,
@@ -1400,10 +1400,18 @@ constexpr int64_t kGatherCachedBytes = int64_t{256} << 20;
 // ROWS rows a block: one row of four waves, or four rows of one wave each
 // where a row is at most kSmallRowBytes (a block a row leaves most of its
 // threads without a column there, and 50257 of them are bound by how fast
-// blocks start).
+// blocks start) and they still give each CU a block (bf16 512 x 768: 7.6 us a
+// block a row, 8.5 so).
 constexpr int64_t kSmallRowBytes = 2048;
+// Blocks a CU: the heavy rows' loads left to themselves take the registers of
+// six, which all the other rows' blocks feel (float32 50257 x 768 from 64
+// indices 38.4 us with six, 31.5 with eight); single bfloat16 columns would
+// spill at eight.
+template <typename T, bool VEC>
+constexpr int gather_blocks() { return VEC || !std::is_same_v<T, bf16_t> ? 8 : 6; }
+
 template <typename T, bool VEC, bool NT, int ROWS>
-__global__ __launch_bounds__(kBlock) void embedding_gather_ordered_kernel(
+__global__ __launch_bounds__(kBlock, (gather_blocks<T, VEC>())) void embedding_gather_ordered_kernel(
     const S_<T>* dy, const int* starts, const int* counts, const int* list, int n_list, int64_t D,
     int64_t V, int scale_grad_by_freq, S_<T>* out, int hot_blocks, const int* hot_n, const int* hot, int plan_blocks,
     int plan_rows) {
@@ -1803,7 +1811,6 @@ int tp_amd_launch_embedding_backward(int device, int dtype, int64_t n, int64_t d
             int* list = counts + num_weights;
             int* hot_n = list + regions * n;
             int* hot = hot_n + range_blocks;
-            const int hot_blocks = n >= kHotSamples ? kHotBlocks : 0;
             dispatch_index<float>(index_dtype, [&](auto tag) {
                 using I = decltype(tag);
                 embedding_plan_range_kernel<I><<<range_blocks, kRangeThreads, 0, st>>>(
@@ -1813,7 +1820,13 @@ int tp_amd_launch_embedding_backward(int device, int dtype, int64_t n, int64_t d
             TP_AMD_DISPATCH_NN(dtype, T, {
                 const bool vec = dim % Packet<T>::N == 0 && aligned16(grad) && aligned16(out);
                 const bool nt = num_weights * dim * static_cast<int64_t>(sizeof(S_<T>)) > kGatherCachedBytes;
-                const bool small = dim * static_cast<int64_t>(sizeof(S_<T>)) <= kSmallRowBytes;
+                const bool small = dim * static_cast<int64_t>(sizeof(S_<T>)) <= kSmallRowBytes &&
+                                   num_weights >= 4 * cu_count(index);
+                // n samples make at most n / kHotSamples heavy rows; for less
+                // than two, looking for them costs more than they do
+                // (3208 x 2670 from 32 uniform indices 12.1 -> 13.1 us)
+                const int64_t pairs = n / kHotSamples * blocks_for(dim, kBlock * (vec && sizeof(S_<T>) == 2 ? 2 : 1));
+                const int hot_blocks = n < 2 * kHotSamples ? 0 : static_cast<int>(std::min<int64_t>(kHotBlocks, pairs));
                 auto gather = [&](auto vec_tag, auto nt_tag) {
                     constexpr bool V = decltype(vec_tag)::value, C = decltype(nt_tag)::value;
                     auto* kernel = small ? embedding_gather_ordered_kernel<T, V, C, 4>

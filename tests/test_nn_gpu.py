@@ -370,6 +370,21 @@ def test_embedding_dense_backward_sample_counts_around_the_split(dev, ops, orc, 
         assert_bitexact(got, sample_order_sum(orc, dtype, dy, idx, V, len(counts) - 1, freq), f"freq={freq}")
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("V,n", [(8, 32), (8, 63), (8, 64), (1023, 200), (1025, 200)])
+@pytest.mark.parametrize("D", [8, 264, 771], ids=lambda d: f"D{d}")
+def test_embedding_dense_backward_few_samples(dev, ops, orc, dtype, V, n, D):
+    """A row with most of a few samples, summed by its own block or by one a
+    column chunk, in tables of one row a block or four: bit-exact against
+    the sum in sample order."""
+    rng = np.random.default_rng(28)
+    idx = rng.integers(0, V, size=n).astype(np.int64)
+    idx[rng.permutation(n)[:n * 3 // 4]] = V - 2
+    dy = sample(orc, (n, D), dtype, 29)
+    got = ops.embedding_dense_backward(dev.from_numpy(dy, dtype=dtype), dev.from_numpy(idx), V, 2, False).numpy()
+    assert_bitexact(got, sample_order_sum(orc, dtype, dy, idx, V, 2, False), "sum in sample order")
+
+
 def test_embedding_declines_sparse(dev, ops, orc):
     w = dev.from_numpy(sample(orc, (10, 8), F32, 17))
     i = dev.from_numpy(np.array([1, 2], np.int64))
