@@ -256,11 +256,13 @@ __device__ __forceinline__ float row_share(const typename Elem<Tin>::storage* p,
 
 // Row segments.  Segment s covers row s / nseg, elements
 // [(s % nseg) * chunk, min(r, ... + chunk)).  WAVES wavefronts share one
-// segment (1: each wave of the block takes its own segment).  ANY: rows that
-// start at any element (r not a whole number of packets); the scalar loop
-// they took ran [8191, 4095] bfloat16 in 23-28 us, 11-12 us so (whole tensor 38-51
-// -> 13).
-template <typename Tin, typename Tout, int OP, int WAVES, bool ANY>
+// segment (1: each wave of the block takes its own segment).  Rows that start
+// at any element (r not a whole number of packets) take unaligned packets, or
+// when short (scalar_rows) one element a thread: a packet loop's fixed work a
+// row is then more than the row's.
+enum class RowLoad { kAligned, kAny, kScalar };
+
+template <typename Tin, typename Tout, int OP, int WAVES, RowLoad LOAD>
 __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(
     const typename Elem<Tin>::storage* x, typename Elem<Tout>::storage* out, int64_t nsegs,
     int64_t r, int64_t chunk, int64_t nseg, bool final_pass, int64_t count) {
@@ -274,7 +276,14 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(
         const int64_t row = seg / nseg, part = seg - row * nseg;
         const int64_t begin = part * chunk;
         const int64_t end = begin + chunk < r ? begin + chunk : r;
-        acc = row_share<Tin, OP, kThreads, 4, true, ANY>(x + row * r, begin, end, tid);
+        const typename Elem<Tin>::storage* p = x + row * r;
+        if constexpr (LOAD == RowLoad::kScalar) {
+            for (int64_t j = begin + tid; j < end; j += kThreads) {
+                acc = Combine<OP>::apply(acc, Elem<Tin>::load(p[j]));
+            }
+        } else {
+            acc = row_share<Tin, OP, kThreads, 4, true, LOAD == RowLoad::kAny>(p, begin, end, tid);
+        }
     }
     acc = lane_reduce<OP>(acc);
     if constexpr (WAVES > 1) {
@@ -726,6 +735,13 @@ SplitPlan plan_split(int64_t outer, int64_t r, int64_t inner, int64_t cus, int64
     return sp;
 }
 
+// Whether rows of r elements that are not whole packets go one element a
+// thread: up to three (float32) or nine (16-bit) loads a lane.  Elements,
+// packets, us: float32 65027 x 129 sum 13.8, 15.1, 43464 x 193 11.7, 10.9 and
+// amin 13.6, 14.1; bf16 63550 x 33 sum 9.2, 15.2, 21788 x 385 6.1, 7.6, 10908
+// x 769 6.1, 5.9 and amin 8.3, 6.2; [8191, 4095] 23-28, 11-12.
+bool scalar_rows(int64_t r, int64_t packet) { return r <= (packet == 4 ? 192 : 576); }
+
 template <typename T, int OP>
 void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const void* xv,
                   void* outv, const Scratch& scratch) {
@@ -759,7 +775,9 @@ void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const voi
             constexpr int W = decltype(waves_tag)::value;
             constexpr int per_block = (kBlock / kWave) / W;
             const int64_t blocks = (outer + per_block - 1) / per_block;
-            auto* kernel = aligned ? reduce_rows_kernel<T, T, OP, W, false> : reduce_rows_kernel<T, T, OP, W, true>;
+            auto* kernel = aligned             ? reduce_rows_kernel<T, T, OP, W, RowLoad::kAligned>
+                           : scalar_rows(r, N) ? reduce_rows_kernel<T, T, OP, W, RowLoad::kScalar>
+                                               : reduce_rows_kernel<T, T, OP, W, RowLoad::kAny>;
             kernel<<<blocks, kBlock, 0, st>>>(x, out, outer, r, r, 1, true, r);
         };
         if (long_rows) {

@@ -143,13 +143,15 @@ def test_few_long_rows_folded_in_one_launch(dev, ops, orc, dtype, shape):
 @pytest.mark.parametrize("shape,dims", [((70, 3), [1]), ((70, 9), [1]), ((33, 515), [1]), ((9, 4099), [1]),
                                         ((3, 8193), [1]), ((2, 70003), [1]), ((19, 4097), None),
                                         ((300, 9), [0]), ((77, 17), [0]), ((2000, 129), [0]), ((400, 4095), [0]),
-                                        ((3, 700, 263), [1]), ((600, 5), [0])],
+                                        ((3, 700, 263), [1]), ((600, 5), [0]),
+                                        ((70, 192), [1]), ((70, 193), [1]), ((70, 575), [1]), ((70, 577), [1])],
                          ids=lambda v: str(v).replace(" ", ""))
 def test_reductions_of_ragged_rows(dev, ops, orc, dtype, shape, dims):
     """Rows that are not a whole number of packets, in a tensor that starts
-    off a 16-byte boundary: packets at any element, the last elements of a
-    row one to a thread, the last packet of a column reduction over columns
-    its neighbour also takes.  NaNs, zeros of both signs and extrema in the
+    off a 16-byte boundary: single elements, or packets at any element, the
+    last elements of a row one to a thread, the last packet of a column
+    reduction over columns its neighbour also takes (sizes on both sides of
+    each rule, rows split or not).  NaNs, zeros of both signs and extrema in the
     first and last elements of rows and columns."""
     n = int(np.prod(shape))
     a = sample(orc, (n + 1,), dtype, 71, mean=0.5)
