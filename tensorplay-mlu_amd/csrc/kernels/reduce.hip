@@ -487,7 +487,8 @@ __device__ __forceinline__ void cols_keys(float (&acc)[Packet<Tin>::N],
 // whole number of them, or x off a 16-byte boundary).  The last packet of a
 // row then starts inner - N in, over columns its neighbour also takes: both
 // compute the same value in the same order and store it.  VEC false: single
-// elements, for rows shorter than a packet.
+// elements, for rows shorter than a packet and others of no whole number of
+// them (plan_columns).
 //
 // FUSE folds the second pass in: the partials are written and read back
 // with agent-coherent accesses; every block counts its arrival in
@@ -742,6 +743,39 @@ SplitPlan plan_split(int64_t outer, int64_t r, int64_t inner, int64_t cus, int64
 // x 769 6.1, 5.9 and amin 8.3, 6.2; [8191, 4095] 23-28, 11-12.
 bool scalar_rows(int64_t r, int64_t packet) { return r <= (packet == 4 ? 192 : 576); }
 
+// The plan over columns, and whether they are read by packets (vec).  Whole
+// packets are; rows of another length (unaligned packets, a block to 256 or
+// 128 columns instead of 64) where the loads saved are more than what fewer
+// and wider column ranges cost: idle lanes, or more chunks of rows for the
+// last block to fold.  Elements, packets, us, of outer x r x inner sums (and
+// amin):
+//   not split: float32 1024 x 64 x 129 10.0, 6.0; 256 x 512 x 77 10.6, 13.0;
+//     8192 x 16 x 77 17.9, 11.1; 16-bit 8192 x 4 x 129 amin 16.8, 22.1
+//   split: float32 8000 x 205 8.5, 15.9 (14.7, 30.8); 8000 x 777 10.5, 11.6;
+//     16000 x 641 15.8, 13.7 (26.9, 19.2); 512 x 8193 5.4, 7.3; 1000 x 8193
+//     11.5, 10.4 (18.2, 11.4); bf16 16000 x 193 9.1, 12.2; 16000 x 513 12.8,
+//     8.7 (23.9, 12.7); 1000 x 4097 5.9, 7.1
+struct ColumnPlan : SplitPlan {
+    bool vec = false;
+};
+
+ColumnPlan plan_columns(int64_t outer, int64_t r, int64_t inner, int64_t cus, int64_t packet) {
+    ColumnPlan cp;
+    if (inner >= packet) {
+        static_cast<SplitPlan&>(cp) = plan_split(outer, r, inner, cus, packet, col_lanes(packet) * packet);
+        const double total = static_cast<double>(outer) * static_cast<double>(r) * static_cast<double>(inner);
+        if (inner % packet == 0) {
+            cp.vec = true;
+        } else if (cp.nchunk == 1) {
+            cp.vec = (inner >= 128 || (inner >= 64 && outer >= 4 * cus)) && (packet == 4 || r >= 16);
+        } else {
+            cp.vec = inner >= 128 && cp.chunk >= 64 && total >= 8e6 && total >= 6e4 * static_cast<double>(cp.nchunk);
+        }
+    }
+    if (!cp.vec) static_cast<SplitPlan&>(cp) = plan_split(outer, r, inner, cus, packet, 64);
+    return cp;
+}
+
 template <typename T, int OP>
 void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const void* xv,
                   void* outv, const Scratch& scratch) {
@@ -789,10 +823,9 @@ void reduce_typed(int device, int64_t outer, int64_t r, int64_t inner, const voi
         return;
     }
     // Column reductions.
-    const bool vec = inner >= N, aligned = inner % N == 0 && aligned16(x);
     constexpr int L = col_lanes(N);
-    const int64_t cols_per_block = vec ? L * N : 64;
-    const SplitPlan sp = plan_split(outer, r, inner, cus, N, cols_per_block);
+    const ColumnPlan sp = plan_columns(outer, r, inner, cus, N);
+    const bool vec = sp.vec, aligned = inner % N == 0 && aligned16(x);
     const int64_t bx = sp.bx, nchunk = sp.nchunk, chunk = sp.chunk;
     const dim3 grid(static_cast<unsigned>(bx), static_cast<unsigned>(nchunk), static_cast<unsigned>(sp.z));
     if (nchunk == 1) {
@@ -911,9 +944,9 @@ int64_t tp_amd_reduce_partial_bytes(int compute_units, int dtype, int64_t outer,
     if (compute_units <= 0 || outer < 0 || r < 0 || inner < 0) return -1;
     if (outer == 0 || inner == 0 || r == 0) return 0;
     const int64_t packet = 16 / esize;
-    const int64_t cols_per_block = inner >= packet ? col_lanes(packet) * packet : 64;
-    return plan_split(outer, r, inner, compute_units, packet, cols_per_block).partial_floats *
-           static_cast<int64_t>(sizeof(float));
+    const SplitPlan sp = inner == 1 ? plan_split(outer, r, 1, compute_units, packet, 0)
+                                    : plan_columns(outer, r, inner, compute_units, packet);
+    return sp.partial_floats * static_cast<int64_t>(sizeof(float));
 }
 
 }  // extern "C"

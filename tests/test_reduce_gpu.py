@@ -144,7 +144,9 @@ def test_few_long_rows_folded_in_one_launch(dev, ops, orc, dtype, shape):
                                         ((3, 8193), [1]), ((2, 70003), [1]), ((19, 4097), None),
                                         ((300, 9), [0]), ((77, 17), [0]), ((2000, 129), [0]), ((400, 4095), [0]),
                                         ((3, 700, 263), [1]), ((600, 5), [0]),
-                                        ((70, 192), [1]), ((70, 193), [1]), ((70, 575), [1]), ((70, 577), [1])],
+                                        ((70, 192), [1]), ((70, 193), [1]), ((70, 575), [1]), ((70, 577), [1]),
+                                        ((1100, 17, 67), [1]), ((300, 20, 131), [1]), ((2, 8, 1025), [1]),
+                                        ((1001, 8193), [0])],
                          ids=lambda v: str(v).replace(" ", ""))
 def test_reductions_of_ragged_rows(dev, ops, orc, dtype, shape, dims):
     """Rows that are not a whole number of packets, in a tensor that starts

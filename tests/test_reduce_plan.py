@@ -37,6 +37,14 @@ def test_exact_figures(lib):
     # rows that fill the chip, or short rows: one segment a row, no partials
     assert q(256, F32, 32768, 4096, 1) == 0
     assert q(256, F32, 3, 4000, 1) == 0
+    # columns that are no whole packets: ranges of 64 single elements where 256 (or 128 in
+    # 16 bits) would mean many more chunks of rows for the last block to fold, else packets
+    assert q(256, F32, 1, 8000, 205) == 64 * 205 * 4       # 4 ranges of 64; 250 chunks with one of 256
+    assert q(256, BF16, 1, 8000, 205) == 64 * 205 * 4
+    assert q(256, F32, 1, 512, 8193) == 2 * 8193 * 4       # 129 ranges of 64; 8 chunks with 33 of 256
+    assert q(256, F32, 1, 2000, 8193) == 8 * 8193 * 4      # 33 ranges of 256
+    assert q(256, BF16, 1, 16000, 641) == 43 * 641 * 4     # 6 ranges of 128
+    assert q(256, F32, 1, 60000, 9) == 256 * 9 * 4
     assert q(256, F32, 0, 10, 10) == 0
     assert q(256, 3, 1, 10, 10) == -1          # float64 has no device reduction
     assert q(0, F32, 1, 10, 10) == -1
