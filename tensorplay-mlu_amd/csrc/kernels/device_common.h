@@ -90,39 +90,6 @@ __device__ __forceinline__ Packet<T> load_packet(const typename Elem<T>::storage
     return out;
 }
 
-template <typename T>
-__device__ __forceinline__ void store_packet(typename Elem<T>::storage* p, const Packet<T>& v) {
-    uint4 raw;
-    __builtin_memcpy(&raw, &v, 16);
-    *reinterpret_cast<uint4*>(p) = raw;
-}
-
-// Streaming variants: the data is touched once, so keep it out of the
-// caches' way (nontemporal loads/stores).
-template <typename T>
-__device__ __forceinline__ Packet<T> load_packet_nt(const typename Elem<T>::storage* p) {
-    Packet<T> out;
-    uint4 raw;
-    const uint4* q = reinterpret_cast<const uint4*>(p);
-    raw.x = __builtin_nontemporal_load(&q->x);
-    raw.y = __builtin_nontemporal_load(&q->y);
-    raw.z = __builtin_nontemporal_load(&q->z);
-    raw.w = __builtin_nontemporal_load(&q->w);
-    __builtin_memcpy(&out, &raw, 16);
-    return out;
-}
-
-template <typename T>
-__device__ __forceinline__ void store_packet_nt(typename Elem<T>::storage* p, const Packet<T>& v) {
-    uint4 raw;
-    __builtin_memcpy(&raw, &v, 16);
-    uint4* q = reinterpret_cast<uint4*>(p);
-    __builtin_nontemporal_store(raw.x, &q->x);
-    __builtin_nontemporal_store(raw.y, &q->y);
-    __builtin_nontemporal_store(raw.z, &q->z);
-    __builtin_nontemporal_store(raw.w, &q->w);
-}
-
 // Raw 16-byte packets converted to and from float32 lanes, for kernels whose
 // per-element arithmetic is the limit (softmax, transcendental activations):
 // bfloat16 unpacks with one shift or mask per element and packs two elements
@@ -169,6 +136,8 @@ __device__ __forceinline__ uint4 pack(const float (&f)[Packet<T>::N]) {
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Streaming variants: the data is touched once, so keep it out of the
+// caches' way (nontemporal loads/stores).
 __device__ __forceinline__ uint4 load_raw_nt(const void* p) {
     const uint4* q = static_cast<const uint4*>(p);
     uint4 raw;

@@ -1168,7 +1168,7 @@ void launch_config(const GemmArgs& whole, hipStream_t stream) {
         const int64_t k = F32OUT ? p.k_total : p.k;
         if (rows_far<T>(p)) {
             constexpr bool kSlices128 = F32OUT && BM == 128 && STAGES == 3;
-            if constexpr (BM == 64 && BN == 64 || kSlices128) launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kFar>(p, stream);
+            if constexpr ((BM == 64 && BN == 64) || kSlices128) launch_chunk<T, BM, BN, STAGES, BLOCKS, F32OUT, Rows::kFar>(p, stream);
             else TP_AMD_CHECK(false, "a tile that cannot take rows this far apart");
         } else if (whole_dwords<T>(p.a, p.lda, p.stride_a, !p.trans_a, p.m, k) &&
                    whole_dwords<T>(p.b, p.ldb, p.stride_b, p.trans_b, p.n, k)) {
@@ -1462,7 +1462,10 @@ void launch_mfma(const GemmArgs& p, hipStream_t stream) {
     Workspace part;
     if (plan.slices > 1) {
         part = Workspace::if_room(static_cast<size_t>(plan.slices * p.m * p.n) * sizeof(float), device);
-        if (part.get() == nullptr) plan = TilePlan{Tile::k64};  // whole K needs no memory
+        if (part.get() == nullptr) {  // whole K needs no memory
+            if (p.k >> 32) return launch_gemm_general<T>(p, stream);  // past a panel's 32-bit K
+            plan = TilePlan{Tile::k64};
+        }
     }
     if (plan.slices > 1) {
         if constexpr (k16) {
