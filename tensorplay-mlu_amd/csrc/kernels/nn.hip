@@ -383,7 +383,7 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
     // writes the block's partial row; dW then dB.  `fold` is laid out by
     // packets, so a whole packet moves at once also where the last one
     // overlaps its neighbour (by columns, such rows' single-element accesses
-    // made this 10 us of 21: bf16 [1000, 118] 21.6 -> 11.0 us).
+    // made this 10 us of 21: bf16 [1000, 118] 21.6 -> 11.3 us).
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
         float (&mine)[VPT][N] = which == 0 ? pw : pb;
@@ -395,10 +395,7 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
                 for (int k = 0; k < VPT; ++k) {
                     if (at[k].first < N) {
                         const int64_t c0 = at[k].off / sizeof(S_<T>);
-                        float* slot = fold + (tid + k * kThreads) * N;
-                        float v[N];
-#pragma unroll
-                        for (int j = 0; j < N; ++j) v[j] = src < GROUPS - 1 ? mine[k][j] + slot[j] : mine[k][j];
+                        float* slot = fold + (ANY ? (tid + k * kThreads) * N : c0);
                         auto put = [](float* to, float value) {
                             // 16-bit rows: non-temporal partials, bf16
                             // [8192, 4096] 35.9-36.2 against 36.5-36.8 us
@@ -409,17 +406,32 @@ __global__ __launch_bounds__(GROUPS * WAVES * kWave) void layer_norm_backward_ro
                         auto column = [&](int64_t c) {
                             return out + c / kFoldChunk * gridDim.x * kFoldChunk + c % kFoldChunk;
                         };
-                        if (src > 0) {
-#pragma unroll
-                            for (int j = 0; j < N; ++j) slot[j] = v[j];
-                        } else if (!ANY || at[k].first == 0) {
-                            float* to = column(c0);  // a whole packet's N columns lie in one chunk
-#pragma unroll
-                            for (int j = 0; j < N; ++j) put(&to[j], v[j]);
-                        } else {
+                        if constexpr (!ANY) {
+                            // a packet's N columns lie in one chunk
+                            float* to = column(c0);
 #pragma unroll
                             for (int j = 0; j < N; ++j) {
-                                if (j >= at[k].first) put(column(c0 + j), v[j]);
+                                float v = mine[k][j];
+                                if (src < GROUPS - 1) v += slot[j];
+                                if (src > 0) slot[j] = v;
+                                else put(&to[j], v);
+                            }
+                        } else {
+                            float v[N];
+#pragma unroll
+                            for (int j = 0; j < N; ++j) v[j] = src < GROUPS - 1 ? mine[k][j] + slot[j] : mine[k][j];
+                            if (src > 0) {
+#pragma unroll
+                                for (int j = 0; j < N; ++j) slot[j] = v[j];
+                            } else if (at[k].first == 0) {
+                                float* to = column(c0);
+#pragma unroll
+                                for (int j = 0; j < N; ++j) put(&to[j], v[j]);
+                            } else {
+#pragma unroll
+                                for (int j = 0; j < N; ++j) {
+                                    if (j >= at[k].first) put(column(c0 + j), v[j]);
+                                }
                             }
                         }
                     }
@@ -564,12 +576,24 @@ __global__ __launch_bounds__(kFoldThreads) void fold_rows_kernel(const float* pa
             acc[l][3] += v[l].w;
         }
     }
-    for (; p < parts; p += kFoldGroups) {
-        const float4 v = part[p * kFoldQuads];
-        acc[0][0] += v.x;
-        acc[0][1] += v.y;
-        acc[0][2] += v.z;
-        acc[0][3] += v.w;
+    // The rows left over, in order into the first sum: their loads go out
+    // together too (one at a time they were 4 of 15 us at bfloat16 [1368, 742]).
+    if (p < parts) {
+        float4 v[kFoldBatch - 1];
+#pragma unroll
+        for (int l = 0; l < kFoldBatch - 1; ++l) {
+            const int64_t q = p + l * kFoldGroups;
+            v[l] = part[(q < parts ? q : p) * kFoldQuads];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int l = 0; l < kFoldBatch - 1; ++l) {
+            const bool in = p + l * kFoldGroups < parts;
+            acc[0][0] = in ? acc[0][0] + v[l].x : acc[0][0];
+            acc[0][1] = in ? acc[0][1] + v[l].y : acc[0][1];
+            acc[0][2] = in ? acc[0][2] + v[l].z : acc[0][2];
+            acc[0][3] = in ? acc[0][3] + v[l].w : acc[0][3];
+        }
     }
 #pragma unroll
     for (int h = kFoldBatch / 2; h >= 1; h /= 2) {
@@ -1405,7 +1429,7 @@ constexpr int64_t kGatherCachedBytes = int64_t{256} << 20;
 constexpr int64_t kSmallRowBytes = 2048;
 // Blocks a CU: the heavy rows' loads left to themselves take the registers of
 // six, which all the other rows' blocks feel (float32 50257 x 768 from 64
-// indices 38.4 us with six, 31.5 with eight); single bfloat16 columns would
+// indices 38.4 us with six, 32.4 with eight); single bfloat16 columns would
 // spill at eight.
 template <typename T, bool VEC>
 constexpr int gather_blocks() { return VEC || !std::is_same_v<T, bf16_t> ? 8 : 6; }
