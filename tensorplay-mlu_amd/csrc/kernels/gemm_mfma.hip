@@ -1400,20 +1400,37 @@ TilePlan plan_tiles(const GemmArgs& p, int64_t cus) {
     } else {
         if (thin <= 64) return plan_small_batch<T>(p, cus);
         // A very long K on few tiles is read from memory: 128 x 128 tiles read
-        // each operand half as often as 64 x 64 ones, one block a CU.  bf16 256
-        // x 256 x 65536 34 us against 37, x 2^20 447 against 628; 128 x 128 x
-        // 2^20 158 against 208; 512 x 512 x 16384 26 against 28; below, 64 x 64
-        // tiles are faster (256 x 256 x 16384 15 against 19).
-        if (t128 <= cus / 4 && p.k >= 16384 && p.k / (cus / t128) >= 1024) {
-            return split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
+        // each operand half as often as 64 x 64 ones, one block a CU.  bf16 512
+        // x 1024 x 15000 35.6 us against 46.0, 256 x 256 x 65536 34 against 37,
+        // x 2^20 447 against 628; 128 x 128 x 2^20 158 against 208; 512 x 512 x
+        // 16384 26 against 28; below, 64 x 64 tiles are level or faster (512 x
+        // 1024 x 12288 28.9 against 30.2, 256 x 256 x 16384 15 against 19).
+        // With so many 64 x 64 tiles that their slices are two, leaving some
+        // CUs two blocks and others one, from K = 4096 on: 200 x 3000 x 3000
+        // 17.8 against 18.2, x 4104 19.3 against 22.5, x 11000 33.4 against
+        // 51.9; 1124 x 624 x 8192 28.4 against 31.3; 1500 x 400 (168 tiles) x
+        // 8192 28.5 against 25.4, x 9000 34.1 against 35.7.  Not where 128 x
+        // 128 tiles are mostly padding (129 x 144 x 84864 32.4 against 29.1).
+        if (t128 <= cus / 4) {
+            if (p.k > 12288 && p.k / (cus / t128) >= 1024 && 2 * t64 >= 5 * t128) {
+                return split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
+            }
+            if (t64 > cus * 5 / 8 && p.k >= (t64 > cus * 11 / 16 ? 4096 : 9000)) {
+                return split_k(Tile::k128Deep, p, cus / t128, 768, BK);
+            }
         }
         // One round of 128 x 128 tiles by splitting K: when K is long, or when
         // one row of tiles reads a wide operand once.  1500 x 700 x 5000
         // 30.8 us in three slices, 40.6 on 64 x 128 tiles whole; 1024 x 1536
         // x 8192 41.8 against 44.5; 128 x 11008 x 4096 33.6 against 37.3 on
-        // 64 x 64 tiles; 1280 x 1280 x 3000 28.0 in two, 26.5 whole.
+        // 64 x 64 tiles; 1280 x 1280 x 3000 28.0 in two, 26.5 whole.  Where
+        // whole slices leave a fifth of the CUs idle and K is long, two blocks a
+        // CU come closer: 1200 x 1100 x 11000 (90 tiles) 69.6 and 63.0, 1536 x
+        // 1024 x 15000 (96) 88 and 82; x 6000 40.6 and 42.
         if (t128 >= cus / 4 && t128 <= cus / 2 && (p.k > 4096 || (thin <= 128 && t64 > cus && p.k >= 2048))) {
-            const TilePlan plan = split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
+            const bool idle = 5 * t128 * (cus / t128) < 4 * cus && p.k > 8192;
+            const TilePlan plan = idle ? split_k(Tile::k128, p, 2 * cus / t128, 1024, BK)
+                                       : split_k(Tile::k128Deep, p, cus / t128, 1024, BK);
             if (plan.slices > 1) return plan;
         }
         // Rounds of 128 x 128 tiles, two a CU.  A short K with at most half

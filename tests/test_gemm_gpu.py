@@ -491,7 +491,7 @@ def test_gemm_fp32_split_k(amd, dev, orc, ta, tb, cin_kind):
 # than one.  (m, n, k); an M/N-major operand needs its extent in packets.
 TILE16 = [(2056, 2200, 72), (1496, 1512, 200), (1112, 1000, 264), (712, 136, 8), (3000, 2904, 40),
           (200, 304, 4104), (1208, 1000, 5000), (1496, 1512, 4104), (40, 8200, 1032), (200, 328, 24),
-          (136, 264, 49160)]
+          (136, 264, 49160), (1128, 624, 4104), (200, 3000, 9000), (1200, 1104, 9000)]
 TILE32 = [(2052, 2044, 36), (1500, 1504, 100), (712, 132, 4), (300, 304, 4004), (20, 8204, 2052),
           (44, 4100, 4108), (1500, 1504, 2100), (132, 60, 28), (132, 140, 40004), (24, 4100, 1028), (36, 8204, 260),
           (4100, 24, 4100), (36, 196, 516)]
