@@ -970,8 +970,8 @@ def profile_launches(what: str, lib, ops, dev) -> None:
     thin:    the thin products of the suite (decode-step Linear layers,
              an LM head's logits and dX), ten launches each, the wide
              operand rotated over its copies;
-    odd:     products whose operands the matrix cores cannot read in place,
-             repacked: ten bf16 mm 2047^3 and five bf16 [2048, 4096] x
+    odd:     products with an odd K or row stride, read where they lie:
+             ten bf16 mm 2047^3 and five bf16 [2048, 4096] x
              [4096, 50257]; then binary ops with transposed inputs, fp32 and
              bf16 4096^2, ten x.t() + y and ten x.t() * y.t() each."""
     import ctypes as C
