@@ -30,7 +30,8 @@ void launch_gemm_general(const GemmArgs& p, hipStream_t stream);
 
 // Products with at most 64 rows or 64 columns whose large operand the
 // matrix cores can read in place (gemm_thin.hip); false when not eligible.
-bool launch_gemm_thin(int dtype, const GemmArgs& p, hipStream_t stream);
+// probe: launches nothing, only says whether it would.
+bool launch_gemm_thin(int dtype, const GemmArgs& p, hipStream_t stream, bool probe = false);
 
 // True when a product of at most 64 rows or columns runs faster on the tile
 // kernel than on the thin one (gemm_mfma.hip).

@@ -1588,68 +1588,105 @@ bool packets_aligned(const void* x, int64_t ld, int64_t stride) {
     return aligned16(x) && ld % V == 0 && stride % V == 0;
 }
 
-// Whether a 16-bit product gains by copies of its operands that are not
-// whole aligned packets.  Read in place, such an operand costs a product that
-// fills the chip time per multiply-add (each load touches twice the cache
-// lines): about 0.70e-15 s for a K-major and 0.40e-15 s for an M/N-major one
-// (bf16 8191 x 11007 x 4095 in place 1172 us NT, 1081 NN, 1006 TN, on copies
-// 760, 794 and 815).  The copies cost one pass at about 5 TB/s and a launch
-// each: 2047^3 takes 32 us in place and would take 40.  float32 is bound by
-// its MFMAs and loses nothing in place.
+// A product on copies of its operands that are not aligned packets: which
+// ones, where in the workspace, and the product on them.  A K that is no whole
+// number of packets is padded in both copies.
+template <typename T>
+struct Repacked {
+    int64_t kp;
+    bool fix_a, fix_b;
+    Repack<T> a, b;
+    size_t off_b, bytes;
+
+    explicit Repacked(const GemmArgs& p)
+        : kp(p.k % Mfma<T>::V != 0 ? (p.k + Mfma<T>::BK - 1) / Mfma<T>::BK * Mfma<T>::BK : p.k),
+          fix_a(kp != p.k || !packets_aligned<T>(p.a, p.lda, p.stride_a)),
+          fix_b(kp != p.k || !packets_aligned<T>(p.b, p.ldb, p.stride_b)),
+          a(p.lda, p.stride_a, !p.trans_a, p.batch, p.m, p.k, kp),
+          b(p.ldb, p.stride_b, p.trans_b, p.batch, p.n, p.k, kp),
+          off_b(fix_a ? (a.elems() * a.E + 255) / 256 * 256 : 0),
+          bytes(off_b + (fix_b ? b.elems() * b.E : 0)) {}
+
+    GemmArgs product(const GemmArgs& p, void* ws) const {
+        GemmArgs q = p;
+        q.k = kp;
+        if (fix_a) {
+            q.a = ws;
+            q.lda = a.ld_out;
+            q.stride_a = a.out_stride();
+        }
+        if (fix_b) {
+            q.b = static_cast<char*>(ws) + off_b;
+            q.ldb = b.ld_out;
+            q.stride_b = b.out_stride();
+        }
+        return q;
+    }
+};
+
+// Whether a product gains by copies of its operands that are not whole
+// aligned packets.
+//   * 16-bit: read in place, such an operand costs a product that fills the
+//     chip time per multiply-add (each load touches twice the cache lines):
+//     about 0.70e-15 s for a K-major and 0.40e-15 s for an M/N-major one (bf16
+//     8191 x 11007 x 4095 in place 1172 us NT, 1081 NN, 1006 TN, on copies
+//     760, 794 and 815).  The copies cost one pass at about 5 TB/s and a launch
+//     each: 2047^3 takes 32 us in place and would take 40.
+//   * float32 is bound by its MFMAs and loses nothing in place, but a batch is
+//     not split over K: a thin product of a long K walks it on few CUs, 18.5
+//     ns a k, where the thin kernel reads its copies faster.  32 x (8 x 15 x
+//     2121) 39.1 us in place, 22.0 on copies; 2 x (256 x 4 x 4001) 70.8 and
+//     25.7; 32 x (256 x 4 x 2121) 43.0 and 46.4; 128 x (8 x 15 x 1023) 20.7
+//     and 21.0.
 template <typename T>
 bool repack_pays(const GemmArgs& p) {
     constexpr int64_t E = sizeof(typename Elem<T>::storage);
-    if (E != 2) return false;
-    const bool pad = p.k % Mfma<T>::V != 0;
-    double in_place = 0.0, copies = 0.0;
-    auto add = [&](const void* x, int64_t ld, int64_t stride, bool kmajor, int64_t mn) {
-        const bool odd = !packets_aligned<T>(x, ld, stride);
-        if (odd) in_place += kmajor ? 0.70e-15 : 0.40e-15;
-        if (odd || pad) {
-            copies += 5e-6 + 2.0 * E * static_cast<double>(stride == 0 ? 1 : p.batch) * static_cast<double>(mn) *
-                                 static_cast<double>(p.k) / 5e12;
-        }
-    };
-    add(p.a, p.lda, p.stride_a, !p.trans_a, p.m);
-    add(p.b, p.ldb, p.stride_b, p.trans_b, p.n);
-    return in_place * static_cast<double>(p.batch) * static_cast<double>(p.m) * static_cast<double>(p.n) *
-               static_cast<double>(p.k) > copies;
+    if constexpr (E == 4) {
+        if (p.batch == 1 || std::min(p.m, p.n) > 64) return false;
+        const Repacked<T> copies(p);
+        if (copies.bytes == 0) return false;
+        int device = 0;
+        TP_AMD_HIP_CHECK(hipGetDevice(&device));
+        const int64_t cus = cu_count(device);
+        const double read = 4.0 * static_cast<double>((p.stride_a == 0 ? 1 : p.batch) * p.m + (p.stride_b == 0 ? 1 : p.batch) * p.n) *
+                            static_cast<double>(p.k);
+        const double in_place = static_cast<double>((tiles_of(p, 64, 64) + cus - 1) / cus) * static_cast<double>(p.k) * 18.5e-9;
+        // two copies, the thin kernel's launch, the bytes at 5 and 4 TB/s
+        if (in_place <= 20e-6 + 2.0 * read / 5e12 + read / 4e12) return false;
+        void* any_aligned = reinterpret_cast<void*>(uintptr_t{256});
+        return launch_gemm_thin(DtypeOf<T>::value, copies.product(p, any_aligned), nullptr, true);
+    } else {
+        const bool pad = p.k % Mfma<T>::V != 0;
+        double in_place = 0.0, copies = 0.0;
+        auto add = [&](const void* x, int64_t ld, int64_t stride, bool kmajor, int64_t mn) {
+            const bool odd = !packets_aligned<T>(x, ld, stride);
+            if (odd) in_place += kmajor ? 0.70e-15 : 0.40e-15;
+            if (odd || pad) {
+                copies += 5e-6 + 2.0 * E * static_cast<double>(stride == 0 ? 1 : p.batch) * static_cast<double>(mn) *
+                                     static_cast<double>(p.k) / 5e12;
+            }
+        };
+        add(p.a, p.lda, p.stride_a, !p.trans_a, p.m);
+        add(p.b, p.ldb, p.stride_b, p.trans_b, p.n);
+        return in_place * static_cast<double>(p.batch) * static_cast<double>(p.m) * static_cast<double>(p.n) *
+                   static_cast<double>(p.k) > copies;
+    }
 }
 
-// A product on copies of its operands that are not aligned packets, where
-// that pays.
+// A product on copies of its operands, where that pays.
 template <typename T>
 void launch_repacked(const GemmArgs& p, hipStream_t stream) {
     int device = 0;
     TP_AMD_HIP_CHECK(hipGetDevice(&device));
-    const bool a_kmajor = !p.trans_a, b_kmajor = p.trans_b;
-    // A K that is no whole number of packets is padded in both copies.
-    const bool pad = p.k % Mfma<T>::V != 0;
-    const int64_t kp = pad ? (p.k + Mfma<T>::BK - 1) / Mfma<T>::BK * Mfma<T>::BK : p.k;
-    const bool fix_a = pad || !packets_aligned<T>(p.a, p.lda, p.stride_a);
-    const bool fix_b = pad || !packets_aligned<T>(p.b, p.ldb, p.stride_b);
-    const Repack<T> a(p.lda, p.stride_a, a_kmajor, p.batch, p.m, p.k, kp), b(p.ldb, p.stride_b, b_kmajor, p.batch, p.n, p.k, kp);
-    const size_t off_b = fix_a ? (a.elems() * a.E + 255) / 256 * 256 : 0;
-    const Workspace ws = Workspace::if_room(off_b + (fix_b ? b.elems() * b.E : 0), device);
+    const Repacked<T> copies(p);
+    const Workspace ws = Workspace::if_room(copies.bytes, device);
     if (ws.get() == nullptr) {
         launch_mfma<T>(p, stream);  // in place
         return;
     }
-    GemmArgs q = p;
-    q.k = kp;
-    if (fix_a) {
-        a.launch(p.a, ws.get(), stream);
-        q.a = ws.get();
-        q.lda = a.ld_out;
-        q.stride_a = a.out_stride();
-    }
-    if (fix_b) {
-        void* wb = static_cast<char*>(ws.get()) + off_b;
-        b.launch(p.b, wb, stream);
-        q.b = wb;
-        q.ldb = b.ld_out;
-        q.stride_b = b.out_stride();
-    }
+    const GemmArgs q = copies.product(p, ws.get());
+    if (copies.fix_a) copies.a.launch(p.a, const_cast<void*>(q.a), stream);
+    if (copies.fix_b) copies.b.launch(p.b, const_cast<void*>(q.b), stream);
     // A thin product reads its copies through the thin kernel.
     if (!launch_gemm_thin(DtypeOf<T>::value, q, stream)) launch_mfma<T>(q, stream);
 }

@@ -660,7 +660,7 @@ void launch_rows(const ThinArgs& q, bool xvec, int64_t batch, hipStream_t stream
 }
 
 template <typename T>
-bool launch_typed(const GemmArgs& p, hipStream_t stream) {
+bool launch_typed(const GemmArgs& p, hipStream_t stream, bool probe) {
     using S = typename Elem<T>::storage;
     constexpr int V = 16 / sizeof(S);
     constexpr int64_t kLimit = int64_t(1) << 31;
@@ -739,6 +739,7 @@ bool launch_typed(const GemmArgs& p, hipStream_t stream) {
     int device = 0;
     TP_AMD_HIP_CHECK(hipGetDevice(&device));
     if (tiles_take_thin(sizeof(S) == 4 ? TP_AMD_FLOAT32 : TP_AMD_BFLOAT16, p, device)) return false;
+    if (probe) return true;
     if (kmajor) {
         launch_rows<T, true>(q, xvec, p.batch, stream);
     } else {
@@ -750,11 +751,11 @@ bool launch_typed(const GemmArgs& p, hipStream_t stream) {
 
 }  // namespace
 
-bool launch_gemm_thin(int dtype, const GemmArgs& p, hipStream_t stream) {
+bool launch_gemm_thin(int dtype, const GemmArgs& p, hipStream_t stream, bool probe) {
     switch (dtype) {
-        case TP_AMD_FLOAT32: return launch_typed<float>(p, stream);
-        case TP_AMD_BFLOAT16: return launch_typed<bf16_t>(p, stream);
-        case TP_AMD_FLOAT16: return launch_typed<f16_t>(p, stream);
+        case TP_AMD_FLOAT32: return launch_typed<float>(p, stream, probe);
+        case TP_AMD_BFLOAT16: return launch_typed<bf16_t>(p, stream, probe);
+        case TP_AMD_FLOAT16: return launch_typed<f16_t>(p, stream, probe);
         default: return false;
     }
 }

@@ -214,14 +214,26 @@ def test_thin_nan_and_inf(dev, ops, orc, dtype, tb):
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=lambda d: IDS[d])
 def test_thin_after_repack(dev, ops, orc, dtype):
     """x [3, 2048] @ W [2048, 1001]: W row-major with an odd leading
-    dimension, which no kernel reads in 16-byte packets, is copied K-major
-    and then multiplied by the thin kernel; against float64."""
+    dimension, which the thin kernel does not read; against float64."""
     g = np.random.default_rng(11)
     x = orc.from_float(g.standard_normal((3, 2048)).astype(np.float32), dtype)
     w = orc.from_float(g.standard_normal((2048, 1001)).astype(np.float32), dtype)
     got = ops.mm(dev.from_numpy(x, dtype=dtype), dev.from_numpy(w, dtype=dtype)).numpy()
     want = orc.to_float(x, dtype).astype(np.float64) @ orc.to_float(w, dtype).astype(np.float64)
     _check(orc, got, want, dtype, "thin product of a repacked operand")
+
+
+@pytest.mark.parametrize("B,m,n,k", [(32, 8, 15, 2121), (2, 256, 4, 4001), (24, 40, 63, 4001), (4, 1, 333, 2123),
+                                     (32, 8, 15, 511)])
+def test_thin_batches_of_an_odd_k(dev, ops, orc, B, m, n, k):
+    """Batches of thin float32 products whose K is no whole number of packets,
+    long enough for the thin kernel on padded copies or not; against float64."""
+    g = np.random.default_rng(12)
+    x, w = (g.standard_normal(s).astype(np.float32) for s in ((B, m, k), (B, n, k)))
+    wd = dev.from_numpy(w)
+    got = ops.bmm(dev.from_numpy(x), wd._view((B, k, n), (n * k, 1, k))).numpy()
+    want = np.matmul(x.astype(np.float64), w.astype(np.float64).transpose(0, 2, 1))
+    _check(orc, got, want, F32, f"batch of {B} x {m}x{n}x{k}")
 
 
 def test_thin_random_shapes(amd, dev, orc):
