@@ -673,7 +673,15 @@ bool launch_typed(const GemmArgs& p, hipStream_t stream, bool probe) {
     q.beta = p.beta;
     q.cin = p.cin;
     bool kmajor;
-    if (thin_m && (!thin_n || p.m <= p.n)) {
+    // The longer side is W; of two thin sides in a float32 batch, which the tile
+    // kernel does not split over K, the one that can be read in packets.  32 x
+    // (8 x 15 x 2122), W row-major, 39.5 -> 26.4 us; 128 x (8 x 15 x 512) 11.8
+    // -> 8.5.  More than 16 rows of X pay from a longer K on: 128 x (40 x 63 x
+    // 512) 12.3 on tiles, 21.7 here, 32 x (40 x 63 x 4002) 78 and 53.
+    const bool a_packets = (p.trans_a ? p.m : p.k) % V == 0, b_packets = (p.trans_b ? p.k : p.n) % V == 0;
+    const bool either = thin_m && thin_n && sizeof(S) == 4 && p.batch > 1 && a_packets != b_packets &&
+                        ((b_packets ? p.m : p.n) <= 16 || p.k >= 4000);
+    if (either ? b_packets : thin_m && (!thin_n || p.m <= p.n)) {
         // X = A, W = B.
         q.m = p.m;
         q.n = p.n;

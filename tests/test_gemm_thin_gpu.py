@@ -224,7 +224,7 @@ def test_thin_after_repack(dev, ops, orc, dtype):
 
 
 @pytest.mark.parametrize("B,m,n,k", [(32, 8, 15, 2121), (2, 256, 4, 4001), (24, 40, 63, 4001), (4, 1, 333, 2123),
-                                     (32, 8, 15, 511)])
+                                     (32, 8, 15, 511), (40, 8, 15, 2124), (40, 16, 17, 1024), (40, 17, 18, 4004)])
 def test_thin_batches_of_an_odd_k(dev, ops, orc, B, m, n, k):
     """Batches of thin float32 products whose K is no whole number of packets,
     long enough for the thin kernel on padded copies or not; against float64."""
@@ -234,6 +234,9 @@ def test_thin_batches_of_an_odd_k(dev, ops, orc, B, m, n, k):
     got = ops.bmm(dev.from_numpy(x), wd._view((B, k, n), (n * k, 1, k))).numpy()
     want = np.matmul(x.astype(np.float64), w.astype(np.float64).transpose(0, 2, 1))
     _check(orc, got, want, F32, f"batch of {B} x {m}x{n}x{k}")
+    # W row-major, its rows no whole packets either
+    rows = dev.from_numpy(np.ascontiguousarray(w.transpose(0, 2, 1)))
+    _check(orc, ops.bmm(dev.from_numpy(x), rows).numpy(), want, F32, f"batch of {B} x {m}x{n}x{k}, W row-major")
 
 
 def test_thin_random_shapes(amd, dev, orc):
